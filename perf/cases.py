@@ -1,0 +1,581 @@
+"""The work this engine is used for, as cases that can be timed.
+
+Families, each over its range of sizes and options:
+  few       run_simulation of a few bodies (orbits, point charges, dipoles) in the default
+            FP64 arithmetic, every step saved, as the reference's own examples do: the
+            smallest calls, where launches and copies count
+  md64      Lennard-Jones argon in FP64 (the default precision), frames saved, with or
+            without a Berendsen thermostat
+  water64   SPC/Fw water in FP64, frames saved
+  rhs       one right-hand side for a caller that integrates by itself (host arrays in and
+            out, the closure protocol's whole-system form), FP64
+  nbody     all-pairs gravity in mixed precision, equal or unequal masses
+  liquid    Lennard-Jones liquids in mixed precision
+  water     SPC/Fw water with a reaction field in mixed precision
+  batch     an ensemble of independent Lennard-Jones replicas
+  energy    energies and temperature of a saved state (total_energy, temperature)
+  rdf       the radial distribution function over saved frames
+
+Each pass starts from the state in host memory (the engine's entry points take host arrays)
+and hands back the whole final state or trajectory.  The FP64 paths return FP64 arrays.  The
+mixed paths evaluate pair forces in FP32, so their final states are handed on as FP32, which
+is what trajectory files hold.  Runs are short enough that a chaotic trajectory still shows
+the arithmetic and not its own divergence.
+"""
+import math
+import os
+import sys
+
+import numpy as np
+import torch
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                                "nbodysimulator.jl_amd"))
+
+import nbodysimulator as nb  # noqa: E402
+from nbodysimulator import _lib  # noqa: E402
+
+# SPC/Fw water in nm, kJ/mol, ps, e
+KCAL = 4.184
+MO, MH, QO, QH = 15.999, 1.00794, -0.82, 0.41
+SIG_O, EPS_O = 0.3165492, 0.1554253 * KCAL
+ROH, KBOND = 0.1012, 1059.162 * KCAL * 100.0
+AHOH, KANGLE = 113.24 * math.pi / 180.0, 75.90 * KCAL
+K_EL, KB_WATER = 138.935458, 8.3144598e-3
+RHO_LJ, DT_LJ = 0.8442, 0.002
+
+
+def listed():
+    return [
+        # a small planetary system, every step saved: the reference's introductory example
+        dict(name="orbits", family="few", law="gravity", n=8, steps=1000),
+        # the argon liquid of the reference's tests, default precision, a frame every 10 steps
+        dict(name="argon-fp64", family="md64", n=864, steps=200, save_every=10, thermostat="none"),
+        # a small water box in the default precision
+        dict(name="water-fp64", family="water64", nmol=343, steps=50, save_every=5, el="coulomb"),
+        # one force evaluation for an external integrator
+        dict(name="rhs-lj", family="rhs", law="lj", n=4000),
+        # the headline workload: a Plummer sphere of equal masses
+        dict(name="plummer-65536", family="nbody", n=65536, steps=10, equal=True),
+        # a star cluster with a mass spectrum, an odd number of bodies
+        dict(name="cluster-3001", family="nbody", n=3001, steps=100, equal=False),
+        # Lennard-Jones liquids, the small and the large benchmark sizes
+        dict(name="lj-864", family="liquid", n=864, steps=300, thermostat="none"),
+        dict(name="lj-32000", family="liquid", n=32000, steps=250, thermostat="none"),
+        # the water benchmark: 4,096 molecules, reaction field 0.9 nm, Berendsen 300 K
+        dict(name="water-4096", family="water", nmol=4096, steps=200, thermostat="berendsen"),
+        # an ensemble of replicas of 108 to 4,000 atoms with their thermostats
+        dict(name="batch-256", family="batch", nrep=256, cmin=3, cmax=10, steps=200),
+        # analysis of one saved state, and of a trajectory
+        dict(name="energy-10976", family="energy", n=10976),
+        dict(name="rdf-4000", family="rdf", n=4000, frames=10, maxbin=1000),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    fam = rng.choice(["few", "md64", "water64", "rhs", "nbody", "liquid", "water", "batch", "energy",
+                      "rdf"])
+    if fam == "few":
+        return dict(family=fam, law=rng.choice(["gravity", "charges", "dipoles"]),
+                    n=_log(rng, 2, 48), steps=_log(rng, 100, 1000))
+    if fam == "md64":
+        return dict(family=fam, n=_log(rng, 100, 2000), steps=_log(rng, 20, 150),
+                    save_every=rng.choice([1, 5, 10, 20]),
+                    thermostat=rng.choice(["none", "berendsen"]))
+    if fam == "water64":
+        return dict(family=fam, nmol=_log(rng, 64, 500), steps=_log(rng, 10, 50),
+                    save_every=rng.choice([1, 5, 10]), el=rng.choice(["coulomb", "rf"]))
+    if fam == "rhs":
+        return dict(family=fam, law=rng.choice(["lj", "gravity", "coulomb"]), n=_log(rng, 200, 8000))
+    if fam == "nbody":
+        n = _log(rng, 1000, 60000)
+        return dict(family=fam, n=n, steps=max(4, min(100, int(3e10 / n / n))),
+                    equal=rng.random() < 0.5)
+    if fam == "liquid":
+        return dict(family=fam, n=_log(rng, 500, 36000), steps=_log(rng, 100, 250),
+                    thermostat=rng.choice(["none", "berendsen", "langevin"]))
+    if fam == "water":
+        return dict(family=fam, nmol=_log(rng, 216, 4500), steps=_log(rng, 50, 200),
+                    thermostat=rng.choice(["none", "berendsen"]))
+    if fam == "batch":
+        lo = rng.randint(3, 6)
+        return dict(family=fam, nrep=_log(rng, 32, 256), cmin=lo, cmax=rng.randint(lo + 1, 10),
+                    steps=_log(rng, 50, 200))
+    if fam == "energy":
+        return dict(family=fam, n=_log(rng, 500, 20000))
+    return dict(family=fam, n=_log(rng, 300, 6000), frames=rng.randint(1, 10),
+                maxbin=_log(rng, 100, 3000))
+
+
+# ---------------------------------------------------------------------------------------
+# inputs
+# ---------------------------------------------------------------------------------------
+
+def _lj_box(n):
+    """Cells per side and box side of the FCC lattice that holds n atoms."""
+    c = math.ceil((n / 4.0) ** (1.0 / 3.0) - 1e-9)
+    return c, (4.0 * c ** 3 / RHO_LJ) ** (1.0 / 3.0)
+
+
+def _lj_state(n, rng, T, jitter=0.06):
+    """n atoms on a jittered FCC lattice, vacancies in it where n is no 4 c^3."""
+    c, L = _lj_box(n)
+    g = np.arange(c)
+    corner = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 1, 3)
+    basis = np.array([[0, 0, 0], [.5, .5, 0], [.5, 0, .5], [0, .5, .5]])
+    sites = (corner + basis).reshape(-1, 3)
+    keep = np.sort(rng.permutation(len(sites))[:n])
+    u = (sites[keep] + 0.25) * (L / c)
+    u = u + jitter * rng.uniform(-1, 1, u.shape)
+    v = math.sqrt(T) * rng.standard_normal((n, 3))
+    v -= v.mean(axis=0)
+    return np.ascontiguousarray(u), np.ascontiguousarray(v), L
+
+
+def _water_state(nmol, rng):
+    c = math.ceil(nmol ** (1.0 / 3.0) - 1e-9)
+    L = (nmol * (MO + 2 * MH) / (0.997 * 602.214076)) ** (1.0 / 3.0)
+    g = np.arange(c) + 0.5
+    sites = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3) * (L / c)
+    O = sites[np.sort(rng.permutation(len(sites))[:nmol])] + 0.01 * rng.standard_normal((nmol, 3))
+    q = rng.standard_normal((nmol, 4))
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    w, x, y, z = q.T
+    R = np.empty((nmol, 3, 2))   # the first two columns of each rotation
+    R[:, 0, 0], R[:, 1, 0], R[:, 2, 0] = 1 - 2 * (y * y + z * z), 2 * (x * y + z * w), 2 * (x * z - y * w)
+    R[:, 0, 1], R[:, 1, 1], R[:, 2, 1] = 2 * (x * y - z * w), 1 - 2 * (x * x + z * z), 2 * (y * z + x * w)
+    u = np.empty((3 * nmol, 3))
+    u[0::3] = O
+    u[1::3] = O + ROH * R[:, :, 0]
+    u[2::3] = O + ROH * (math.cos(AHOH) * R[:, :, 0] + math.sin(AHOH) * R[:, :, 1])
+    ms = np.tile([MO, MH, MH], nmol)
+    v = np.sqrt(KB_WATER * 300.0 / ms)[:, None] * rng.standard_normal((3 * nmol, 3))
+    return u, v, L, ms, np.tile([QO, QH, QH], nmol)
+
+
+def _plummer(n, rng, equal):
+    r = 1.0 / np.sqrt(rng.uniform(1e-6, 0.99, n) ** (-2.0 / 3.0) - 1.0)
+    d = rng.standard_normal((n, 3))
+    u = d / np.linalg.norm(d, axis=1, keepdims=True) * r[:, None]
+    v = rng.standard_normal((n, 3)) / np.sqrt(6.0 * np.sqrt(1.0 + r * r))[:, None]
+    m = np.full(n, 1.0 / n) if equal else np.exp(0.7 * rng.standard_normal(n))
+    m /= m.sum()
+    if equal:
+        m[:] = 1.0 / n
+    return np.ascontiguousarray(u - u.mean(0)), np.ascontiguousarray(v - v.mean(0)), m
+
+
+def _few_state(case, rng):
+    """(u, v, m, extra, dt) of a small system that stays regular over the run."""
+    n, law = case["n"], case["law"]
+    if law == "gravity":    # light planets around a star, radii spaced apart
+        r = 1.0 + 0.35 * np.arange(n)
+        ph = rng.uniform(0, 2 * math.pi, n)
+        u = np.stack([r * np.cos(ph), r * np.sin(ph), 0.02 * rng.standard_normal(n)], 1)
+        s = 1.0 / np.sqrt(r)
+        v = np.stack([-s * np.sin(ph), s * np.cos(ph), 0.01 * rng.standard_normal(n)], 1)
+        m = rng.uniform(1e-7, 1e-5, n)
+        u[0], v[0], m[0] = 0.0, 0.0, 1.0
+        return u, v, m, None, 2e-3
+    c = math.ceil(n ** (1.0 / 3.0))
+    g = np.arange(c) - (c - 1) / 2
+    u = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)[:n] * 2.0
+    u = u + 0.2 * rng.standard_normal((n, 3))
+    v = 0.1 * rng.standard_normal((n, 3))
+    m = rng.uniform(0.5, 2.0, n)
+    extra = rng.uniform(0.2, 0.5, n) if law == "charges" else 0.05 * rng.standard_normal((n, 3))
+    return u, v, m, extra, 2e-3
+
+
+def _inputs(case, seed):
+    rng = np.random.default_rng([seed, 20240])
+    fam = case["family"]
+    if fam == "few":
+        return _few_state(case, rng)
+    if fam in ("water64", "water"):
+        return _water_state(case["nmol"], rng)
+    if fam == "nbody":
+        return _plummer(case["n"], rng, case["equal"])
+    if fam == "rhs" and case["law"] == "gravity":
+        return _plummer(case["n"], rng, False)
+    if fam == "batch":
+        reps = []
+        sizes = np.random.default_rng(case["nrep"]).integers(case["cmin"], case["cmax"] + 1, case["nrep"])
+        for c in sizes:   # the ensemble's sizes belong to the case, its states to the seed
+            n = 4 * int(c) ** 3
+            T = float(rng.uniform(0.7, 1.5))
+            reps.append((*_lj_state(n, rng, T, 0.03), T, bool(rng.random() < 0.5)))
+        return reps
+    if fam == "rdf":
+        u, _, L = _lj_state(case["n"], rng, 1.0)
+        # a short diffusive trajectory, unwrapped as the engine returns it
+        walk = np.cumsum(0.05 * rng.standard_normal((case["frames"], *u.shape)), axis=0)
+        return u[None] + walk, L
+    return _lj_state(case["n"], rng, 0.9)
+
+
+def _liquid_context(n, L, charges=None):
+    ctx = _lib.Context(n, _lib.SYS_POTENTIAL, np.ones(n), charges)
+    ctx.set_boundary(_lib.BC_CUBIC, [L, 0, 0, 0, 0, 0])
+    ctx.set_kb(1.0)
+    return ctx
+
+
+def _charges(n):
+    return np.where(np.arange(n) % 2 == 0, 1.0, -1.0) * 0.5
+
+
+def _thermostat(ctx, kind, T, tau, gamma=1.0):
+    if kind == "berendsen":
+        ctx.set_thermostat(_lib.THERM_BERENDSEN, T, tau)
+    elif kind == "langevin":
+        ctx.set_thermostat(_lib.THERM_LANGEVIN, T, gamma)
+
+
+def prepare(case, seed):
+    fam = case["family"]
+    s = dict(case=dict(case))
+    got = _inputs(case, seed)
+    if fam == "few":
+        u, v, m, extra, dt = got
+        if case["law"] == "gravity":
+            system = nb.GravitationalSystem([nb.MassBody(a, b, c) for a, b, c in zip(u, v, m)], 1.0)
+        elif case["law"] == "charges":
+            system = nb.ChargedParticles([nb.ChargedParticle(a, b, c, q)
+                                          for a, b, c, q in zip(u, v, m, extra)], 1.0)
+        else:
+            system = nb.PotentialNBodySystem(
+                [nb.MagneticParticle(a, b, c, mm) for a, b, c, mm in zip(u, v, m, extra)],
+                {"magnetic": nb.MagnetostaticParameters(1.0)})
+        s["sim"] = nb.NBodySimulation(system, (0.0, case["steps"] * dt))
+        s["dt"] = dt
+        return s
+    if fam == "batch":
+        ns = [len(r[0]) for r in got]
+        b = _lib.Batch(ns, [r[2] for r in got], np.ones(sum(ns)))
+        for k, r in enumerate(got):
+            if r[4]:
+                b.set_thermostat(k, _lib.THERM_LANGEVIN, r[3], 1.0)
+            else:
+                b.set_thermostat(k, _lib.THERM_ANDERSEN, r[3], 0.01)
+        s.update(batch=b, u=np.concatenate([r[0] for r in got]), v=np.concatenate([r[1] for r in got]))
+        return s
+    if fam in ("water64", "water"):
+        u, v, L, ms, qs = got
+        rc = min(0.9, 0.45 * L)
+        ctx = _lib.Context(len(ms), _lib.SYS_WATER, ms, qs)
+        ctx.set_boundary(_lib.BC_CUBIC, [L, 0, 0, 0, 0, 0])
+        ctx.set_kb(KB_WATER)
+        ctx.add_lennard_jones(EPS_O, SIG_O, rc)
+        if fam == "water" or case["el"] == "rf":
+            ctx.add_reaction_field(K_EL, rc, math.inf)
+        else:
+            ctx.add_electrostatic(K_EL, rc)
+        ctx.set_spcfw(ROH, AHOH, KBOND, KANGLE)
+        _thermostat(ctx, case.get("thermostat", "none"), 300.0, 0.1)
+        s["dt"] = 0.0005
+    elif fam == "nbody" or (fam == "rhs" and case["law"] == "gravity"):
+        u, v, m = got
+        ctx = _lib.Context(len(m), _lib.SYS_POTENTIAL, m)
+        ctx.add_gravitational(1.0)
+        s["dt"] = 1e-3
+    elif fam == "rdf":
+        frames, L = got
+        s.update(ctx=_liquid_context(case["n"], L), frames=frames)
+        return s
+    else:
+        u, v, L = got
+        n = case["n"]
+        coul = fam == "rhs" and case["law"] == "coulomb"
+        ctx = _liquid_context(n, L, _charges(n) if coul else None)
+        ctx.add_lennard_jones(1.0, 1.0, min(2.5, 0.49 * L))
+        if coul:
+            ctx.add_electrostatic(1.0, 0.49 * L)
+        _thermostat(ctx, case.get("thermostat", "none"), 1.0, 0.5)
+        s["dt"] = DT_LJ
+    if fam in ("nbody", "liquid", "water"):
+        ctx.set_precision(_lib.PREC_MIXED)
+    s.update(ctx=ctx, u=u, v=v)
+    return s
+
+
+# ---------------------------------------------------------------------------------------
+# one pass
+# ---------------------------------------------------------------------------------------
+
+def run(state):
+    case = state["case"]
+    fam = case["family"]
+    if fam == "few":
+        sol = nb.run_simulation(state["sim"], nb.VelocityVerlet(), dt=state["dt"]).solution
+        return {"u": sol.u, "v": sol.v}
+    if fam == "batch":
+        b = state["batch"]
+        b.set_state(state["u"], state["v"])
+        b.run(DT_LJ, case["steps"], seed=1)
+        u, v = b.get_state()
+        return {"u": u.astype(np.float32), "v": v.astype(np.float32)}
+    ctx = state["ctx"]
+    if fam == "rhs":
+        return {"a": ctx.rhs(state["u"], state["v"])}
+    if fam == "rdf":
+        rs, gr = ctx.rdf(state["frames"], case["maxbin"])
+        return {"r": rs, "g": gr}
+    ctx.set_state(state["u"], state["v"])
+    if fam == "energy":
+        ke, pe, _ = ctx.energies()
+        return {"ke": np.float64(ke), "pe": np.float64(pe), "T": np.float64(ctx.temperature())}
+    if fam in ("md64", "water64"):
+        uf, vf = ctx.vv_run(state["dt"], case["steps"], seed=1, save_every=case["save_every"])
+        return {"u": uf, "v": vf}
+    ctx.vv_run(state["dt"], case["steps"], seed=1)
+    u, v = ctx.get_state()
+    return {"u": u.astype(np.float32), "v": v.astype(np.float32)}
+
+
+# ---------------------------------------------------------------------------------------
+# what a pass cannot do without
+# ---------------------------------------------------------------------------------------
+
+def _lj_pairs(n, L, R):
+    return n * min(n - 1.0, (n / L ** 3) * 4.0 / 3.0 * math.pi * R ** 3)   # ordered, in the cutoff
+
+
+def work(case):
+    fam = case["family"]
+    steps = case.get("steps", 1)
+    if fam == "few":
+        n = case["n"]
+        return {"bytes": 48.0 * n * (steps + 2), "flops": 25.0 * n * (n - 1) * (steps + 1)}
+    if fam == "rdf":
+        n = case["n"]
+        return {"bytes": 24.0 * n * case["frames"] + 16.0 * case["maxbin"],
+                "flops": 15.0 * case["frames"] * n * (n - 1) / 2}
+    if fam == "energy":
+        n = case["n"]
+        L = _lj_box(n)[1]
+        return {"bytes": 56.0 * n + 24, "flops": 15.0 * _lj_pairs(n, L, 2.5) + 10.0 * n}
+    if fam == "rhs":
+        n = case["n"]
+        L = _lj_box(n)[1]
+        pairs = n * (n - 1.0) if case["law"] == "gravity" else \
+            _lj_pairs(n, L, 0.49 * L if case["law"] == "coulomb" else 2.5)
+        return {"bytes": 80.0 * n, "flops": 29.0 * pairs}
+    if fam == "batch":
+        n = case["nrep"] * 2.0 * sum(c ** 3 for c in range(case["cmin"], case["cmax"] + 1)) * 2.0 / \
+            (case["cmax"] - case["cmin"] + 1)
+        return {"bytes": 104.0 * n, "flops": 29.0 * 55.0 * n * (steps + 1)}
+    if fam in ("water", "water64"):
+        n = 3 * case["nmol"]
+        L = (case["nmol"] * (MO + 2 * MH) / (0.997 * 602.214076)) ** (1.0 / 3.0)
+        rc = min(0.9, 0.45 * L)
+        pairs = _lj_pairs(n, L, rc) * (27.0 + 10.0 / 9.0) + 200.0 * case["nmol"]
+    elif fam == "nbody":
+        n = case["n"]
+        pairs = 20.0 * n * (n - 1.0)
+    else:
+        n = case["n"]
+        L = _lj_box(n)[1]
+        pairs = 29.0 * _lj_pairs(n, L, min(2.5, 0.49 * L))
+    frames = steps // case["save_every"] if "save_every" in case else 1
+    return {"bytes": 56.0 * n + 48.0 * n * frames, "flops": pairs * (steps + 1)}
+
+
+# ---------------------------------------------------------------------------------------
+# the same in 64 bits, in plain torch
+# ---------------------------------------------------------------------------------------
+
+def _dev():
+    return "cuda" if torch.cuda.is_available() else "cpu"
+
+
+def _t(a):
+    return torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device=_dev())
+
+
+class _Pairs:
+    """The pairs i < j within a cutoff in a cubic box, from a list with a skin."""
+
+    def __init__(self, L, R, skin, stride=1, mol=False):
+        self.L, self.R, self.skin, self.stride, self.mol = L, R, skin, stride, mol
+        self.at = None
+
+    def get(self, x):
+        if self.at is None or float((x - self.at).square().sum(1).max()) > 0.24 * self.skin ** 2:
+            self.at = x.clone()
+            y = x[::self.stride]
+            w = y - self.L * torch.floor(y / self.L)
+            n, ii, jj = len(w), [], []
+            rl2 = (self.R + self.skin) ** 2
+            idx = torch.arange(n, device=x.device)
+            for b in range(0, n, 512):
+                d2 = 0.0
+                for k in range(3):
+                    d = w[b:b + 512, None, k] - w[None, b:, k]
+                    d -= self.L * torch.round(d / self.L)
+                    d2 = d2 + d * d
+                m = (d2 < rl2) & (idx[None, b:] > idx[b:b + 512, None])
+                if self.mol:
+                    m &= (idx[None, b:] // 3) != (idx[b:b + 512, None] // 3)
+                i, j = torch.nonzero(m, as_tuple=True)
+                ii.append((i + b) * self.stride)
+                jj.append((j + b) * self.stride)
+            self.i, self.j = torch.cat(ii), torch.cat(jj)
+        d = x[self.i] - x[self.j]
+        d = d - self.L * torch.round(d / self.L)
+        r2 = d.square().sum(1)
+        k = r2 < self.R * self.R
+        return self.i[k], self.j[k], d[k], r2[k]
+
+
+def _add(a, i, j, f):
+    a.index_add_(0, i, f)
+    a.index_add_(0, j, -f)
+
+
+def _lj_force(f, i, j, d, r2, eps, sig):
+    s6 = (sig * sig / r2) ** 3
+    _add(f, i, j, (24.0 * eps * (2.0 * s6 * s6 - s6) / r2)[:, None] * d)
+
+
+def _gravity(x, m):
+    a = torch.empty_like(x)
+    for b in range(0, len(x), 1024):
+        d = [x[None, :, k] - x[b:b + 1024, None, k] for k in range(3)]
+        r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2]
+        w = torch.where(r2 > 0, m[None, :] * r2 ** -1.5, torch.zeros((), dtype=x.dtype, device=x.device))
+        a[b:b + 1024] = torch.stack([(w * c).sum(1) for c in d], 1)
+    return a
+
+
+def _verlet(x, v, force, dt, steps, save_every=None):
+    fu, fv = [x], [v]
+    a = force(x, v)
+    for k in range(1, steps + 1):
+        x = x + dt * v + (0.5 * dt * dt) * a
+        vh = v + (0.5 * dt) * a
+        a = force(x, vh)
+        v = vh + (0.5 * dt) * a
+        if save_every and k % save_every == 0:
+            fu.append(x)
+            fv.append(v)
+    if save_every:
+        return torch.stack(fu), torch.stack(fv)
+    return x, v
+
+
+def _berendsen(kind, m, kb, ndf, T0, tau):
+    def add(a, v):
+        if kind != "berendsen":
+            return a
+        T = (m[:, None] * v * v).sum() / (kb * ndf)
+        return a + (0.5 / tau * (T0 / T - 1.0)) * v
+    return add
+
+
+def exact(case, seed):
+    fam = case["family"]
+    got = _inputs(case, seed)
+    if fam == "batch" or case.get("thermostat") == "langevin":
+        return None   # random numbers: no value without the engine's generator
+    out = lambda u, v: {"u": u.cpu(), "v": v.cpu()}  # noqa: E731
+    if fam == "few":
+        u, v, m, extra, dt = got
+        x, v, m = (torch.as_tensor(a, dtype=torch.float64) for a in (u, v, m))   # small: on the CPU
+        n = len(m)
+        off = ~torch.eye(n, dtype=torch.bool)
+        q = None if extra is None else torch.as_tensor(extra, dtype=torch.float64)
+
+        def force(x, v):
+            d = x[:, None] - x[None]
+            r = d.square().sum(-1).add(torch.eye(n, dtype=torch.float64)).sqrt()
+            if case["law"] == "gravity":
+                return -(torch.where(off, m[None] / r ** 3, 0.0)[..., None] * d).sum(1)
+            if case["law"] == "charges":
+                return (torch.where(off, q[None] / r ** 3, 0.0)[..., None] * d).sum(1) * (q / m)[:, None]
+            e = d / r[..., None]
+            mi, mj = (q[:, None] * e).sum(-1, keepdim=True), (q[None] * e).sum(-1, keepdim=True)
+            dot = (q @ q.T)[..., None]
+            f = q[:, None] * mj + q[None] * mi + e * dot - 5.0 * e * mi * mj
+            return (torch.where(off, r ** -4, 0.0)[..., None] * f).sum(1) * (3.0 / m)[:, None]
+        return out(*_verlet(x, v, force, dt, case["steps"], 1))
+    if fam == "rdf":
+        frames, L = got
+        nbin, n = case["maxbin"], case["n"]
+        hist = torch.zeros(nbin + 1, dtype=torch.float64, device=_dev())
+        for f in frames:
+            x = _t(f)
+            for b in range(0, n, 512):
+                d = x[b:b + 512, None] - x[None]
+                d = d - L * torch.round(d / L)
+                r2 = d.square().sum(-1)
+                r = r2[(r2 < 0.25 * L * L) & (r2 > 0)].sqrt()
+                k = torch.ceil(r / (L / nbin)).long()
+                hist += torch.bincount(k[(k > 1) & (k <= nbin)], minlength=nbin + 1)[:nbin + 1]
+        rl = torch.arange(nbin, dtype=torch.float64, device=_dev()) * (L / nbin)
+        ideal = 4.0 / 3.0 * math.pi * n / L ** 3 * ((rl + L / nbin) ** 3 - rl ** 3)
+        return {"r": (rl + 0.5 * L / nbin).cpu(), "g": (hist[1:] / (len(frames) * n) / ideal).cpu()}
+    if fam == "nbody" or (fam == "rhs" and case["law"] == "gravity"):
+        u, v, m = (_t(a) for a in got)
+        if fam == "rhs":
+            return {"a": _gravity(u, m).cpu()}
+        return out(*_verlet(u, v, lambda x, _: _gravity(x, m), 1e-3, case["steps"]))
+    if fam in ("water", "water64"):
+        u, v, L, ms, qs = got
+        x, v, m, q = _t(u), _t(v), _t(ms), _t(qs)
+        rc = min(0.9, 0.45 * L)
+        oo, all_ = _Pairs(L, rc, 0.1, 3), _Pairs(L, rc, 0.1, 1, True)
+        krf = 1.0 / rc ** 3 if fam == "water" or case["el"] == "rf" else 0.0
+        ther = _berendsen(case.get("thermostat"), m, KB_WATER, 3 * len(ms) - 2 * (len(ms) // 3), 300.0, 0.1)
+
+        def force(x, v):
+            f = torch.zeros_like(x)
+            _lj_force(f, *oo.get(x), EPS_O, SIG_O)
+            i, j, d, r2 = all_.get(x)
+            _add(f, i, j, (K_EL * q[i] * q[j] * (r2 ** -1.5 - krf))[:, None] * d)
+            O = x[0::3]
+            b = [x[1::3] - O, x[2::3] - O]
+            r = [torch.linalg.norm(e, dim=1, keepdim=True) for e in b]
+            c = ((b[0] * b[1]).sum(1, keepdim=True) / (r[0] * r[1])).clamp(-1, 1)
+            th = torch.acos(c)
+            g = KANGLE * (th - AHOH) / torch.sqrt(1.0 - c * c)   # -dU/dcos
+            h = []
+            for p, o in ((0, 1), (1, 0)):
+                h.append(-KBOND * (r[p] - ROH) / r[p] * b[p]
+                         + g * (b[o] / (r[0] * r[1]) - c * b[p] / (r[p] * r[p])))
+            f[1::3] += h[0]
+            f[2::3] += h[1]
+            f[0::3] -= h[0] + h[1]
+            return ther(f / m[:, None], v)
+        return out(*_verlet(x, v, force, 0.0005, case["steps"], case.get("save_every")))
+    u, v, L = got
+    x, v = _t(u), _t(v)
+    n, R = case["n"], min(2.5, 0.49 * L)
+    pairs = _Pairs(L, R, 0.6)
+    if fam == "energy":
+        _, _, _, r2 = pairs.get(x)
+        s6 = r2 ** -3
+        c = R ** -12 - R ** -6
+        pe = 4.0 * float((s6 * s6 - s6 - c).sum() + c * (n * (n - 1) / 2))
+        ke = 0.5 * float((v * v).sum())
+        return {"ke": np.float64(ke), "pe": np.float64(pe), "T": np.float64(2.0 * ke / (3 * n))}
+    one = torch.ones(n, dtype=torch.float64, device=x.device)
+    ther = _berendsen(case.get("thermostat"), one, 1.0, 3 * n, 1.0, 0.5)
+    coul = fam == "rhs" and case["law"] == "coulomb"
+    q = _t(_charges(n))
+    far = _Pairs(L, 0.49 * L, 0.0)
+
+    def force(x, v):
+        f = torch.zeros_like(x)
+        _lj_force(f, *pairs.get(x), 1.0, 1.0)
+        if coul:
+            i, j, d, r2 = far.get(x)
+            _add(f, i, j, (q[i] * q[j] * r2 ** -1.5)[:, None] * d)
+        return ther(f, v)
+    if fam == "rhs":
+        return {"a": force(x, v).cpu()}
+    return out(*_verlet(x, v, force, DT_LJ, case["steps"], case.get("save_every")))
