@@ -92,9 +92,14 @@ def draw(rng):
     if fam == "rhs":
         return dict(family=fam, law=rng.choice(["lj", "gravity", "coulomb"]), n=_log(rng, 200, 8000))
     if fam == "nbody":
-        n = _log(rng, 1000, 60000)
-        return dict(family=fam, n=n, steps=max(4, min(100, int(3e10 / n / n))),
-                    equal=rng.random() < 0.5)
+        n, equal = _log(rng, 1000, 60000), rng.random() < 0.5
+        if equal:
+            # whole source tiles: the equal-mass kernel took the padding of a partial tile for
+            # bodies at the origin (forces off by percents), so results of other sizes made
+            # with it are nothing to compare with
+            unit = 4096 if n >= 4096 else 256
+            n = max(1, round(n / unit)) * unit
+        return dict(family=fam, n=n, steps=max(4, min(100, int(3e10 / n / n))), equal=equal)
     if fam == "liquid":
         return dict(family=fam, n=_log(rng, 500, 36000), steps=_log(rng, 100, 250),
                     thermostat=rng.choice(["none", "berendsen", "langevin"]))
