@@ -133,8 +133,8 @@ struct nbx_ctx {
     void* d_pos = nullptr;    // mixed path: double4 wrapped positions (+charge) or float4 (+mass)
     void* d_pos2 = nullptr;   // second position buffer (odd steps)
     double* d_x2 = nullptr;   // second unwrapped-position buffer (odd steps)
-    double* d_part = nullptr; // gravity: per-chunk partial accelerations
-    int grav_chunks = 1;
+    double* d_part = nullptr; // gravity: partial accelerations (see nbx_gravity.hip)
+    size_t part_doubles = 0;  // their size
     int grav_tpt_set = 0;     // targets per thread of the gravity kernel (0: by size)
     int grav_chunks_set = 0;  // source chunks of the gravity kernel (0: by size)
     bool equal_masses = false;  // every body has mass h_ms[0] (gravity takes m out of the sum)

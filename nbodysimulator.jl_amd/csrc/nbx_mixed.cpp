@@ -20,8 +20,6 @@
 
 #include "nbx_mixed.h"
 
-int mx_gravity_chunks(const nbx_ctx* c);
-
 namespace {
 
 enum { PLAN_NONBONDED = 1, PLAN_WATER = 2, PLAN_GRAVITY = 3, PLAN_MAGNETIC = 4 };
@@ -408,12 +406,12 @@ static int prepare(nbx_ctx* c, mx_plan& p, double grow) {
         NBX_HIP(c, hipMalloc((void**)&c->d_x2, sizeof(double) * 3 * (size_t)std::max<int64_t>(n, 1)));
     if (!c->d_step) NBX_HIP(c, hipMalloc((void**)&c->d_step, sizeof(int64_t)));
     if (all_pairs_tiled(p)) {
-        const int chunks = p.kind == PLAN_GRAVITY ? mx_gravity_chunks(c) : 1;
-        if (!c->d_part || c->grav_chunks != chunks) {
+        const size_t doubles = p.kind == PLAN_GRAVITY ? mx_gravity_shape(c).part_doubles : 3 * (size_t)n;
+        if (!c->d_part || c->part_doubles != doubles) {
             if (c->d_part) (void)hipFree(c->d_part);
             c->d_part = nullptr;
-            NBX_HIP(c, hipMalloc((void**)&c->d_part, sizeof(double) * 3 * (size_t)n * chunks));
-            c->grav_chunks = chunks;
+            NBX_HIP(c, hipMalloc((void**)&c->d_part, sizeof(double) * std::max<size_t>(doubles, 1)));
+            c->part_doubles = doubles;
         }
     }
     if (p.kind == PLAN_GRAVITY || !p.nb.mode_list) {
@@ -695,7 +693,7 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
         key.flags = c->nl.d_flags;
         key.pos = c->d_pos;
         key.part = c->d_part;
-        key.chunks = c->grav_chunks;
+        key.chunks = c->grav_chunks_set;
         key.tpt = c->grav_tpt_set;
         key.em = c->em;
         key.cap = c->nl.cap;
@@ -1510,8 +1508,8 @@ int mx_autotune(nbx_ctx* c, double dt, int trial, double* out, int nout) {
         }
         c->grav_tpt_set = (int)best0;
         c->grav_chunks_set = (int)best1;
-        if (!c->grav_tpt_set) best0 = n >= 16384 ? 2 : 1;
-        if (!c->grav_chunks_set) best1 = mx_gravity_chunks(c);
+        if (!c->grav_tpt_set) best0 = mx_gravity_shape(c).tpt;
+        if (!c->grav_chunks_set) best1 = mx_gravity_shape(c).chunks;
     } else {
         const int lanes0 = c->nl.lanes;
         const double skin0 = c->skin;

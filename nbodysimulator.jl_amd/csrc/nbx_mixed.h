@@ -412,6 +412,20 @@ void mx_launch_temperature(hipStream_t s, const nbx_ctx* c, const double* v, int
 void mx_launch_count_pairs(hipStream_t s, const nbx_ctx* c, const mx_nb_launch& L,
                            const void* pos, const mx_pair_params& pp,
                            unsigned long long* d_count);
+// launch shape of the gravity kernel for a context, and the partial slots of one of its
+// launches (nbx_gravity.hip)
+struct mx_grav_shape {
+    bool wide;            // the block's wavefronts hold different targets
+    int tpt;              // targets per lane
+    int S, tiles;         // bodies per tile, tiles
+    int chunks;           // blocks per target tile
+    int passes, per_pass; // launches per force evaluation, ring offsets per launch
+    size_t part_doubles;  // size of the partials
+};
+struct mx_grav_slots {
+    int tiles, S, chunks, o0, o1;
+};
+mx_grav_shape mx_gravity_shape(const nbx_ctx* c);
 void mx_launch_gravity(hipStream_t s, const nbx_ctx* c, const void* pos, double G,
                        const mx_kick_params& kp, const mx_io& io, int force_only_kernel,
                        hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
