@@ -43,6 +43,8 @@ static void release(nbx_ctx* c) {
     free_ptr(c->d_x); free_ptr(c->d_v); free_ptr(c->d_a); free_ptr(c->d_vh);
     free_ptr(c->d_tmp); free_ptr(c->d_ms); free_ptr(c->d_qs); free_ptr(c->d_red);
     free_ptr(c->d_scal);
+    free_ptr(c->d_rdf_work);
+    c->d_rdf_work = nullptr;
     free_ptr(c->d_mm);
     free_ptr(c->d_mm4);
     if (c->d_perm) (void)hipFree(c->d_perm);
@@ -829,22 +831,32 @@ extern "C" int nbx_rdf(nbx_ctx* c, const double* frames, int64_t nframes, int64_
     const int jstride = water ? 3 : 1;
     const int64_t nj = water ? c->n / 3 : c->n;
     const double L = c->bc.b[0];
-    unsigned long long* d_hist = nullptr;
-    NBX_HIP(c, hipMalloc((void**)&d_hist, sizeof(unsigned long long) * (size_t)(maxbin + 1)));
-    (void)hipMemsetAsync(d_hist, 0, sizeof(unsigned long long) * (size_t)(maxbin + 1), c->stream);
-    const size_t b = sizeof(double) * (size_t)(3 * c->n);
-    for (int64_t t = 0; t < nframes; ++t) {
-        hipError_t e = hipMemcpyAsync(c->d_tmp, frames + t * 3 * c->n, b, hipMemcpyHostToDevice,
-                                      c->stream);
-        if (e != hipSuccess) { free_ptr(d_hist); return nbx_fail(c, NBX_ERR_DEVICE, "rdf copy"); }
-        ref64_rdf_hist(c->stream, c->d_tmp, c->n, jstride, nj, L, maxbin, d_hist);
+    // frames go over in batches of at most 32 MiB (one frame at least), each batch one copy
+    // and one launch; the workspace stays with the context
+    const int64_t n3 = 3 * c->n;
+    const int64_t batch = std::max<int64_t>(1, std::min<int64_t>(nframes, ((int64_t)4 << 20) / std::max<int64_t>(n3, 1)));
+    const size_t work = (size_t)(batch * n3 + maxbin + 1);
+    if (c->rdf_work_doubles < work) {
+        free_ptr(c->d_rdf_work);
+        c->d_rdf_work = nullptr;
+        c->rdf_work_doubles = 0;
+        NBX_HIP(c, hipMalloc((void**)&c->d_rdf_work, sizeof(double) * work));
+        c->rdf_work_doubles = work;
     }
+    auto* d_hist = reinterpret_cast<unsigned long long*>(c->d_rdf_work + batch * n3);
+    ref64_zero_u64(c->stream, d_hist, maxbin + 1);
+    for (int64_t t = 0; t < nframes; t += batch) {
+        const int64_t k = std::min(batch, nframes - t);
+        if (n3 > 0)
+            NBX_HIP(c, hipMemcpyAsync(c->d_rdf_work, frames + t * n3, sizeof(double) * (size_t)(k * n3),
+                                      hipMemcpyHostToDevice, c->stream));
+        ref64_rdf_hist(c->stream, c->d_rdf_work, k, c->n, jstride, nj, L, maxbin, d_hist);
+    }
+    NBX_HIP(c, hipGetLastError());
     std::vector<unsigned long long> h((size_t)maxbin + 1);
-    hipError_t e = hipMemcpyAsync(h.data(), d_hist, sizeof(unsigned long long) * h.size(),
-                                  hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    free_ptr(d_hist);
-    if (e != hipSuccess) return nbx_fail(c, NBX_ERR_DEVICE, "rdf histogram copy");
+    NBX_HIP(c, hipMemcpyAsync(h.data(), d_hist, sizeof(unsigned long long) * h.size(),
+                              hipMemcpyDeviceToHost, c->stream));
+    NBX_HIP(c, hipStreamSynchronize(c->stream));
     rdf_normalize(h.data() + 1, nframes, nj, L, maxbin, rs, gr);
     return NBX_OK;
 }
@@ -872,7 +884,7 @@ extern "C" int nbx_rdf_noalloc(nbx_ctx* c, const double* frames, int64_t nframes
     for (int64_t t = 0; t < nframes; ++t) {
         NBX_HIP(c, hipMemcpyAsync(c->d_tmp, frames + t * 3 * c->n, b, hipMemcpyHostToDevice,
                                   c->stream));
-        ref64_rdf_hist(c->stream, c->d_tmp, c->n, jstride, nj, L, maxbin, hist);
+        ref64_rdf_hist(c->stream, c->d_tmp, 1, c->n, jstride, nj, L, maxbin, hist);
     }
     NBX_HIP(c, hipGetLastError());
     // the counts of bins 1..maxbin land in gr (8 bytes each) and are turned into g(r) there,

@@ -16,12 +16,23 @@ struct nbx_bcv {
 // while x >= radius: x -= size; while x < -radius: x += size
 // (src/boundary_conditions.jl:143-160), capped at NBX_WRAP_PASSES passes, after
 // which the remainder is removed with floor() (the reference would keep looping).
-__device__ __forceinline__ double nbx_wrap_cubic(double x, double size, double radius) {
+__device__ __forceinline__ double nbx_wrap_cubic_loop(double x, double size, double radius) {
     int k = 0;
     while (x >= radius && k < NBX_WRAP_PASSES) { x -= size; ++k; }
     while (x < -radius && k < NBX_WRAP_PASSES) { x += size; ++k; }
     if (k >= NBX_WRAP_PASSES && isfinite(x)) x -= size * floor((x + radius) / size);
     return x;
+}
+
+// One pass of each loop as selects, which is the loops' result unless a coordinate is more
+// than one box away (then every lane takes the loops): no divergent branch for the
+// displacements of neighbouring images.
+__device__ __forceinline__ double nbx_wrap_cubic(double x, double size, double radius) {
+    const double y = x >= radius ? x - size : x;
+    const double z = y < -radius ? y + size : y;
+    if (__builtin_expect(__any(y >= radius || z < -radius), 0))
+        return nbx_wrap_cubic_loop(x, size, radius);
+    return z;
 }
 
 // while x < lo: x += hi - lo; while x >= hi: x -= hi - lo

@@ -123,6 +123,8 @@ struct nbx_ctx {
     double* d_vh = nullptr;   // half-kicked velocities, 3n
     double* d_tmp = nullptr;  // scratch 3n (host transfers, rhs)
     unsigned long long* d_rdf_hist = nullptr;  // device address of the rdf_noalloc histogram
+    double* d_rdf_work = nullptr;  // nbx_rdf: frames in transfer and its histogram
+    size_t rdf_work_doubles = 0;
     double* d_ms = nullptr;
     double* d_qs = nullptr;
     double* d_mm = nullptr;   // magnetic moments (SoA 3n), when set
@@ -255,8 +257,10 @@ void ref64_grav_pe(hipStream_t s, const double* x, const double* ms, int64_t n, 
                    double* d_tmp, double* d_out);
 void ref64_bonded_pe(hipStream_t s, const double* x, int64_t n, double rOH, double kbond,
                      double aHOH, double ka, double* d_tmp, double* d_out2);
-void ref64_rdf_hist(hipStream_t s, const double* frame_aos, int64_t n, int jstride,
-                    int64_t nj, double L, int64_t maxbin, unsigned long long* d_hist);
+// adds twice the pairs i < j of every frame (3 x n each, consecutive) to hist[bin]
+void ref64_rdf_hist(hipStream_t s, const double* frames_aos, int64_t nframes, int64_t n,
+                    int jstride, int64_t nj, double L, int64_t maxbin,
+                    unsigned long long* d_hist);
 // address of the library-owned rdf histogram array on `device` (looked up once per device
 // with hipGetSymbolAddress, with that device current); 0 or -1
 #define NBX_MAX_DEVICES 64
