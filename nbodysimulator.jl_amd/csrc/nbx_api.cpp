@@ -487,11 +487,11 @@ static int ref_rhs(nbx_ctx* c, const double* x, const double* v, double* dv, dou
     }
     const int64_t Nc = c->sys == NBX_SYS_WATER ? 2 * (n / 3) : 0;
     if (c->therm == NBX_THERM_BERENDSEN) {
-        ref64_temperature(s, v, c->d_ms, n, c->kb, Nc, c->d_red, c->d_scal);
+        ref64_temperature(s, v, c->d_ms, n, c->kb, Nc, c->d_scal);
         ref64_berendsen(s, dv, v, n, c->d_scal, c->therm_T, 0.5 / c->therm_p);
     } else if (c->therm == NBX_THERM_NOSEHOOVER) {
         // src/thermostats.jl:116-122 (md_temperature over the n atoms, ndf = 3n - Nc)
-        ref64_temperature(s, v, c->d_ms, n, c->kb, Nc, c->d_red, c->d_scal);
+        ref64_temperature(s, v, c->d_ms, n, c->kb, Nc, c->d_scal);
         ref64_nosehoover(s, dv, v, n, c->d_scal, xi_out, c->therm_T, c->therm_p, 3 * n - Nc);
     }
     NBX_HIP(c, hipGetLastError());
@@ -741,51 +741,76 @@ extern "C" int nbx_energies(nbx_ctx* c, double* ke, double* pe, double* pe_grav)
     if (rc) return rc;
     hipStream_t s = c->stream;
     const int64_t n = c->n;
-    double* out = c->d_scal + 1;  // [1] ke, [2..7] terms
-    ref64_fill(s, out, 7, 0.0);
-    ref64_kinetic(s, c->d_v, c->d_ms, n, c->d_tmp, out);
-    double grav = 0.0;
-    auto fetch = [&](double* d) -> double {
-        double h = 0.0;
-        (void)hipMemcpyAsync(&h, d, sizeof(double), hipMemcpyDeviceToHost, s);
-        (void)hipStreamSynchronize(s);
-        return h;
+    // every sum is enqueued, then all of them are read at once: out[0] the kinetic energy,
+    // then a slot per potential term (the scalars up to the finite flag hold few: more
+    // terms are read in several rounds)
+    double* out = c->d_scal + 1;
+    constexpr int SLOTS = 7;   // d_scal[1..7]
+    double h_ke = 0.0, h_pe = 0.0, grav = 0.0;
+    struct slot { int at; double factor; double* into; };
+    std::vector<slot> want;
+    int used = 1;
+    const auto collect = [&]() -> int {
+        double h[SLOTS];
+        NBX_HIP(c, hipGetLastError());
+        NBX_HIP(c, hipMemcpyAsync(h, out, sizeof(double) * (size_t)used, hipMemcpyDeviceToHost, s));
+        NBX_HIP(c, hipStreamSynchronize(s));
+        for (const slot& w : want) *w.into += w.factor * h[w.at];
+        want.clear();
+        used = 1;
+        return NBX_OK;
     };
-    const double h_ke = fetch(out);
-    double h_pe = 0.0;
-    if (c->sys == NBX_SYS_WATER) {
+    const auto take = [&](int count) -> int { return used + count > SLOTS ? collect() : NBX_OK; };
+    ref64_ke kin{c->d_v, c->d_ms, out};   // the first pair sum's launch adds it
+    const bool pairs = c->sys == NBX_SYS_WATER ||
+                       std::any_of(c->terms.begin(), c->terms.end(), [](const nbx_term& t) {
+                           return t.kind == NBX_TERM_LJ || t.kind == NBX_TERM_ELEC ||
+                                  t.kind == NBX_TERM_RF;
+                       });
+    if (!pairs || n <= 0) {
+        ref64_kinetic(s, c->d_v, c->d_ms, n, out);
+        kin.out = nullptr;
+    }
+    want.push_back({0, 1.0, &h_ke});
+    const auto lj_term = [&](const nbx_term& t, int stride, int64_t nj) {
+        ref64_lj_pe(s, c->d_x, n, stride, nj, t.p[1], t.p[2], c->bc, c->d_red, out + used, kin);
+        kin.out = nullptr;
+        want.push_back({used++, 4.0 * t.p[0], &h_pe});
+    };
+    const auto elec_term = [&](const nbx_term& t, int water) {
+        ref64_elec_pe(s, c->d_x, c->d_qs, n, water, t.p[1], t.kind == NBX_TERM_RF, t.p[2], c->bc,
+                      c->d_red, out + used, kin);
+        kin.out = nullptr;
+        want.push_back({used++, t.p[0], &h_pe});
+    };
+    if (n > 0 && c->sys == NBX_SYS_WATER) {
         // src/nbody_simulation_result.jl:266-291: LJ (O atoms), electrostatic, bonds, angles
-        const nbx_term& lj = c->water_lj;
-        ref64_lj_pe(s, c->d_x, n, 3, n / 3, lj.p[0], lj.p[1], lj.p[2], c->bc, c->d_tmp, out + 1);
-        h_pe += 4.0 * lj.p[0] * fetch(out + 1);
-        const nbx_term& el = c->water_elec;
-        ref64_elec_pe(s, c->d_x, c->d_qs, n, 1, el.p[0], el.p[1], el.kind == NBX_TERM_RF, el.p[2],
-                      c->bc, c->d_tmp, out + 2);
-        h_pe += fetch(out + 2) * el.p[0];
-        ref64_bonded_pe(s, c->d_x, n, c->rOH, c->kbond, c->aHOH, c->kangle, c->d_tmp, out + 3);
-        h_pe += fetch(out + 3);
-        h_pe += fetch(out + 4);
-    } else {
+        lj_term(c->water_lj, 3, n / 3);
+        elec_term(c->water_elec, 1);
+        ref64_bonded_pe(s, c->d_x, n, c->rOH, c->kbond, c->aHOH, c->kangle, c->d_tmp, out + used);
+        want.push_back({used++, 1.0, &h_pe});
+        want.push_back({used++, 1.0, &h_pe});
+    } else if (n > 0) {
         // src/nbody_simulation_result.jl:239-264: Lennard-Jones first, then electrostatics;
         // gravity has no potential energy there and is reported separately
         for (const nbx_term& t : c->terms) {
             if (t.kind != NBX_TERM_LJ) continue;
-            ref64_lj_pe(s, c->d_x, n, 1, n, t.p[0], t.p[1], t.p[2], c->bc, c->d_tmp, out + 1);
-            h_pe += 4.0 * t.p[0] * fetch(out + 1);
+            if ((rc = take(1))) return rc;
+            lj_term(t, 1, n);
         }
         for (const nbx_term& t : c->terms) {
             if (t.kind != NBX_TERM_ELEC && t.kind != NBX_TERM_RF) continue;
-            ref64_elec_pe(s, c->d_x, c->d_qs, n, 0, t.p[0], t.p[1], t.kind == NBX_TERM_RF,
-                          t.p[2], c->bc, c->d_tmp, out + 2);
-            h_pe += fetch(out + 2) * t.p[0];
+            if ((rc = take(1))) return rc;
+            elec_term(t, 0);
         }
         for (const nbx_term& t : c->terms) {
             if (t.kind != NBX_TERM_GRAV) continue;
-            ref64_grav_pe(s, c->d_x, c->d_ms, n, t.p[0], c->d_tmp, out + 3);
-            grav += fetch(out + 3);
+            if ((rc = take(1))) return rc;
+            ref64_grav_pe(s, c->d_x, c->d_ms, n, t.p[0], c->d_tmp, out + used);
+            want.push_back({used++, 1.0, &grav});
         }
     }
-    NBX_HIP(c, hipGetLastError());
+    if ((rc = collect())) return rc;
     if (ke) *ke = h_ke;
     if (pe) *pe = h_pe;
     if (pe_grav) *pe_grav = grav;
@@ -797,7 +822,7 @@ extern "C" int nbx_temperature(nbx_ctx* c, double* T) {
     if (!c->state_set) return nbx_fail(c, NBX_ERR_INVALID, "no state set");
     const int64_t Nc = c->sys == NBX_SYS_WATER ? 2 * (c->n / 3) : 0;
     if (c->n == 0) { *T = NAN; return NBX_OK; }
-    ref64_temperature(c->stream, c->d_v, c->d_ms, c->n, c->kb, Nc, c->d_tmp, c->d_scal + 9);
+    ref64_temperature(c->stream, c->d_v, c->d_ms, c->n, c->kb, Nc, c->d_scal + 9);
     NBX_HIP(c, hipMemcpyAsync(T, c->d_scal + 9, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     NBX_HIP(c, hipStreamSynchronize(c->stream));
     return NBX_OK;

@@ -230,7 +230,7 @@ void ref64_angle(hipStream_t s, const double* x, double* dv, const double* ms, i
                  int64_t mb, int64_t me, double aHOH, double ka);
 // T = sum m v^2 / (kb (3N - Nc)) into *d_T (sequential order), then dv += ... (Berendsen)
 void ref64_temperature(hipStream_t s, const double* v, const double* ms, int64_t n,
-                       double kb, int64_t Nc, double* d_tmp, double* d_T);
+                       double kb, int64_t Nc, double* d_T);
 void ref64_berendsen(hipStream_t s, double* dv, const double* v, int64_t n, const double* d_T,
                      double T0, double gamma);
 // VV pieces
@@ -245,14 +245,23 @@ void ref64_langevin_half(hipStream_t s, double* v, const double* ms, int64_t n, 
                          uint32_t stream);
 void ref64_andersen(hipStream_t s, double* v, const double* ms, int64_t n, int water,
                     double kb, double T, double prob, uint64_t seed, int64_t step);
-// energies: per-term sums into *d_out (FP64, sequential final sum)
-void ref64_kinetic(hipStream_t s, const double* v, const double* ms, int64_t n, double* d_tmp,
+// energies: sums into *d_out (FP64).  Kinetic energy, gravity, bonds and angles in the
+// reference's order; Lennard-Jones (without the factor 4 eps) and electrostatics (without
+// k) over tiles of pairs, block partials in d_part (8,192 doubles)
+void ref64_kinetic(hipStream_t s, const double* v, const double* ms, int64_t n,
                    double* d_out);
-void ref64_lj_pe(hipStream_t s, const double* x, int64_t n, int jstride, int64_t nj, double eps,
-                 double sigma, double R, const nbx_bcv& bc, double* d_tmp, double* d_out);
+// kinetic energy added by the same launch (out = nullptr: not)
+struct ref64_ke {
+    const double* v;
+    const double* ms;
+    double* out;
+};
+void ref64_lj_pe(hipStream_t s, const double* x, int64_t n, int jstride, int64_t nj,
+                 double sigma, double R, const nbx_bcv& bc, double* d_part, double* d_out,
+                 const ref64_ke& ke);
 void ref64_elec_pe(hipStream_t s, const double* x, const double* qs, int64_t n, int water,
-                   double k, double R, int rf, double eps_rf, const nbx_bcv& bc,
-                   double* d_tmp, double* d_out);
+                   double R, int rf, double eps_rf, const nbx_bcv& bc, double* d_part,
+                   double* d_out, const ref64_ke& ke);
 void ref64_grav_pe(hipStream_t s, const double* x, const double* ms, int64_t n, double G,
                    double* d_tmp, double* d_out);
 void ref64_bonded_pe(hipStream_t s, const double* x, int64_t n, double rOH, double kbond,

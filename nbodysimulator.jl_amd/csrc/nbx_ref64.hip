@@ -425,33 +425,85 @@ void ref64_angle(hipStream_t s, const double* x, double* dv, const double* ms, i
 // Temperature and Berendsen: src/thermostats.jl:76-91
 // ---------------------------------------------------------------------------
 
-// per-atom terms in parallel, then one thread sums them in index order
-__global__ void k_ref_m_v2(const double* __restrict__ v, const double* __restrict__ ms,
-                           int64_t n, double half_mass, double* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double a = v[i], b = v[n + i], c = v[2 * n + i];
-    double s = a * a + b * b;
-    s = s + c * c;
-    if (half_mass != 0.0) out[i] = s * (ms[i] / 2.0);   // kinetic_energy term
-    else out[i] = ms[i] * s;                             // md_temperature term
+// Sum of term(0) .. term(count - 1) in index order, by one block of 256 threads: the block
+// computes 1,024 terms at a time into LDS (the next ones while these are added) and the
+// first wavefront adds them one after another, every lane the same sum.  Bound by the
+// dependent FP64 adds of a single wavefront, 5.6 ns per term (one thread reading its terms
+// from memory took 51 ns; 10,976 terms 560 -> 62 us; batches of 64 terms per LDS wait, and
+// reading ahead of the adds, measured the same or slower).  The result is valid in
+// wavefront 0.
+#define SEQ_CHUNK 1024
+template <class Term>
+__device__ __forceinline__ double ref_ordered_sum(int64_t count, Term term) {
+    __shared__ __attribute__((aligned(16))) double buf[2][SEQ_CHUNK];
+    const int tid = threadIdx.x;
+    constexpr int PER = SEQ_CHUNK / 256;
+    double w[PER];
+    const auto fetch = [&](int64_t base) {
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int64_t i = base + tid + q * 256;
+            w[q] = i < count ? term(i) : 0.0;
+        }
+    };
+    double e = 0.0;
+    fetch(0);
+    int par = 0;
+    for (int64_t base = 0; base < count; base += SEQ_CHUNK, par ^= 1) {
+#pragma unroll
+        for (int q = 0; q < PER; ++q) buf[par][tid + q * 256] = w[q];
+        __syncthreads();   // the other buffer is written after the adds of the chunk before it
+        if (base + SEQ_CHUNK < count) fetch(base + SEQ_CHUNK);
+        if (tid < 64) {
+            const int cnt = (int)(count - base < SEQ_CHUNK ? count - base : SEQ_CHUNK);
+            const double* p = buf[par];
+            int q = 0;
+            for (; q + 16 <= cnt; q += 16) {
+                double t[16];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) t[u] = p[q + u];
+#pragma unroll
+                for (int u = 0; u < 16; ++u) e += t[u];
+            }
+            for (; q < cnt; ++q) e += p[q];
+        }
+    }
+    return e;
 }
 
-// mode 0: out = e; 1: out = e / c; 2: out = c * e
-__global__ void k_seq_sum(const double* __restrict__ terms, int64_t count, int mode, double c,
-                          double* __restrict__ out) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double e = 0.0;
-    for (int64_t i = 0; i < count; ++i) e += terms[i];
-    out[0] = mode == 1 ? e / c : (mode == 2 ? c * e : e);
+// term i of the kinetic energy (half mass) or of md_temperature
+__device__ __forceinline__ double ref_mv2(const double* __restrict__ v,
+                                          const double* __restrict__ ms, int64_t n, int64_t i,
+                                          bool half_mass) {
+    const double a = v[i], b = v[n + i], c = v[2 * n + i];
+    double s = a * a + b * b;
+    s = s + c * c;
+    return half_mass ? s * (ms[i] / 2.0) : ms[i] * s;
+}
+
+// mode 0: out = sum; 1: out = sum / c; 2: out = c * sum
+__device__ __forceinline__ void ref_store_sum(double e, int mode, double c, double* out) {
+    if (threadIdx.x == 0) out[0] = mode == 1 ? e / c : (mode == 2 ? c * e : e);
+}
+
+__global__ void __launch_bounds__(256)
+k_seq_sum(const double* __restrict__ terms, int64_t count, int mode, double c,
+          double* __restrict__ out) {
+    ref_store_sum(ref_ordered_sum(count, [&](int64_t i) { return terms[i]; }), mode, c, out);
+}
+
+__global__ void __launch_bounds__(256)
+k_seq_mv2(const double* __restrict__ v, const double* __restrict__ ms, int64_t n, int half_mass,
+          int mode, double c, double* __restrict__ out) {
+    const bool half = half_mass != 0;
+    ref_store_sum(ref_ordered_sum(n, [&](int64_t i) { return ref_mv2(v, ms, n, i, half); }), mode,
+                  c, out);
 }
 
 void ref64_temperature(hipStream_t s, const double* v, const double* ms, int64_t n,
-                       double kb, int64_t Nc, double* d_tmp, double* d_T) {
+                       double kb, int64_t Nc, double* d_T) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_ref_m_v2, dim3(nbx_blocks(n, 256)), dim3(256), 0, s, v, ms, n, 0.0,
-                       d_tmp);
-    hipLaunchKernelGGL(k_seq_sum, dim3(1), dim3(64), 0, s, d_tmp, n, 1,
+    hipLaunchKernelGGL(k_seq_mv2, dim3(1), dim3(256), 0, s, v, ms, n, 0, 1,
                        kb * (double)(3 * n - Nc), d_T);
 }
 
@@ -588,74 +640,155 @@ void ref64_andersen(hipStream_t s, double* v, const double* ms, int64_t n, int w
 // Energies: src/nbody_simulation_result.jl:209-397
 // ---------------------------------------------------------------------------
 
-void ref64_kinetic(hipStream_t s, const double* v, const double* ms, int64_t n, double* d_tmp,
+void ref64_kinetic(hipStream_t s, const double* v, const double* ms, int64_t n,
                    double* d_out) {
     if (n <= 0) { ref64_fill(s, d_out, 1, 0.0); return; }
-    hipLaunchKernelGGL(k_ref_m_v2, dim3(nbx_blocks(n, 256)), dim3(256), 0, s, v, ms, n, 1.0,
-                       d_tmp);
-    hipLaunchKernelGGL(k_seq_sum, dim3(1), dim3(64), 0, s, d_tmp, n, 0, 0.0, d_out);
+    hipLaunchKernelGGL(k_seq_mv2, dim3(1), dim3(256), 0, s, v, ms, n, 1, 0, 0.0, d_out);
 }
 
-// LJ energy: per-i partial sums over the later atoms of the index set
-__global__ void k_ref_lj_pe(const double* __restrict__ x, int64_t n, int jstride, int64_t nj,
-                            double s2, double R2, nbx_bcv bc, double* __restrict__ out) {
-    const int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= nj) return;
-    const int64_t i = a * jstride;
-    const double xi = x[i], yi = x[n + i], zi = x[2 * n + i];
+// Pair energies of the pairs i < j of nj atoms: a wavefront takes 64 x 64 tiles of the upper
+// triangle (64 atoms i in its lanes, 64 atoms j from LDS), adds per lane in FP64, and the
+// lanes, wavefronts and blocks are added in a fixed order (k_ref_pe_sum).  Bound by FP64
+// VALU work; one thread per atom i with the triangle's long and short rows took 5,300 us for
+// 10,976 Lennard-Jones atoms, this takes 108.
+//   LJ (:293-319): 4 (s12 - s6), a pair beyond the cutoff at the cutoff's value; those are
+//   counted and their constant is added once per lane.
+//   Coulomb (:321-351): q_j / r, beyond the cutoff q_j / R; reaction field: in the cutoff only.
+// Block 0 of the launch adds the kinetic energy in index order meanwhile (ke_out).
+enum { REF_PE_LJ = 0, REF_PE_COULOMB = 1, REF_PE_RF = 2 };
+struct ref_pe_law {
+    double s2, R, R2, krf, crf;
+    int jstride, water;
+};
+
+template <int KIND>
+__global__ void __launch_bounds__(256)
+k_ref_pair_pe(const double* __restrict__ x, const double* __restrict__ qs, int64_t n, int64_t nj,
+              ref_pe_law law, nbx_bcv bc, double* __restrict__ part,
+              const double* __restrict__ v, const double* __restrict__ ms,
+              double* __restrict__ ke_out) {
+    if (blockIdx.x == 0) {
+        if (ke_out != nullptr)
+            ref_store_sum(ref_ordered_sum(n, [&](int64_t i) { return ref_mv2(v, ms, n, i, true); }),
+                          0, 0.0, ke_out);
+        return;
+    }
+    __shared__ double sj[4][64][4];
+    __shared__ double red[4];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t T = (nj + 63) >> 6, items = T * (T + 1) / 2;
     double e = 0.0;
-    for (int64_t b = a + 1; b < nj; ++b) {
-        const int64_t j = b * jstride;
-        double rx, ry, rz, r2;
-        nbx_displacement(xi, yi, zi, x[j], x[n + j], x[2 * n + j], bc, rx, ry, rz, r2);
-        if (!(r2 < R2)) r2 = R2;                    // :308-310
-        double q = s2 / r2;
-        double s6 = q * q * q;
-        double s12 = s6 * s6;
-        e += (s12 - s6);
-    }
-    out[a] = e;
-}
-
-void ref64_lj_pe(hipStream_t s, const double* x, int64_t n, int jstride, int64_t nj, double eps,
-                 double sigma, double R, const nbx_bcv& bc, double* d_tmp, double* d_out) {
-    if (nj <= 0) { ref64_fill(s, d_out, 1, 0.0); return; }
-    hipLaunchKernelGGL(k_ref_lj_pe, dim3(nbx_blocks(nj, 128)), dim3(128), 0, s, x, n, jstride,
-                       nj, sigma * sigma, R * R, bc, d_tmp);
-    hipLaunchKernelGGL(k_seq_sum, dim3(1), dim3(64), 0, s, d_tmp, nj, 0, 0.0, d_out);
-}
-
-// Coulomb energy (:321-351): e += (sum_j>i q_j / r) * q_i, then * k
-__global__ void k_ref_elec_pe(const double* __restrict__ x, const double* __restrict__ qs,
-                              int64_t n, int water, double R, double R2, int rf, double krf,
-                              double crf, nbx_bcv bc, double* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double xi = x[i], yi = x[n + i], zi = x[2 * n + i];
-    double ei = 0.0;
-    for (int64_t j = i + 1; j < n; ++j) {
-        if (ref_excluded(i, j, water)) continue;
-        double rx, ry, rz, r2;
-        nbx_displacement(xi, yi, zi, x[j], x[n + j], x[2 * n + j], bc, rx, ry, rz, r2);
-        if (rf) {
-            if (r2 < R2) ei += qs[j] * (1.0 / sqrt(r2) + krf * r2 - crf);
-        } else {
-            if (r2 < R2) ei += qs[j] / sqrt(r2);
-            else ei += qs[j] / R;
+    int64_t far = 0;
+    for (int64_t it = (int64_t)(blockIdx.x - 1) * 4 + wave; it < items;
+         it += (int64_t)(gridDim.x - 1) * 4) {
+        // row J of the triangle holds the tiles I = 0..J
+        int64_t J = (int64_t)((sqrt(8.0 * (double)it + 1.0) - 1.0) * 0.5);
+        while (J * (J + 1) / 2 > it) --J;
+        while ((J + 1) * (J + 2) / 2 <= it) ++J;
+        const int64_t I = it - J * (J + 1) / 2;
+        const int64_t a = (I << 6) + lane, b0 = J << 6;
+        const int nb = (int)(nj - b0 < 64 ? nj - b0 : 64);
+        double xi = 0.0, yi = 0.0, zi = 0.0, qi = 0.0;
+        if (a < nj) {
+            const int64_t i = a * law.jstride;
+            xi = x[i]; yi = x[n + i]; zi = x[2 * n + i];
+            if (KIND != REF_PE_LJ) qi = qs[i];
         }
+        if (lane < nb) {
+            const int64_t j = (b0 + lane) * law.jstride;
+            sj[wave][lane][0] = x[j]; sj[wave][lane][1] = x[n + j]; sj[wave][lane][2] = x[2 * n + j];
+            sj[wave][lane][3] = KIND != REF_PE_LJ ? qs[j] : 0.0;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        double ei = 0.0;
+        for (int k = 0; k < nb; ++k) {
+            double rx, ry, rz, r2;
+            nbx_displacement(xi, yi, zi, sj[wave][k][0], sj[wave][k][1], sj[wave][k][2], bc, rx, ry,
+                             rz, r2);
+            const bool pair = a < nj && b0 + k > a &&
+                              (KIND == REF_PE_LJ || !ref_excluded(a, b0 + k, law.water));
+            const bool in = pair && r2 < law.R2;
+            if (KIND == REF_PE_LJ) {
+                if (in) {
+                    const double q = law.s2 / r2;
+                    const double s6 = q * q * q;
+                    const double s12 = s6 * s6;
+                    ei += s12 - s6;
+                }
+                far += pair && !in;
+            } else if (KIND == REF_PE_RF) {
+                if (in) ei += sj[wave][k][3] * (1.0 / sqrt(r2) + law.krf * r2 - law.crf);
+            } else if (pair) {
+                ei += sj[wave][k][3] / (in ? sqrt(r2) : law.R);
+            }
+        }
+        e += KIND == REF_PE_LJ ? ei : ei * qi;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    out[i] = ei * qs[i];
+    if (KIND == REF_PE_LJ) {
+        const double q = law.s2 / law.R2;
+        const double s6 = q * q * q;
+        if (far) e += (double)far * (s6 * s6 - s6);   // R = Inf has no far pairs
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
+    if (lane == 0) red[wave] = e;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x - 1] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+__global__ void __launch_bounds__(256)
+k_ref_pe_sum(const double* __restrict__ part, int count, double* __restrict__ out) {
+    __shared__ double red[256];
+    double e = 0.0;
+    for (int p = threadIdx.x; p < count; p += 256) e += part[p];
+    red[threadIdx.x] = e;
+    __syncthreads();
+    for (int off = 128; off > 0; off >>= 1) {
+        if (threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[0] = red[0];
+}
+
+template <int KIND>
+static void pair_pe(hipStream_t s, const double* x, const double* qs, int64_t n, int64_t nj,
+                    const ref_pe_law& law, const nbx_bcv& bc, double* d_part, double* d_out,
+                    const ref64_ke& ke) {
+    const int64_t T = (nj + 63) >> 6;
+    // 2,048 blocks of four wavefronts fill the chip (d_part holds 8,192 doubles at least)
+    const int blocks = (int)std::min<int64_t>((T * (T + 1) / 2 + 3) / 4, 2048);
+    hipLaunchKernelGGL(k_ref_pair_pe<KIND>, dim3(blocks + 1), dim3(256), 0, s, x, qs, n, nj, law,
+                       bc, d_part, ke.v, ke.ms, ke.out);
+    hipLaunchKernelGGL(k_ref_pe_sum, dim3(1), dim3(256), 0, s, d_part, blocks, d_out);
+}
+
+void ref64_lj_pe(hipStream_t s, const double* x, int64_t n, int jstride, int64_t nj,
+                 double sigma, double R, const nbx_bcv& bc, double* d_part, double* d_out,
+                 const ref64_ke& ke) {
+    ref_pe_law law{};
+    law.s2 = sigma * sigma;
+    law.R2 = R * R;
+    law.jstride = jstride;
+    pair_pe<REF_PE_LJ>(s, x, nullptr, n, nj, law, bc, d_part, d_out, ke);
 }
 
 void ref64_elec_pe(hipStream_t s, const double* x, const double* qs, int64_t n, int water,
-                   double k, double R, int rf, double eps_rf, const nbx_bcv& bc,
-                   double* d_tmp, double* d_out) {
-    if (n <= 0) { ref64_fill(s, d_out, 1, 0.0); return; }
-    const double krf = rf ? rf_krf(R, eps_rf) : 0.0;
-    const double crf = rf ? 1.0 / R + krf * (R * R) : 0.0;
-    hipLaunchKernelGGL(k_ref_elec_pe, dim3(nbx_blocks(n, 128)), dim3(128), 0, s, x, qs, n,
-                       water, R, R * R, rf, krf, crf, bc, d_tmp);
-    hipLaunchKernelGGL(k_seq_sum, dim3(1), dim3(64), 0, s, d_tmp, n, 0, 0.0, d_out);
+                   double R, int rf, double eps_rf, const nbx_bcv& bc, double* d_part,
+                   double* d_out, const ref64_ke& ke) {
+    ref_pe_law law{};
+    law.R = R;
+    law.R2 = R * R;
+    law.jstride = 1;
+    law.water = water;
+    if (rf) {
+        law.krf = rf_krf(R, eps_rf);
+        law.crf = 1.0 / R + law.krf * (R * R);
+        pair_pe<REF_PE_RF>(s, x, qs, n, n, law, bc, d_part, d_out, ke);
+    } else {
+        pair_pe<REF_PE_COULOMB>(s, x, qs, n, n, law, bc, d_part, d_out, ke);
+    }
 }
 
 __global__ void k_ref_grav_pe(const double* __restrict__ x, const double* __restrict__ ms,
@@ -674,7 +807,7 @@ void ref64_grav_pe(hipStream_t s, const double* x, const double* ms, int64_t n, 
     if (n <= 0) { ref64_fill(s, d_out, 1, 0.0); return; }
     hipLaunchKernelGGL(k_ref_grav_pe, dim3(nbx_blocks(n, 128)), dim3(128), 0, s, x, ms, n,
                        d_tmp);
-    hipLaunchKernelGGL(k_seq_sum, dim3(1), dim3(64), 0, s, d_tmp, n, 2, -G, d_out);
+    hipLaunchKernelGGL(k_seq_sum, dim3(1), dim3(256), 0, s, d_tmp, n, 2, -G, d_out);
 }
 
 // Bonds (:353-372, each bond seen from both ends, / 4) and angles (:374-397, / 2)
@@ -703,14 +836,13 @@ __global__ void k_ref_bonded_terms(const double* __restrict__ x, int64_t n, doub
     out[4 * nmol + m] = ka * (d * d);
 }
 
-__global__ void k_ref_bonded_sum(const double* __restrict__ terms, int64_t nmol,
-                                 double* __restrict__ out2) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double eb = 0.0, ea = 0.0;
-    for (int64_t t = 0; t < 4 * nmol; ++t) eb += terms[t];
-    for (int64_t m = 0; m < nmol; ++m) ea += terms[4 * nmol + m];
-    out2[0] = eb / 4.0;
-    out2[1] = ea / 2.0;
+// block 0: the bonds, block 1: the angles
+__global__ void __launch_bounds__(256)
+k_ref_bonded_sum(const double* __restrict__ terms, int64_t nmol, double* __restrict__ out2) {
+    const int64_t first = blockIdx.x ? 4 * nmol : 0;
+    ref_store_sum(ref_ordered_sum(blockIdx.x ? nmol : 4 * nmol,
+                                  [&](int64_t t) { return terms[first + t]; }),
+                  1, blockIdx.x ? 2.0 : 4.0, out2 + blockIdx.x);
 }
 
 void ref64_bonded_pe(hipStream_t s, const double* x, int64_t n, double rOH, double kbond,
@@ -719,7 +851,7 @@ void ref64_bonded_pe(hipStream_t s, const double* x, int64_t n, double rOH, doub
     if (nmol <= 0) { ref64_fill(s, d_out2, 2, 0.0); return; }
     hipLaunchKernelGGL(k_ref_bonded_terms, dim3(nbx_blocks(nmol, 256)), dim3(256), 0, s, x, n,
                        rOH, kbond, aHOH, ka, d_tmp);
-    hipLaunchKernelGGL(k_ref_bonded_sum, dim3(1), dim3(64), 0, s, d_tmp, nmol, d_out2);
+    hipLaunchKernelGGL(k_ref_bonded_sum, dim3(2), dim3(256), 0, s, d_tmp, nmol, d_out2);
 }
 
 // ---------------------------------------------------------------------------
