@@ -43,8 +43,10 @@ static void release(nbx_ctx* c) {
     free_ptr(c->d_x); free_ptr(c->d_v); free_ptr(c->d_a); free_ptr(c->d_vh);
     free_ptr(c->d_tmp); free_ptr(c->d_ms); free_ptr(c->d_qs); free_ptr(c->d_red);
     free_ptr(c->d_scal);
-    free_ptr(c->d_rdf_work);
-    c->d_rdf_work = nullptr;
+    free_ptr(c->d_rdf_work); free_ptr(c->d_frac); free_ptr(c->d_rhs); free_ptr(c->d_water);
+    free_ptr(c->d_frames);
+    c->d_rdf_work = c->d_rhs = c->d_water = c->d_frames = nullptr;
+    c->d_frac = nullptr;
     free_ptr(c->d_mm);
     free_ptr(c->d_mm4);
     if (c->d_perm) (void)hipFree(c->d_perm);
@@ -435,36 +437,58 @@ static int check_config(nbx_ctx* c) {
     return NBX_OK;
 }
 
-// one potential term's closure for atoms [ib, ie), adding into dv (SoA)
-static void ref_term(nbx_ctx* c, const nbx_term& t, const double* x, double* dv, int64_t ib,
-                     int64_t ie) {
-    hipStream_t s = c->stream;
+// the pair kernel's form of a term; false for the terms with kernels of their own
+// (magnetic dipoles, gravity of many bodies)
+static bool ref_pair_term(const nbx_ctx* c, const nbx_term& t, ref64_term* out) {
+    if (t.kind == NBX_TERM_MAG || (t.kind == NBX_TERM_GRAV && c->n > NBX_REF_GRAV_WAVES)) return false;
+    ref64_term r{};
+    r.kind = t.kind;
+    for (int k = 0; k < 4; ++k) r.p[k] = t.p[k];
     const int water = c->sys == NBX_SYS_WATER;
-    switch (t.kind) {
-    case NBX_TERM_LJ:
-        if (water) {
-            // O atoms only, partners = O atoms (src/nbody_to_ode.jl:302-314)
-            int64_t first = ((ib + 2) / 3) * 3;
-            ref64_lj(s, x, dv, c->d_ms, c->n, first, ie, 3, 3, c->n / 3, t.p[0], t.p[1], t.p[2],
-                     c->bc);
-        } else {
-            ref64_lj(s, x, dv, c->d_ms, c->n, ib, ie, 1, 1, c->n, t.p[0], t.p[1], t.p[2], c->bc);
-        }
-        break;
-    case NBX_TERM_ELEC:
-        ref64_elec(s, x, dv, c->d_ms, c->d_qs, c->n, ib, ie, water, t.p[0], t.p[1], c->bc);
-        break;
-    case NBX_TERM_RF:
-        ref64_rf(s, x, dv, c->d_ms, c->d_qs, c->n, ib, ie, water, t.p[0], t.p[1], t.p[2], c->bc);
-        break;
-    case NBX_TERM_GRAV:
+    // water's Lennard-Jones: O atoms only, partners = O atoms (src/nbody_to_ode.jl:302-314)
+    r.istride = r.jstride = water && t.kind == NBX_TERM_LJ ? 3 : 1;
+    r.nj = c->n / r.jstride;
+    r.water = water && t.kind != NBX_TERM_LJ;
+    r.filter = ref64_filters(r, c->bc);
+    *out = r;
+    return true;
+}
+
+template <class T>
+static int ensure(nbx_ctx* c, T** p, size_t count) {
+    if (!*p) NBX_HIP(c, hipMalloc((void**)p, sizeof(T) * std::max<size_t>(count, 1)));
+    return NBX_OK;
+}
+
+// box fractions of x into the given set when a term filters its sources with them
+static int ref_fractions(nbx_ctx* c, const double* x, int set) {
+    bool any = false;
+    ref64_term r;
+    if (c->sys == NBX_SYS_WATER) {
+        for (const nbx_term* t : {&c->water_elec, &c->water_lj})
+            any = any || (t->kind && ref_pair_term(c, *t, &r) && r.filter);
+    }
+    for (const nbx_term& t : c->terms) any = any || (ref_pair_term(c, t, &r) && r.filter);
+    if (!any) return NBX_OK;
+    if (int rc = ensure(c, &c->d_frac, 2 * (size_t)c->n)) return rc;
+    ref64_fractions(c->stream, x, c->n, c->bc.b[0], c->d_frac + (size_t)set * c->n);
+    return NBX_OK;
+}
+
+// one potential term's closure for atoms [ib, ie), adding into dv (SoA); set: the box
+// fractions of x
+static void ref_term(nbx_ctx* c, const nbx_term& t, const double* x, double* dv, int64_t ib,
+                     int64_t ie, int set = 0) {
+    hipStream_t s = c->stream;
+    ref64_term r;
+    if (ref_pair_term(c, t, &r)) {
+        const int64_t first = (ib + r.istride - 1) / r.istride * r.istride;
+        ref64_pairs(s, r, x, c->d_frac ? c->d_frac + (size_t)set * c->n : nullptr, c->d_ms, c->d_qs,
+                    c->n, first, ie, c->bc, dv, nullptr);
+    } else if (t.kind == NBX_TERM_GRAV) {
         ref64_grav(s, x, dv, c->d_ms, c->n, ib, ie, t.p[0]);
-        break;
-    case NBX_TERM_MAG:
+    } else if (t.kind == NBX_TERM_MAG) {
         ref64_mag(s, x, dv, c->d_ms, c->d_mm, c->n, ib, ie, t.p[0]);
-        break;
-    default:
-        break;
     }
 }
 
@@ -474,6 +498,7 @@ static int ref_rhs(nbx_ctx* c, const double* x, const double* v, double* dv, dou
     hipStream_t s = c->stream;
     const int64_t n = c->n;
     ref64_fill(s, dv, 3 * n, 0.0);
+    if (int rc = ref_fractions(c, x, 0)) return rc;
     if (c->sys == NBX_SYS_WATER) {
         // per-atom closure order: O = (electrostatic, bond, LJ); H = (electrostatic, bond).
         // Each atom's dv only receives its own closures, so running the terms as
@@ -498,17 +523,17 @@ static int ref_rhs(nbx_ctx* c, const double* x, const double* v, double* dv, dou
     return NBX_OK;
 }
 
-// Scratch triple for calls that must not touch the context state
+// Scratch triple for calls that must not touch the context state (kept with the context)
 struct scratch3 {
     double *x = nullptr, *v = nullptr, *dv = nullptr;
-    ~scratch3() { free_ptr(x); free_ptr(v); free_ptr(dv); }
 };
 
 static int alloc_scratch(nbx_ctx* c, scratch3& s) {
-    const size_t b = sizeof(double) * (size_t)(3 * c->n);
-    NBX_HIP(c, hipMalloc((void**)&s.x, b));
-    NBX_HIP(c, hipMalloc((void**)&s.v, b));
-    NBX_HIP(c, hipMalloc((void**)&s.dv, b));
+    const size_t n3 = 3 * (size_t)c->n;
+    if (int rc = ensure(c, &c->d_rhs, 3 * n3)) return rc;
+    s.x = c->d_rhs;
+    s.v = c->d_rhs + n3;
+    s.dv = c->d_rhs + 2 * n3;
     return NBX_OK;
 }
 
@@ -524,8 +549,9 @@ extern "C" int nbx_rhs(nbx_ctx* c, const double* u, const double* v, double* dv)
     scratch3 s;
     if ((rc = alloc_scratch(c, s))) return rc;
     if ((rc = upload_aos(c, u, s.x))) return rc;
-    if (v) { if ((rc = upload_aos(c, v, s.v))) return rc; }
-    else ref64_fill(c->stream, s.v, 3 * c->n, 0.0);
+    // v enters through the thermostat terms only
+    if (c->therm == NBX_THERM_BERENDSEN || c->therm == NBX_THERM_NOSEHOOVER)
+        if ((rc = upload_aos(c, v, s.v))) return rc;
     if ((rc = ref_rhs(c, s.x, s.v, s.dv, c->d_scal + NBX_SCAL_XI_SCRATCH))) return rc;
     return download_aos(c, s.dv, dv);
 }
@@ -553,6 +579,7 @@ extern "C" int nbx_accelerations(nbx_ctx* c, int32_t term, const double* u, int6
     if ((rc = alloc_scratch(c, s))) return rc;
     if ((rc = upload_aos(c, u, s.x))) return rc;
     if ((rc = upload_aos(c, dv, s.dv))) return rc;
+    if ((rc = ref_fractions(c, s.x, 0))) return rc;
     if (c->sys == NBX_SYS_WATER) {
         if (term == 0) ref_term(c, c->water_elec, s.x, s.dv, i_begin, i_end);
         else if (term == 1) ref_term(c, c->water_lj, s.x, s.dv, i_begin, i_end);
@@ -581,11 +608,149 @@ static int save_frame(nbx_ctx* c, int64_t f, double* uf, double* vf) {
     return download_aos(c, c->d_v, vf + f * n3);
 }
 
+// Frames of an FP64 run: collected on the device in the caller's layout and copied to the
+// host many at a time (32 MiB of both arrays at most, one frame at least), not one by one with
+// two synchronisations each
+struct frame_sink {
+    nbx_ctx* c;
+    double *uf, *vf;
+    int64_t cap = 0, pending = 0, done = 0;
+
+    int open(int64_t frames) {
+        const int64_t n3 = 3 * c->n;
+        cap = std::max<int64_t>(1, std::min<int64_t>(frames, ((int64_t)2 << 20) / n3));
+        const size_t doubles = 2 * (size_t)(cap * n3);
+        if (c->frames_doubles < doubles) {
+            free_ptr(c->d_frames);
+            c->d_frames = nullptr;
+            c->frames_doubles = 0;
+            NBX_HIP(c, hipMalloc((void**)&c->d_frames, sizeof(double) * doubles));
+            c->frames_doubles = doubles;
+        }
+        return NBX_OK;
+    }
+    int add(const double* x, const double* v) {
+        const int64_t n3 = 3 * c->n;
+        ref64_save_frame(c->stream, x, v, c->d_frames + pending * n3,
+                         c->d_frames + (cap + pending) * n3, c->n);
+        return ++pending == cap ? flush() : NBX_OK;
+    }
+    int flush() {
+        const int64_t n3 = 3 * c->n;
+        if (pending == 0) return NBX_OK;
+        const size_t bytes = sizeof(double) * (size_t)(pending * n3);
+        NBX_HIP(c, hipMemcpyAsync(uf + done * n3, c->d_frames, bytes, hipMemcpyDeviceToHost, c->stream));
+        NBX_HIP(c, hipMemcpyAsync(vf + done * n3, c->d_frames + cap * n3, bytes, hipMemcpyDeviceToHost,
+                                  c->stream));
+        NBX_HIP(c, hipStreamSynchronize(c->stream));
+        done += pending;
+        pending = 0;
+        return NBX_OK;
+    }
+};
+
+// Runs whose steps end inside the kernel that completes the accelerations: water, and
+// potential systems whose last term is a pair term, with a thermostat that acts per atom or
+// through the temperature of the half-kicked velocities (Nose-Hoover advances its own
+// coordinate between the pieces)
+static bool ref_fuses(const nbx_ctx* c) {
+    if (c->therm == NBX_THERM_NOSEHOOVER) return false;
+    if (c->sys == NBX_SYS_WATER) return true;
+    ref64_term r;
+    return !c->terms.empty() && ref_pair_term(c, c->terms.back(), &r);
+}
+
+// nsteps of such a run from (d_x, d_v, d_a): positions alternate between d_x and d_x2
+// (a kernel that writes the next positions cannot overwrite those that other targets still
+// read), and end in d_x.  Launches per step: one (one more per further potential, two for
+// water, one more for Berendsen's temperature) instead of a fill, one per term, kick, drift
+// and thermostat.
+static int ref_vv_fused(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t save_every,
+                        frame_sink* frames) {
+    hipStream_t s = c->stream;
+    const int64_t n = c->n;
+    const bool water = c->sys == NBX_SYS_WATER;
+    int rc;
+    if ((rc = ensure(c, &c->d_x2, 3 * (size_t)n))) return rc;
+    if (water && (rc = ensure(c, &c->d_water, 6 * (size_t)n))) return rc;
+    ref64_term last{}, lj{};
+    bool filter = false;
+    if (water) {
+        if (!ref_pair_term(c, c->water_elec, &last) || !ref_pair_term(c, c->water_lj, &lj))
+            return nbx_fail(c, NBX_ERR_INVALID, "water takes Lennard-Jones and electrostatics");
+        filter = last.filter = lj.filter = last.filter && lj.filter;
+    } else {
+        (void)ref_pair_term(c, c->terms.back(), &last);
+        ref64_term r;
+        for (const nbx_term& t : c->terms) filter = filter || (ref_pair_term(c, t, &r) && r.filter);
+    }
+    if (filter && (rc = ensure(c, &c->d_frac, 2 * (size_t)n))) return rc;
+    double* const xb[2] = {c->d_x, c->d_x2};
+    float4* const fb[2] = {filter ? c->d_frac : nullptr, filter ? c->d_frac + n : nullptr};
+    ref64_step st{};
+    st.a = c->d_a;
+    st.v = c->d_v;
+    st.vh = c->d_vh;
+    st.d_T = c->d_scal;
+    st.dt = dt;
+    st.invL = filter ? 1.0 / c->bc.b[0] : 0.0;
+    st.kb = c->kb;
+    st.T = c->therm_T;
+    st.therm = c->therm;
+    st.seed = seed;
+    if (c->therm == NBX_THERM_LANGEVIN) {
+        st.c1 = std::exp(-c->therm_p * (0.5 * dt));
+        st.c2 = std::sqrt(1.0 - st.c1 * st.c1);
+    } else if (c->therm == NBX_THERM_ANDERSEN) {
+        st.prob = c->therm_p * dt;
+    } else if (c->therm == NBX_THERM_BERENDSEN) {
+        st.gamma = 0.5 / c->therm_p;
+    }
+    const int64_t Nc = water ? 2 * (n / 3) : 0;
+    const int64_t step0 = c->steps_taken;
+    if (c->therm == NBX_THERM_LANGEVIN)
+        ref64_langevin_half(s, c->d_v, c->d_ms, n, c->kb, c->therm_T, c->therm_p, dt, seed, step0 + 1,
+                            NBX_RNG_LANGEVIN_A);
+    ref64_drift(s, xb[0], xb[1], c->d_v, c->d_a, c->d_vh, n, dt, fb[1], c->bc.b[0]);
+    for (int64_t k = 1; k <= nsteps; ++k) {
+        const int cur = (int)(k & 1);
+        if (c->therm == NBX_THERM_BERENDSEN)
+            ref64_temperature(s, c->d_vh, c->d_ms, n, c->kb, Nc, c->d_scal);
+        st.x_in = xb[cur];
+        st.x_out = xb[cur ^ 1];
+        st.frac_out = fb[cur ^ 1];
+        st.step = step0 + k;
+        st.drift = k < nsteps;
+        if (water) {
+            ref64_water_step(s, last, lj, fb[cur], c->d_ms, c->d_qs, n, c->bc, c->d_water,
+                             c->d_water + 3 * n, c->rOH, c->kbond, c->aHOH, c->kangle, st);
+        } else {
+            if (c->terms.size() > 1) {
+                ref64_fill(s, c->d_a, 3 * n, 0.0);
+                for (size_t q = 0; q + 1 < c->terms.size(); ++q)
+                    ref_term(c, c->terms[q], xb[cur], c->d_a, 0, n, cur);
+                st.a_in = c->d_a;
+            }
+            ref64_pairs(s, last, xb[cur], fb[cur], c->d_ms, c->d_qs, n, 0, n, c->bc, nullptr, &st);
+        }
+        NBX_HIP(c, hipGetLastError());
+        c->steps_taken = step0 + k;
+        if (frames && k % save_every == 0 && (rc = frames->add(xb[cur], c->d_v))) return rc;
+    }
+    if (nsteps & 1)
+        NBX_HIP(c, hipMemcpyAsync(c->d_x, c->d_x2, sizeof(double) * 3 * (size_t)n,
+                                  hipMemcpyDeviceToDevice, s));
+    return NBX_OK;
+}
+
 static int ref_vv(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t save_every,
-                  double* uf, double* vf, int64_t* nframes) {
+                  double* uf, double* vf) {
     hipStream_t s = c->stream;
     const int64_t n = c->n;
     int rc;
+    frame_sink sink{c, uf, vf};
+    frame_sink* const frames = save_every > 0 ? &sink : nullptr;
+    if (frames && ((rc = sink.open(1 + nsteps / save_every)) || (rc = sink.add(c->d_x, c->d_v)))) return rc;
     if (c->nh_advanced && c->therm == NBX_THERM_NOSEHOOVER) {
         // a mixed run before this one left zeta and xi advanced for the next step: back to
         // the state's values, which this path advances at its first drift
@@ -598,12 +763,16 @@ static int ref_vv(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t 
         c->accel_valid = true;
     }
     const int water = c->sys == NBX_SYS_WATER;
+    if (nsteps > 0 && ref_fuses(c)) {
+        if ((rc = ref_vv_fused(c, dt, nsteps, seed, save_every, frames))) return rc;
+        return frames ? sink.flush() : NBX_OK;
+    }
     for (int64_t k = 1; k <= nsteps; ++k) {
         const int64_t step = c->steps_taken + 1;
         if (c->therm == NBX_THERM_LANGEVIN)
             ref64_langevin_half(s, c->d_v, c->d_ms, n, c->kb, c->therm_T, c->therm_p, dt, seed,
                                 step, NBX_RNG_LANGEVIN_A);
-        ref64_drift(s, c->d_x, c->d_v, c->d_a, c->d_vh, n, dt);
+        ref64_drift(s, c->d_x, c->d_x, c->d_v, c->d_a, c->d_vh, n, dt, nullptr, 1.0);
         if (c->therm == NBX_THERM_NOSEHOOVER) ref64_nh_drift(s, c->d_scal, dt);
         if ((rc = ref_rhs(c, c->d_x, c->d_vh, c->d_a, c->d_scal + NBX_SCAL_XI))) return rc;
         ref64_kick(s, c->d_v, c->d_vh, c->d_a, n, dt);
@@ -615,12 +784,9 @@ static int ref_vv(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t 
                            step);
         NBX_HIP(c, hipGetLastError());
         c->steps_taken = step;
-        if (save_every > 0 && uf && k % save_every == 0) {
-            if ((rc = save_frame(c, *nframes, uf, vf))) return rc;
-            ++*nframes;
-        }
+        if (frames && k % save_every == 0 && (rc = sink.add(c->d_x, c->d_v))) return rc;
     }
-    return NBX_OK;
+    return frames ? sink.flush() : NBX_OK;
 }
 
 int mx_vv(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t save_every, double* uf,
@@ -650,17 +816,17 @@ extern "C" int nbx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed,
     int rc = check_config(c);
     if (rc) return rc;
     if (c->n == 0) { c->steps_taken += nsteps; return NBX_OK; }
-    int64_t nframes = 0;
-    if (save_every > 0) {
-        if ((rc = save_frame(c, 0, u_frames, v_frames))) return rc;
-        nframes = 1;
-    }
     if (c->prec == NBX_PREC_MIXED) {
+        int64_t nframes = 0;
+        if (save_every > 0) {
+            if ((rc = save_frame(c, 0, u_frames, v_frames))) return rc;
+            nframes = 1;
+        }
         std::string why;
         if (!mx_supported(c, &why)) return nbx_fail(c, NBX_ERR_UNSUPPORTED, why);
         rc = mx_vv(c, dt, nsteps, seed, save_every, u_frames, v_frames, &nframes);
     } else {
-        rc = ref_vv(c, dt, nsteps, seed, save_every, u_frames, v_frames, &nframes);
+        rc = ref_vv(c, dt, nsteps, seed, save_every, u_frames, v_frames);
     }
     if (rc) return rc;
     NBX_HIP(c, hipStreamSynchronize(c->stream));
@@ -672,9 +838,12 @@ extern "C" int nbx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed,
 // ---------------------------------------------------------------------------
 
 static int ref_em(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t save_every,
-                  double* uf, double* vf, int64_t* nframes) {
+                  double* uf, double* vf) {
     hipStream_t s = c->stream;
     int rc;
+    frame_sink sink{c, uf, vf};
+    if (save_every > 0 &&
+        ((rc = sink.open(1 + nsteps / save_every)) || (rc = sink.add(c->d_x, c->d_v)))) return rc;
     if (!c->accel_valid) {
         if ((rc = ref_rhs(c, c->d_x, c->d_v, c->d_a, c->d_scal + NBX_SCAL_XI))) return rc;
         c->accel_valid = true;
@@ -686,12 +855,9 @@ static int ref_em(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t 
         if ((rc = ref_rhs(c, c->d_x, c->d_v, c->d_a, c->d_scal + NBX_SCAL_XI))) return rc;
         NBX_HIP(c, hipGetLastError());
         c->steps_taken = step;
-        if (save_every > 0 && uf && k % save_every == 0) {
-            if ((rc = save_frame(c, *nframes, uf, vf))) return rc;
-            ++*nframes;
-        }
+        if (save_every > 0 && k % save_every == 0 && (rc = sink.add(c->d_x, c->d_v))) return rc;
     }
-    return NBX_OK;
+    return save_every > 0 ? sink.flush() : NBX_OK;
 }
 
 extern "C" int nbx_em_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed,
@@ -711,19 +877,19 @@ extern "C" int nbx_em_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed,
     int rc = check_config(c);
     if (rc) return rc;
     if (c->n == 0) { c->steps_taken += nsteps; return NBX_OK; }
-    int64_t nframes = 0;
-    if (save_every > 0) {
-        if ((rc = save_frame(c, 0, u_frames, v_frames))) return rc;
-        nframes = 1;
-    }
     if (c->prec == NBX_PREC_MIXED) {
+        int64_t nframes = 0;
+        if (save_every > 0) {
+            if ((rc = save_frame(c, 0, u_frames, v_frames))) return rc;
+            nframes = 1;
+        }
         std::string why;
         if (!mx_supported(c, &why)) return nbx_fail(c, NBX_ERR_UNSUPPORTED, why);
         c->em = 1;
         rc = mx_vv(c, dt, nsteps, seed, save_every, u_frames, v_frames, &nframes);
         c->em = 0;
     } else {
-        rc = ref_em(c, dt, nsteps, seed, save_every, u_frames, v_frames, &nframes);
+        rc = ref_em(c, dt, nsteps, seed, save_every, u_frames, v_frames);
     }
     if (rc) return rc;
     NBX_HIP(c, hipStreamSynchronize(c->stream));

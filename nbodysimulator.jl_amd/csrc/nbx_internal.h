@@ -125,6 +125,12 @@ struct nbx_ctx {
     unsigned long long* d_rdf_hist = nullptr;  // device address of the rdf_noalloc histogram
     double* d_rdf_work = nullptr;  // nbx_rdf: frames in transfer and its histogram
     size_t rdf_work_doubles = 0;
+    // FP64 path workspaces, allocated when first needed and kept
+    float4* d_frac = nullptr;      // box fractions, one set per position buffer (2n)
+    double* d_rhs = nullptr;       // state-free right-hand sides: x, v, dv (9n)
+    double* d_water = nullptr;     // water: electrostatic and Lennard-Jones sums (6n)
+    double* d_frames = nullptr;    // saved frames on their way to the host
+    size_t frames_doubles = 0;
     double* d_ms = nullptr;
     double* d_qs = nullptr;
     double* d_mm = nullptr;   // magnetic moments (SoA 3n), when set
@@ -203,16 +209,55 @@ static inline unsigned nbx_blocks(int64_t work, int threads) {
 void ref64_fill(hipStream_t s, double* p, int64_t count, double value);
 void ref64_aos_to_soa(hipStream_t s, const double* aos, double* soa, int64_t n);
 void ref64_soa_to_aos(hipStream_t s, const double* soa, double* aos, int64_t n);
-// LJ: i = ib, ib+istride, ... < ie; j = 0, jstride, ..., (nj-1)*jstride
-void ref64_lj(hipStream_t s, const double* x, double* dv, const double* ms, int64_t n,
-              int64_t ib, int64_t ie, int istride, int jstride, int64_t nj, double eps,
-              double sigma, double R, const nbx_bcv& bc);
-void ref64_elec(hipStream_t s, const double* x, double* dv, const double* ms,
-                const double* qs, int64_t n, int64_t ib, int64_t ie, int water, double k,
-                double R, const nbx_bcv& bc);
-void ref64_rf(hipStream_t s, const double* x, double* dv, const double* ms, const double* qs,
-              int64_t n, int64_t ib, int64_t ie, int water, double k, double R,
-              double eps_rf, const nbx_bcv& bc);
+void ref64_save_frame(hipStream_t s, const double* x, const double* v, double* uf, double* vf,
+                      int64_t n);
+
+// a pair potential over the sources j = 0, jstride, ..., (nj - 1) jstride for targets
+// ib, ib + istride, ...; water: the atoms of a molecule exclude each other
+struct ref64_term {
+    int kind;              // NBX_TERM_LJ, _ELEC, _RF, _GRAV
+    double p[4];           // as nbx_term
+    int istride, jstride;
+    int64_t nj;
+    int water;
+    bool filter;           // sources pass the box-fraction test first (needs frac)
+};
+// whether the box-fraction test pays for a term
+bool ref64_filters(const ref64_term& t, const nbx_bcv& bc);
+// box fractions of the positions for the filter
+void ref64_fractions(hipStream_t s, const double* x, int64_t n, double L, float4* frac);
+
+// The end of a velocity-Verlet step and the start of the next one, fused into the kernel
+// that completes the accelerations (nbx_ref64.hip: ref_end_step)
+struct ref64_step {
+    const double* a_in;    // acceleration of the terms before this one (nullptr: 0)
+    const double* x_in;    // positions of the step
+    double* x_out;         // next positions (another buffer: other blocks still read x_in)
+    float4* frac_out;      // their box fractions (nullptr: none)
+    double* a;
+    double* v;
+    double* vh;            // half-kicked velocities, in and out
+    const double* d_T;     // Berendsen: temperature of vh
+    double dt, invL;
+    double kb, T, c1, c2, prob, gamma;
+    uint64_t seed;
+    int64_t step;
+    int therm;
+    int drift;             // 0: the step's end only
+};
+// one pair term: into dv, or (step) added to step->a_in and the step ended
+void ref64_pairs(hipStream_t s, const ref64_term& t, const double* x, const float4* frac,
+                 const double* ms, const double* qs, int64_t n, int64_t ib, int64_t ie,
+                 const nbx_bcv& bc, double* dv, const ref64_step* step);
+// water: every term of the right-hand side and the end of the step (elec, ljv: scratch, 3n
+// each; the two laws filter alike)
+void ref64_water_step(hipStream_t s, const ref64_term& el, const ref64_term& lj, const float4* frac,
+                      const double* ms, const double* qs, int64_t n, const nbx_bcv& bc,
+                      double* elec, double* ljv, double rOH, double kbond, double aHOH, double ka,
+                      const ref64_step& st);
+// up to this many bodies gravity gives each target a wavefront (n = 16,000: 2.0 ms per
+// evaluation against 2.9 with a thread per target; twice the bodies 8 against 5.3)
+#define NBX_REF_GRAV_WAVES 16384
 void ref64_mag(hipStream_t s, const double* x, double* dv, const double* ms, const double* mm,
                int64_t n, int64_t ib, int64_t ie, double mu_4pi);
 // Nose-Hoover (src/thermostats.jl:116-122): dv -= zeta v; xi_out = (1/tau)^2 (T/T0 - (ndf+1)/ndf)
@@ -234,8 +279,8 @@ void ref64_temperature(hipStream_t s, const double* v, const double* ms, int64_t
 void ref64_berendsen(hipStream_t s, double* dv, const double* v, int64_t n, const double* d_T,
                      double T0, double gamma);
 // VV pieces
-void ref64_drift(hipStream_t s, double* x, const double* v, const double* a, double* vh,
-                 int64_t n, double dt);
+void ref64_drift(hipStream_t s, const double* x, double* x_out, const double* v, const double* a,
+                 double* vh, int64_t n, double dt, float4* frac, double L);
 void ref64_kick(hipStream_t s, double* v, const double* vh, const double* a, int64_t n,
                 double dt);
 void ref64_em(hipStream_t s, double* x, double* v, const double* a, int64_t n, double dt,

@@ -1,12 +1,11 @@
 // nbx_ref64.hip -- FP64 kernels that reproduce the reference's arithmetic bit for bit.
 //
 // Built with -ffp-contract=off: every a*b+c rounds twice, as Julia does without
-// @fastmath/@muladd.  Every per-target sum walks the source atoms in ascending index
-// order (the reference's `for j in indxs`): gravity keeps one thread per target with
-// sources staged through LDS tiles, Lennard-Jones and Coulomb give each target a
-// wavefront whose lanes compute the pair terms of 64 sources at once before the terms
-// are added in j order.  Neither changes the order or the rounding of the sums.  Device
-// state is SoA: x[k * n + i].
+// @fastmath/@muladd.  Every per-target sum takes the source atoms in ascending index
+// order (the reference's `for j in indxs`): a target has a wavefront whose lanes compute
+// the pair terms of 64 sources at once before the terms are added in j order (gravity of
+// many bodies: one thread per target, sources staged through LDS tiles).  Neither changes
+// the order or the rounding of the sums.  Device state is SoA: x[k * n + i].
 #include <algorithm>
 #include <mutex>
 
@@ -41,6 +40,22 @@ __global__ void k_soa_to_aos(const double* __restrict__ soa, double* __restrict_
     }
 }
 
+// one saved frame: positions and velocities to the caller's layout
+__global__ void k_save_frame(const double* __restrict__ x, const double* __restrict__ v,
+                             double* __restrict__ uf, double* __restrict__ vf, int64_t n) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 3 * n) return;
+    const int64_t i = t / 3, k = t - 3 * i;
+    uf[t] = x[k * n + i];
+    vf[t] = v[k * n + i];
+}
+
+void ref64_save_frame(hipStream_t s, const double* x, const double* v, double* uf, double* vf,
+                      int64_t n) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_save_frame, dim3(nbx_blocks(3 * n, 256)), dim3(256), 0, s, x, v, uf, vf, n);
+}
+
 void ref64_fill(hipStream_t s, double* p, int64_t count, double value) {
     if (count <= 0) return;
     hipLaunchKernelGGL(k_fill, dim3(nbx_blocks(count, 256)), dim3(256), 0, s, p, count, value);
@@ -55,134 +70,275 @@ void ref64_soa_to_aos(hipStream_t s, const double* soa, double* aos, int64_t n) 
 }
 
 // ---------------------------------------------------------------------------
-// Lennard-Jones: src/basic_potentials.jl:240-272
+// Pair terms in the reference's order: Lennard-Jones (src/basic_potentials.jl:240-272),
+// truncated Coulomb (:274-304) and reaction field, gravity (:306-331)
 // ---------------------------------------------------------------------------
 
-// Wavefront per target.  The one-thread-per-target loop leaves the chip idle at small n
-// (n = 864 is 14 wavefronts on 1,024 SIMDs), and its cost is the per-pair work: the wrap
-// loops and two FP64 divides.  Here the 64 lanes of a wavefront evaluate the pair terms
-// factor * r_ij of 64 consecutive sources j at once, and the x, y, z sums then take those
-// terms one j after another (each term read from its lane with v_readlane, the adds in
-// ascending j), so every sum sees the reference's terms in the reference's order: the
-// result is bit for bit the one-thread loop's.  A skipped pair contributes +0.0, which
-// leaves a sum unchanged (the sums start at +0.0 and never become -0.0 under
-// round-to-nearest).
+// Wavefront per target.  Its 64 lanes evaluate the pair terms factor * r_ij of up to 64
+// sources at once; the terms of the pairs in range go to LDS in ascending j, and lanes 0..2
+// add them to the x, y, z sums one after another, so every sum sees the reference's terms in
+// the reference's order: the result is bit for bit a loop over j.  A pair out of range is
+// left out: its term would be +0.0, which leaves a sum unchanged (the sums start at +0.0 and
+// never become -0.0 under round-to-nearest).
+//
+// FILTER (cubic box, finite cutoff): sources first pass an FP32 distance test on box
+// fractions, widened by 2e-6 of the box (the fractions are within 1e-7), and only the
+// survivors are gathered, 64 at a time, for the FP64 evaluation.  With 55 of 4,000 sources in
+// range the FP64 work per target is one or two passes instead of 63, and the ordered adds
+// are 55 instead of 4,032.  us per evaluation, against adding all 64 lanes' terms of every
+// chunk through v_readlane: n = 864 36.6 -> 7.9 (the fused step included), n = 4,000
+// 341 -> 22; water's Coulomb and Lennard-Jones terms (1,029 atoms, cutoff 0.45 L) 71 -> 13.6.
+// A few targets per SIMD make it a latency chain: one wavefront's fractions, gathers, pair
+// terms and about 13 cycles per ordered add.
 #define REF_WAVES 4   // targets (wavefronts) per block
+enum { REF_LJ = 0, REF_COULOMB = 1, REF_RF = 2, REF_GRAV = 3 };
 
-__device__ __forceinline__ double ref_lane(double v, int q) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), q);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), q);
-    return __hiloint2double(hi, lo);
-}
+struct ref_law {
+    double s2, R2;     // sigma^2, cutoff^2
+    double c;          // Lennard-Jones eps, Coulomb k, gravity G
+    double krf2;       // 2 k_rf
+    float lim;         // FILTER: squared cutoff in box fractions, widened
+    int jstride, water;
+    int64_t nj;
+};
 
-// f += t_q for q = 0..cnt-1 (lane q holds t_q), in q order
-__device__ __forceinline__ void ref_add_lanes(double& f1, double& f2, double& f3, double t1,
-                                              double t2, double t3, int cnt) {
-    if (cnt == 64) {
-#pragma unroll
-        for (int q = 0; q < 64; ++q) {
-            f1 += ref_lane(t1, q);
-            f2 += ref_lane(t2, q);
-            f3 += ref_lane(t3, q);
-        }
-    } else {
-        for (int q = 0; q < cnt; ++q) {
-            f1 += ref_lane(t1, q);
-            f2 += ref_lane(t2, q);
-            f3 += ref_lane(t3, q);
-        }
-    }
-}
-
-__global__ void __launch_bounds__(64 * REF_WAVES)
-k_ref_lj(const double* __restrict__ x, double* __restrict__ dv, const double* __restrict__ ms,
-         int64_t n, int64_t ib, int64_t cnt, int istride, int jstride, int64_t nj, double s2,
-         double R2, double eps, nbx_bcv bc) {
-    const int lane = threadIdx.x & 63;
-    const int64_t t = (int64_t)blockIdx.x * REF_WAVES + (threadIdx.x >> 6);
-    if (t >= cnt) return;   // the whole wavefront
-    const int64_t i = ib + t * istride;
-    const double xi = x[i], yi = x[n + i], zi = x[2 * n + i];
-    double f1 = 0.0, f2 = 0.0, f3 = 0.0;
-    for (int64_t base = 0; base < nj; base += 64) {
-        const int64_t jj = base + lane;
-        const int64_t j = jj * jstride;
-        double t1 = 0.0, t2 = 0.0, t3 = 0.0;
-        if (jj < nj && j != i) {
-            double rx, ry, rz, rij_2;
-            nbx_displacement(xi, yi, zi, x[j], x[n + j], x[2 * n + j], bc, rx, ry, rz, rij_2);
-            if (rij_2 < R2) {
-                double qq = s2 / rij_2;
-                double s6 = qq * qq * qq;
-                double s12 = s6 * s6;
-                double factor = (2.0 * s12 - s6) / rij_2;
-                t1 = factor * rx;
-                t2 = factor * ry;
-                t3 = factor * rz;
-            }
-        }
-        ref_add_lanes(f1, f2, f3, t1, t2, t3, (int)((nj - base) < 64 ? (nj - base) : 64));
-    }
-    if (lane == 0) {
-        double coeff = 24.0 * eps / ms[i];
-        dv[i] += coeff * f1;
-        dv[n + i] += coeff * f2;
-        dv[2 * n + i] += coeff * f3;
-    }
-}
-
-void ref64_lj(hipStream_t s, const double* x, double* dv, const double* ms, int64_t n,
-              int64_t ib, int64_t ie, int istride, int jstride, int64_t nj, double eps,
-              double sigma, double R, const nbx_bcv& bc) {
-    if (ie <= ib) return;
-    const int64_t cnt = (ie - ib + istride - 1) / istride;
-    hipLaunchKernelGGL(k_ref_lj, dim3(nbx_blocks(cnt, REF_WAVES)), dim3(64 * REF_WAVES), 0, s, x,
-                       dv, ms, n, ib, cnt, istride, jstride, nj, sigma * sigma, R * R, eps, bc);
-}
-
-// ---------------------------------------------------------------------------
-// Electrostatics (truncated Coulomb, src/basic_potentials.jl:274-304) and reaction field
-// ---------------------------------------------------------------------------
+struct ref_atoms {
+    const double* x;       // SoA
+    const float4* frac;    // box fractions (FILTER)
+    const double* ms;
+    const double* qs;
+    int64_t n;
+};
 
 __device__ __forceinline__ bool ref_excluded(int64_t i, int64_t j, int water) {
     return water ? (i / 3) == (j / 3) : i == j;   // src/nbody_to_ode.jl:326, :346-348
 }
 
-template <bool RF>
-__global__ void __launch_bounds__(64 * REF_WAVES)
-k_ref_coulomb(const double* __restrict__ x, double* __restrict__ dv,
-              const double* __restrict__ ms, const double* __restrict__ qs, int64_t n,
-              int64_t ib, int64_t ie, int water, double k, double R2, double krf2,
-              nbx_bcv bc) {
+// box fraction of a coordinate for the filter; NaN (passes every test) where x / L is too
+// large for the margin to hold
+__device__ __forceinline__ float ref_frac(double x, double invL) {
+    const double t = x * invL;
+    return fabs(t) < 1048576.0 ? (float)(t - floor(t)) : __builtin_nanf("");
+}
+
+// factor * r_ij of one pair; false when it is out of range
+template <int KIND>
+__device__ __forceinline__ bool ref_pair_term(const ref_law& law, double xi, double yi, double zi,
+                                              double xj, double yj, double zj, double wj,
+                                              const nbx_bcv& bc, double* t) {
+    if (KIND == REF_GRAV) {
+        const double rx = xi - xj, ry = yi - yj, rz = zi - zj;
+        const double ss = rx * rx + ry * ry;
+        const double nr = sqrt(ss + rz * rz);
+        const double factor = -law.c * wj / (nr * nr * nr);
+        t[0] = factor * rx;
+        t[1] = factor * ry;
+        t[2] = factor * rz;
+        return true;
+    }
+    double rx, ry, rz, r2;
+    nbx_displacement(xi, yi, zi, xj, yj, zj, bc, rx, ry, rz, r2);
+    if (!(r2 < law.R2)) return false;
+    double factor;
+    if (KIND == REF_LJ) {
+        const double qq = law.s2 / r2;
+        const double s6 = qq * qq * qq;
+        const double s12 = s6 * s6;
+        factor = (2.0 * s12 - s6) / r2;
+    } else {
+        const double r = sqrt(r2);
+        if (KIND == REF_RF) factor = wj * (1.0 / (r * r2) - law.krf2);
+        else factor = wj / (r * r2);
+    }
+    t[0] = factor * rx;
+    t[1] = factor * ry;
+    t[2] = factor * rz;
+    return true;
+}
+
+// the whole wavefront's sum over the sources of target i: component min(lane, 2) in each lane
+template <int KIND, bool FILTER>
+__device__ __forceinline__ double ref_wave_sum(const ref_atoms& A, const ref_law& law,
+                                               const nbx_bcv& bc, int64_t i, int* cand,
+                                               double* term) {
     const int lane = threadIdx.x & 63;
-    const int64_t i = ib + (int64_t)blockIdx.x * REF_WAVES + (threadIdx.x >> 6);
-    if (i >= ie) return;   // the whole wavefront
-    const double xi = x[i], yi = x[n + i], zi = x[2 * n + i];
-    double f1 = 0.0, f2 = 0.0, f3 = 0.0;
-    for (int64_t base = 0; base < n; base += 64) {
-        const int64_t jj = base + lane;
-        double t1 = 0.0, t2 = 0.0, t3 = 0.0;
-        if (jj < n && !ref_excluded(i, jj, water)) {
-            double rx, ry, rz, r2;
-            nbx_displacement(xi, yi, zi, x[jj], x[n + jj], x[2 * n + jj], bc, rx, ry, rz, r2);
-            if (r2 < R2) {
-                const double qj = qs[jj];
-                double r = sqrt(r2);
-                double factor;
-                if (RF) factor = qj * (1.0 / (r * r2) - krf2);
-                else factor = qj / (r * r2);
-                t1 = factor * rx;
-                t2 = factor * ry;
-                t3 = factor * rz;
+    const int c = lane < 2 ? lane : 2;
+    const int64_t n = A.n;
+    const double xi = A.x[i], yi = A.x[n + i], zi = A.x[2 * n + i];
+    const double* const w = KIND == REF_GRAV ? A.ms : (KIND == REF_LJ ? nullptr : A.qs);
+    double f = 0.0;
+    // the terms of up to 64 sources, one per lane (in ascending j), added in order
+    const auto add = [&](bool ok, double xj, double yj, double zj, double wj) {
+        double t[3] = {0.0, 0.0, 0.0};
+        const bool hit = ok && ref_pair_term<KIND>(law, xi, yi, zi, xj, yj, zj, wj, bc, t);
+        const unsigned long long mask = __ballot(hit);
+        if (mask == 0ull) return;
+        const int at = (int)__builtin_amdgcn_mbcnt_hi(
+            (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+        if (hit) {
+            term[3 * at] = t[0];
+            term[3 * at + 1] = t[1];
+            term[3 * at + 2] = t[2];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int cnt = __popcll(mask);
+        int q = 0;
+        for (; q + 16 <= cnt; q += 16) {
+            double u[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) u[k] = term[3 * (q + k) + c];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) f += u[k];
+        }
+        for (; q + 4 <= cnt; q += 4) {
+            double u[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) u[k] = term[3 * (q + k) + c];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) f += u[k];
+        }
+        for (; q < cnt; ++q) f += term[3 * q + c];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    if constexpr (FILTER) {
+        const float4 fi = A.frac[i];
+        int pending = 0;   // uniform
+        const auto eval = [&](int cnt) {
+            const bool ok = lane < cnt;
+            const int64_t j = ok ? cand[lane] : i;
+            add(ok, A.x[j], A.x[n + j], A.x[2 * n + j], w != nullptr ? w[j] : 0.0);
+        };
+        constexpr int U = 4;   // chunks of 64 whose fractions are in flight together
+        for (int64_t base = 0; base < law.nj; base += 64 * U) {
+            float4 fj[U];
+#pragma unroll
+            for (int q = 0; q < U; ++q) {
+                const int64_t jj = base + 64 * q + lane;
+                fj[q] = A.frac[jj < law.nj ? jj * law.jstride : i];
+            }
+#pragma unroll
+            for (int q = 0; q < U; ++q) {
+                const int64_t jj = base + 64 * q + lane, j = jj * law.jstride;
+                float dx = fi.x - fj[q].x, dy = fi.y - fj[q].y, dz = fi.z - fj[q].z;
+                dx -= rintf(dx);
+                dy -= rintf(dy);
+                dz -= rintf(dz);
+                const bool near = jj < law.nj && !ref_excluded(i, j, law.water) &&
+                                  !(dx * dx + dy * dy + dz * dz >= law.lim);
+                const unsigned long long mask = __ballot(near);
+                if (mask == 0ull) continue;
+                const int at = pending + (int)__builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+                if (near) cand[at] = (int)j;
+                pending += __popcll(mask);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (pending >= 64) {
+                    eval(64);
+                    pending -= 64;
+                    const int rest = cand[64 + lane];   // moved down (past the count: unused)
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    cand[lane] = rest;
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                }
             }
         }
-        ref_add_lanes(f1, f2, f3, t1, t2, t3, (int)((n - base) < 64 ? (n - base) : 64));
+        if (pending > 0) eval(pending);
+    } else {
+        // every source: the next chunk's atoms are loaded while this one is added
+        const auto load = [&](int64_t jj, double* p) {
+            const int64_t j = jj < law.nj ? jj * law.jstride : i;
+            p[0] = A.x[j]; p[1] = A.x[n + j]; p[2] = A.x[2 * n + j];
+            p[3] = w != nullptr ? w[j] : 0.0;
+        };
+        double nx[4];
+        load(lane, nx);
+        for (int64_t base = 0; base < law.nj; base += 64) {
+            const double px = nx[0], py = nx[1], pz = nx[2], pw = nx[3];
+            if (base + 64 < law.nj) load(base + 64 + lane, nx);
+            const int64_t jj = base + lane;
+            add(jj < law.nj && !ref_excluded(i, jj * law.jstride, law.water), px, py, pz, pw);
+        }
     }
-    if (lane == 0) {
-        double coeff = k * qs[i] / ms[i];
-        dv[i] += coeff * f1;
-        dv[n + i] += coeff * f2;
-        dv[2 * n + i] += coeff * f3;
+    return f;
+}
+
+// the closure's contribution to atom i from the sum: dv += coeff * f
+template <int KIND>
+__device__ __forceinline__ double ref_contribution(const ref_atoms& A, const ref_law& law,
+                                                   int64_t i, double f) {
+    if (KIND == REF_LJ) return 24.0 * law.c / A.ms[i] * f;
+    if (KIND == REF_GRAV) return f;
+    return law.c * A.qs[i] / A.ms[i] * f;
+}
+
+// End of step `step` for component c of atom i, with the acceleration a of its potentials:
+// thermostat force, kick, Langevin B and Andersen; then (drift) the start of step + 1:
+// Langevin A, positions into the other buffer, half-kicked velocity, box fraction.  The
+// expressions of k_ref_berendsen, k_ref_kick, k_ref_langevin_half, k_ref_andersen and
+// k_ref_drift; counter: the atom whose number decides an Andersen collision (the molecule's
+// O for water), m_andersen its mass.
+__device__ __forceinline__ void ref_end_step(const ref64_step& st, int64_t n, int64_t i, int c,
+                                             double a, double mi, int64_t counter,
+                                             double m_andersen) {
+    const int64_t k = c * n + i;
+    const double h = st.vh[k];
+    if (st.therm == NBX_THERM_BERENDSEN) {
+        const double T = st.d_T[0];
+        if (1.0 / T == __builtin_inf()) a += st.gamma * h;
+        else {
+            const double cb = st.gamma * (st.T / T - 1.0);
+            a += cb * h;
+        }
+    }
+    st.a[k] = a;
+    double v = h + st.dt * (0.5 * a);
+    double g[3], sig = 0.0;
+    if (st.therm == NBX_THERM_LANGEVIN) {
+        sig = st.c2 * sqrt(st.kb * st.T / mi);
+        nbx_rng_normals3(st.seed, i, st.step, NBX_RNG_LANGEVIN_B, g);
+        v = st.c1 * v + sig * (c == 0 ? g[0] : (c == 1 ? g[1] : g[2]));
+    } else if (st.therm == NBX_THERM_ANDERSEN &&
+               nbx_rng_uniform(st.seed, counter, st.step, NBX_RNG_ANDERSEN) < st.prob) {
+        const double vdev = sqrt(st.kb * st.T / m_andersen);
+        nbx_rng_normals3(st.seed, i, st.step, NBX_RNG_ANDERSEN, g);
+        v = vdev * (c == 0 ? g[0] : (c == 1 ? g[1] : g[2]));
+    }
+    st.v[k] = v;
+    if (!st.drift) return;
+    if (st.therm == NBX_THERM_LANGEVIN) {
+        nbx_rng_normals3(st.seed, i, st.step + 1, NBX_RNG_LANGEVIN_A, g);
+        v = st.c1 * v + sig * (c == 0 ? g[0] : (c == 1 ? g[1] : g[2]));
+    }
+    const double half = 0.5, dtsq = st.dt * st.dt;
+    const double px = st.x_in[k] + st.dt * v + dtsq * (half * a);
+    st.x_out[k] = px;
+    st.vh[k] = v + st.dt * (half * a);
+    if (st.frac_out != nullptr)
+        reinterpret_cast<float*>(st.frac_out + i)[c] = ref_frac(px, st.invL);
+}
+
+// targets i = ib, ib + istride, ...: dv += contribution, or (STEP) the acceleration a_in
+// (nullptr: 0) + contribution and the end of the step
+template <int KIND, bool FILTER, bool STEP>
+__global__ void __launch_bounds__(64 * REF_WAVES)
+k_ref_pairs(ref_atoms A, ref_law law, nbx_bcv bc, int64_t ib, int64_t cnt, int istride,
+            double* __restrict__ dv, ref64_step st) {
+    __shared__ int cand[REF_WAVES][128];
+    __shared__ double term[REF_WAVES][192];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int64_t t = (int64_t)blockIdx.x * REF_WAVES + wave;
+    if (t >= cnt) return;   // the whole wavefront
+    const int64_t i = ib + t * istride;
+    const double f = ref_wave_sum<KIND, FILTER>(A, law, bc, i, cand[wave], term[wave]);
+    if (lane >= 3) return;
+    const double add = ref_contribution<KIND>(A, law, i, f);
+    const int64_t k = lane * A.n + i;
+    if constexpr (STEP) {
+        ref_end_step(st, A.n, i, lane, (st.a_in != nullptr ? st.a_in[k] : 0.0) + add, A.ms[i], i,
+                     A.ms[0]);
+    } else {
+        dv[k] += add;
     }
 }
 
@@ -191,26 +347,93 @@ static double rf_krf(double R, double eps_rf) {
     return (eps_rf - 1.0) / ((2.0 * eps_rf + 1.0) * (R * R * R));
 }
 
-void ref64_elec(hipStream_t s, const double* x, double* dv, const double* ms,
-                const double* qs, int64_t n, int64_t ib, int64_t ie, int water, double k,
-                double R, const nbx_bcv& bc) {
-    if (ie <= ib) return;
-    hipLaunchKernelGGL(k_ref_coulomb<false>, dim3(nbx_blocks(ie - ib, REF_WAVES)),
-                       dim3(64 * REF_WAVES), 0, s, x, dv, ms, qs, n, ib, ie, water, k, R * R,
-                       0.0, bc);
+static ref_law make_law(const ref64_term& t, const nbx_bcv& bc) {
+    ref_law law{};
+    law.jstride = t.jstride;
+    law.nj = t.nj;
+    law.water = t.water;
+    if (t.kind == NBX_TERM_LJ) {
+        law.c = t.p[0];
+        law.s2 = t.p[1] * t.p[1];
+        law.R2 = t.p[2] * t.p[2];
+    } else if (t.kind == NBX_TERM_GRAV) {
+        law.c = t.p[0];
+    } else {
+        law.c = t.p[0];
+        law.R2 = t.p[1] * t.p[1];
+        if (t.kind == NBX_TERM_RF) law.krf2 = 2.0 * rf_krf(t.p[1], t.p[2]);
+    }
+    if (t.filter) {
+        const double R = (t.kind == NBX_TERM_LJ ? t.p[2] : t.p[1]) / bc.b[0] + 2e-6;
+        law.lim = (float)(R * R * (1.0 + 1e-6));
+    }
+    return law;
 }
 
-void ref64_rf(hipStream_t s, const double* x, double* dv, const double* ms, const double* qs,
-              int64_t n, int64_t ib, int64_t ie, int water, double k, double R,
-              double eps_rf, const nbx_bcv& bc) {
+bool ref64_filters(const ref64_term& t, const nbx_bcv& bc) {
+    if (bc.kind != NBX_BC_CUBIC || t.kind == NBX_TERM_GRAV) return false;
+    const double R = t.kind == NBX_TERM_LJ ? t.p[2] : t.p[1];
+    // from half the box on nearly every source passes: the test would only add work
+    return R < 0.5 * bc.b[0];
+}
+
+template <int KIND, bool STEP>
+static void launch_pairs(hipStream_t s, const ref64_term& t, const ref_atoms& A,
+                         const nbx_bcv& bc, int64_t ib, int64_t ie, double* dv,
+                         const ref64_step& st) {
+    const ref_law law = make_law(t, bc);
+    const int64_t cnt = (ie - ib + t.istride - 1) / t.istride;
+    const dim3 grid(nbx_blocks(cnt, REF_WAVES)), block(64 * REF_WAVES);
+    if constexpr (KIND != REF_GRAV) {
+        if (t.filter) {
+            hipLaunchKernelGGL((k_ref_pairs<KIND, true, STEP>), grid, block, 0, s, A, law, bc, ib,
+                               cnt, t.istride, dv, st);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_ref_pairs<KIND, false, STEP>), grid, block, 0, s, A, law, bc, ib, cnt,
+                       t.istride, dv, st);
+}
+
+void ref64_pairs(hipStream_t s, const ref64_term& t, const double* x, const float4* frac,
+                 const double* ms, const double* qs, int64_t n, int64_t ib, int64_t ie,
+                 const nbx_bcv& bc, double* dv, const ref64_step* step) {
     if (ie <= ib) return;
-    hipLaunchKernelGGL(k_ref_coulomb<true>, dim3(nbx_blocks(ie - ib, REF_WAVES)),
-                       dim3(64 * REF_WAVES), 0, s, x, dv, ms, qs, n, ib, ie, water, k, R * R,
-                       2.0 * rf_krf(R, eps_rf), bc);
+    const ref_atoms A{x, frac, ms, qs, n};
+    const ref64_step st = step ? *step : ref64_step{};
+#define REF_GO(KIND)                                                            \
+    do {                                                                        \
+        if (step) launch_pairs<KIND, true>(s, t, A, bc, ib, ie, dv, st);        \
+        else launch_pairs<KIND, false>(s, t, A, bc, ib, ie, dv, st);            \
+    } while (0)
+    switch (t.kind) {
+    case NBX_TERM_LJ: REF_GO(REF_LJ); break;
+    case NBX_TERM_ELEC: REF_GO(REF_COULOMB); break;
+    case NBX_TERM_RF: REF_GO(REF_RF); break;
+    case NBX_TERM_GRAV: REF_GO(REF_GRAV); break;
+    default: break;
+    }
+#undef REF_GO
+}
+
+__global__ void k_ref_fractions(const double* __restrict__ x, int64_t n, double invL,
+                                float4* __restrict__ frac) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    frac[i] = make_float4(ref_frac(x[i], invL), ref_frac(x[n + i], invL),
+                          ref_frac(x[2 * n + i], invL), 0.0f);
+}
+
+void ref64_fractions(hipStream_t s, const double* x, int64_t n, double L, float4* frac) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_ref_fractions, dim3(nbx_blocks(n, 256)), dim3(256), 0, s, x, n, 1.0 / L,
+                       frac);
 }
 
 // ---------------------------------------------------------------------------
-// Gravity: src/basic_potentials.jl:306-331 (no boundary conditions, no cutoff)
+// Gravity of many bodies: src/basic_potentials.jl:306-331 (no boundary conditions, no
+// cutoff).  One thread per target walks the sources: a third of the instructions of a
+// wavefront per target, once there are targets enough to fill the chip (NBX_REF_GRAV_WAVES).
 // ---------------------------------------------------------------------------
 
 __global__ void __launch_bounds__(REF_TILE)
@@ -330,15 +553,13 @@ void ref64_mag(hipStream_t s, const double* x, double* dv, const double* ms, con
 // SPC/Fw bonded terms: src/basic_potentials.jl:367-433
 // ---------------------------------------------------------------------------
 
-__global__ void k_ref_bond(const double* __restrict__ x, double* __restrict__ dv,
-                           const double* __restrict__ ms, int64_t n, int64_t ib, int64_t ie,
-                           double rOH, double kbond) {
-    const int64_t i = ib + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ie) return;
+// bond force / mass-free sum of atom i (src/nbody_to_ode.jl:274-284)
+__device__ __forceinline__ void ref_bond_force(const double* __restrict__ x, int64_t n, int64_t i,
+                                               double rOH, double kbond, double* f) {
     const int64_t o = 3 * (i / 3);
     int64_t nb[2];
     int nn;
-    if (i == o) { nb[0] = o + 1; nb[1] = o + 2; nn = 2; }   // src/nbody_to_ode.jl:274-284
+    if (i == o) { nb[0] = o + 1; nb[1] = o + 2; nn = 2; }
     else { nb[0] = o; nb[1] = o; nn = 1; }
     double f1 = 0.0, f2 = 0.0, f3 = 0.0;
     const double xi = x[i], yi = x[n + i], zi = x[2 * n + i];
@@ -352,10 +573,20 @@ __global__ void k_ref_bond(const double* __restrict__ x, double* __restrict__ dv
         f2 += factor * ry;
         f3 += factor * rz;
     }
+    f[0] = f1; f[1] = f2; f[2] = f3;
+}
+
+__global__ void k_ref_bond(const double* __restrict__ x, double* __restrict__ dv,
+                           const double* __restrict__ ms, int64_t n, int64_t ib, int64_t ie,
+                           double rOH, double kbond) {
+    const int64_t i = ib + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= ie) return;
+    double f[3];
+    ref_bond_force(x, n, i, rOH, kbond, f);
     double coeff = 1.0 / ms[i];
-    dv[i] += coeff * f1;
-    dv[n + i] += coeff * f2;
-    dv[2 * n + i] += coeff * f3;
+    dv[i] += coeff * f[0];
+    dv[n + i] += coeff * f[1];
+    dv[2 * n + i] += coeff * f[2];
 }
 
 void ref64_bond(hipStream_t s, const double* x, double* dv, const double* ms, int64_t n,
@@ -372,12 +603,10 @@ __device__ __forceinline__ void ref_cross(double a0, double a1, double a2, doubl
     c2 = a0 * b1 - a1 * b0;
 }
 
-// valence_angle_potential_acceleration!(dv, rs, a=H1, b=O, c=H2, ...) per molecule
-__global__ void k_ref_angle(const double* __restrict__ x, double* __restrict__ dv,
-                            const double* __restrict__ ms, int64_t n, int64_t mb, int64_t me,
-                            double aHOH, double ka) {
-    const int64_t m = mb + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= me) return;
+// valence_angle_potential_acceleration!(dv, rs, a=H1, b=O, c=H2, ...) of molecule m: the
+// forces on H1 (fa) and H2 (fc); O takes -(fa + fc)
+__device__ __forceinline__ void ref_angle_force(const double* __restrict__ x, int64_t n, int64_t m,
+                                                double aHOH, double ka, double* fa, double* fc) {
     const int64_t a = 3 * m + 1, b = 3 * m, c = 3 * m + 2;
     double ra[3] = {x[a], x[n + a], x[2 * n + a]};
     double rb[3] = {x[b], x[n + b], x[2 * n + b]};
@@ -405,13 +634,97 @@ __global__ void k_ref_angle(const double* __restrict__ x, double* __restrict__ d
     double force = -ka * (ang - aHOH);
     for (int k = 0; k < 3; ++k) {
         double pa = ia * ta[k], pc = ic * tc[k];
-        double fa = pa * force / nba;
-        double fc = pc * force / nbc;
-        double fb = -(fa + fc);
-        dv[k * n + a] += fa / ms[a];
-        dv[k * n + b] += fb / ms[b];
-        dv[k * n + c] += fc / ms[c];
+        fa[k] = pa * force / nba;
+        fc[k] = pc * force / nbc;
     }
+}
+
+__global__ void k_ref_angle(const double* __restrict__ x, double* __restrict__ dv,
+                            const double* __restrict__ ms, int64_t n, int64_t mb, int64_t me,
+                            double aHOH, double ka) {
+    const int64_t m = mb + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= me) return;
+    const int64_t a = 3 * m + 1, b = 3 * m, c = 3 * m + 2;
+    double fa[3], fc[3];
+    ref_angle_force(x, n, m, aHOH, ka, fa, fc);
+    for (int k = 0; k < 3; ++k) {
+        double fb = -(fa[k] + fc[k]);
+        dv[k * n + a] += fa[k] / ms[a];
+        dv[k * n + b] += fb / ms[b];
+        dv[k * n + c] += fc[k] / ms[c];
+    }
+}
+
+// Water, one step's right-hand side and end in two launches: the electrostatic sums of all
+// atoms into elec and the Lennard-Jones sums of the O atoms into lj (one launch, a wavefront
+// per sum), then per atom the reference's closure order -- electrostatic, bond, LJ (O), then
+// the molecule's angle -- and the end of the step.
+template <int KIND, bool FILTER>
+__global__ void __launch_bounds__(64 * REF_WAVES)
+k_ref_water_pairs(ref_atoms A, ref_law el, ref_law lj, nbx_bcv bc, double* __restrict__ elec,
+                  double* __restrict__ ljv) {
+    __shared__ int cand[REF_WAVES][128];
+    __shared__ double term[REF_WAVES][192];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int64_t t = (int64_t)blockIdx.x * REF_WAVES + wave;
+    const int64_t n = A.n;
+    if (t < n) {
+        const double f = ref_wave_sum<KIND, FILTER>(A, el, bc, t, cand[wave], term[wave]);
+        if (lane < 3) elec[lane * n + t] = ref_contribution<KIND>(A, el, t, f);
+    } else if (t < n + n / 3) {
+        const int64_t i = 3 * (t - n);
+        const double f = ref_wave_sum<REF_LJ, FILTER>(A, lj, bc, i, cand[wave], term[wave]);
+        if (lane < 3) ljv[lane * n + i] = ref_contribution<REF_LJ>(A, lj, i, f);
+    }
+}
+
+// one thread per component of an atom (thread t: atom t / 3, component t % 3)
+__global__ void __launch_bounds__(192)
+k_ref_water_step(const double* __restrict__ ms, int64_t n, const double* __restrict__ elec,
+                 const double* __restrict__ ljv, double rOH, double kbond, double aHOH, double ka,
+                 ref64_step st) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = t / 3;
+    if (i >= n) return;
+    const int c = (int)(t - 3 * i);
+    const int64_t m = i / 3, o = 3 * m;
+    const double* const x = st.x_in;
+    double fb[3], fa[3], fc[3];
+    ref_bond_force(x, n, i, rOH, kbond, fb);
+    ref_angle_force(x, n, m, aHOH, ka, fa, fc);
+    const auto pick = [c](const double* f) { return c == 0 ? f[0] : (c == 1 ? f[1] : f[2]); };
+    const double mi = ms[i];
+    double a = 0.0 + elec[c * n + i];
+    const double coeff = 1.0 / mi;
+    a += coeff * pick(fb);
+    if (i == o) a += ljv[c * n + i];
+    const double f1 = pick(fa), f2 = pick(fc);
+    if (i == o) a += -(f1 + f2) / mi;
+    else if (i == o + 1) a += f1 / mi;
+    else a += f2 / mi;
+    ref_end_step(st, n, i, c, a, mi, o, mi);
+}
+
+void ref64_water_step(hipStream_t s, const ref64_term& el, const ref64_term& lj, const float4* frac,
+                      const double* ms, const double* qs, int64_t n, const nbx_bcv& bc,
+                      double* elec, double* ljv, double rOH, double kbond, double aHOH, double ka,
+                      const ref64_step& st) {
+    if (n <= 0) return;
+    const ref_atoms A{st.x_in, frac, ms, qs, n};
+    const ref_law le = make_law(el, bc), ll = make_law(lj, bc);
+    const dim3 grid(nbx_blocks(n + n / 3, REF_WAVES)), block(64 * REF_WAVES);
+    const bool rf = el.kind == NBX_TERM_RF;
+    // both laws filter, or neither (el.filter == lj.filter)
+    if (el.filter) {
+        if (rf) hipLaunchKernelGGL((k_ref_water_pairs<REF_RF, true>), grid, block, 0, s, A, le, ll, bc, elec, ljv);
+        else hipLaunchKernelGGL((k_ref_water_pairs<REF_COULOMB, true>), grid, block, 0, s, A, le, ll, bc, elec, ljv);
+    } else {
+        if (rf) hipLaunchKernelGGL((k_ref_water_pairs<REF_RF, false>), grid, block, 0, s, A, le, ll, bc, elec, ljv);
+        else hipLaunchKernelGGL((k_ref_water_pairs<REF_COULOMB, false>), grid, block, 0, s, A, le, ll, bc, elec, ljv);
+    }
+    hipLaunchKernelGGL(k_ref_water_step, dim3(nbx_blocks(3 * n, 192)), dim3(192), 0, s, ms, n, elec,
+                       ljv, rOH, kbond, aHOH, ka, st);
 }
 
 void ref64_angle(hipStream_t s, const double* x, double* dv, const double* ms, int64_t n,
@@ -531,14 +844,20 @@ void ref64_berendsen(hipStream_t s, double* dv, const double* v, int64_t n, cons
 // Velocity Verlet and stochastic thermostats
 // ---------------------------------------------------------------------------
 
-__global__ void k_ref_drift(double* __restrict__ x, const double* __restrict__ v,
-                            const double* __restrict__ a, double* __restrict__ vh, int64_t n3,
-                            double dt) {
+// x_out may be x; frac: box fractions of the new positions (nullptr: none)
+__global__ void k_ref_drift(const double* x, double* x_out, const double* __restrict__ v,
+                            const double* __restrict__ a, double* __restrict__ vh, int64_t n,
+                            double dt, float4* frac, double invL) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n3) return;
+    if (t >= 3 * n) return;
     const double half = 0.5, dtsq = dt * dt;
-    x[t] = x[t] + dt * v[t] + dtsq * (half * a[t]);
+    const double px = x[t] + dt * v[t] + dtsq * (half * a[t]);
+    x_out[t] = px;
     vh[t] = v[t] + dt * (half * a[t]);
+    if (frac != nullptr) {
+        const int64_t c = t / n;
+        reinterpret_cast<float*>(frac + (t - c * n))[c] = ref_frac(px, invL);
+    }
 }
 
 __global__ void k_ref_kick(double* __restrict__ v, const double* __restrict__ vh,
@@ -548,11 +867,11 @@ __global__ void k_ref_kick(double* __restrict__ v, const double* __restrict__ vh
     v[t] = vh[t] + dt * (0.5 * a[t]);
 }
 
-void ref64_drift(hipStream_t s, double* x, const double* v, const double* a, double* vh,
-                 int64_t n, double dt) {
+void ref64_drift(hipStream_t s, const double* x, double* x_out, const double* v, const double* a,
+                 double* vh, int64_t n, double dt, float4* frac, double L) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_ref_drift, dim3(nbx_blocks(3 * n, 256)), dim3(256), 0, s, x, v, a, vh,
-                       3 * n, dt);
+    hipLaunchKernelGGL(k_ref_drift, dim3(nbx_blocks(3 * n, 256)), dim3(256), 0, s, x, x_out, v, a,
+                       vh, n, dt, frac, 1.0 / L);
 }
 
 void ref64_kick(hipStream_t s, double* v, const double* vh, const double* a, int64_t n,
