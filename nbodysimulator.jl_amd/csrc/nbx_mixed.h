@@ -298,6 +298,61 @@ __device__ __forceinline__ double mx_drift_atom(int64_t i, int64_t n, const doub
     return mi * (hx * hx + hy * hy + hz * hz);
 }
 
+// One component of an atom at the end of a step (mx_load_component, mx_end_component): the
+// kernels whose atoms have several lanes give three neighbouring lanes the x, y and z of an
+// atom, 16 atoms to a wavefront, so that loads and stores are shared by all of them and the
+// FP64 work of the three components runs side by side.
+#define MX_GROUP 16
+struct mx_component {
+    double m, q;          // mass, charge (0 without charges)
+    double vh, x, xr;     // as mx_atom
+};
+
+__device__ __forceinline__ void mx_load_component(int64_t i, int c, int64_t n, const mx_io& io,
+                                                  mx_component& A) {
+    const int64_t k = (int64_t)c * n + i;
+    A.m = io.ms[i];
+    A.q = io.qs != nullptr ? io.qs[i] : 0.0;
+    A.vh = io.vh[k];
+    if (io.do_drift) {
+        A.x = io.x_in[k];
+        if (io.xref != nullptr) A.xr = io.xref[k];
+    }
+}
+
+// position of step kp.step + 1: buffers of the list plans, and the skin test (the lane of
+// component 0 collects the three squares from its neighbours)
+__device__ __forceinline__ void mx_store_component(int64_t i, int c, int64_t n, double px,
+                                                   const mx_component& A, const mx_io& io,
+                                                   bool act) {
+    if (act) {
+        io.x_out[(int64_t)c * n + i] = px;
+        if (io.pos_kind == 1) {
+            const double q = c == 0 ? A.q : 0.0;
+            double* const p4 = reinterpret_cast<double*>(io.pos_out) + 4 * i;
+            uint32_t* const p1 = reinterpret_cast<uint32_t*>(mx_posq(io.pos_out, n) + i);
+            p4[c] = mx_wrap(px, io.L);
+            p1[c] = mx_frac32(px, io.invL);
+            if (c == 0) {
+                p4[3] = q;
+                p1[3] = __float_as_uint((float)q);
+            }
+        }
+    }
+    if (io.xref != nullptr) {
+        const double e = act ? px - A.xr : 0.0;
+        const double ee = e * e;
+        const int l = threadIdx.x & 63;
+        const double e1 = __shfl(ee, l + 1, 64), e2 = __shfl(ee, l + 2, 64);
+        const double r2 = ee + e1 + e2;
+        if (act && c == 0) {
+            if (r2 > io.half_skin2) io.req_out[0] = 1;
+            if (r2 > io.guard2) io.flags[1] = 1;
+            if (!io.next_opp && r2 > io.stale2) io.flags[7] = 1;
+        }
+    }
+}
+
 // Thermostat force a += c vh: Berendsen c = gamma (T0/T - 1) (src/thermostats.jl:76-83),
 // Nose-Hoover c = -zeta (src/thermostats.jl:116-122)
 __device__ __forceinline__ bool mx_therm_force(const mx_kick_params& kp) {
@@ -312,6 +367,61 @@ __device__ __forceinline__ double mx_berendsen_from_T(const mx_kick_params& kp, 
 __device__ __forceinline__ double mx_berendsen_coeff(const mx_kick_params& kp) {
     if (kp.therm == NBX_THERM_NOSEHOOVER) return -kp.d_T[NBX_SCAL_ZETA];
     return mx_berendsen_from_T(kp, kp.d_T[0]);
+}
+
+// The end of step kp.step for component c of atom i from its acceleration a (potentials
+// only), and the start of the next one; act: the lane holds a component.  Every lane of the
+// wavefront calls it.  Returns the component's part of m vh^2 of the next step.
+__device__ __forceinline__ double mx_end_component(int64_t i, int c, int64_t n, double a,
+                                                   const mx_component& A, const mx_kick_params& kp,
+                                                   const mx_io& io, bool act) {
+    const int64_t k = (int64_t)c * n + i;
+    if (act && mx_therm_force(kp)) a += mx_berendsen_coeff(kp) * A.vh;
+    if (act) io.a[k] = a;
+    if (!kp.do_kick) return 0.0;
+    const auto pick = [c](const double* g) { return c == 0 ? g[0] : (c == 1 ? g[1] : g[2]); };
+    double v = 0.0, px = 0.0, tval = 0.0;
+    if (act) {
+        double g[3];
+        double sig = 0.0;
+        if (kp.em) {   // Euler-Maruyama: vh already holds v of the step being finished
+            v = A.vh;
+        } else {
+            v = A.vh + kp.dt * (0.5 * a);
+            if (kp.therm == NBX_THERM_LANGEVIN) {
+                sig = kp.c2 * sqrt(kp.kb * kp.T / A.m);
+                nbx_rng_normals3(kp.seed, mx_atom_id(kp, i), kp.step, NBX_RNG_LANGEVIN_B, g);
+                v = kp.c1 * v + sig * pick(g);
+            }
+        }
+        if (kp.therm == NBX_THERM_ANDERSEN &&
+            nbx_rng_uniform(kp.seed, mx_atom_id(kp, i), kp.step, NBX_RNG_ANDERSEN) < kp.prob) {
+            const double vdev = sqrt(kp.kb * kp.T / kp.m0);
+            nbx_rng_normals3(kp.seed, mx_atom_id(kp, i), kp.step, NBX_RNG_ANDERSEN, g);
+            v = vdev * pick(g);
+        }
+        io.v[k] = v;
+        if (io.do_drift) {
+            const double dt = kp.dt;
+            if (kp.em) {
+                px = A.x + dt * v;
+                nbx_rng_normals3(kp.seed, mx_atom_id(kp, i), kp.step + 1, NBX_RNG_EM, g);
+                io.vh[k] = v + dt * (a - kp.em_gamma * v) + kp.em_sigma * (kp.em_sqrt_dt * pick(g));
+            } else {
+                if (kp.therm == NBX_THERM_LANGEVIN) {
+                    nbx_rng_normals3(kp.seed, mx_atom_id(kp, i), kp.step + 1, NBX_RNG_LANGEVIN_A, g);
+                    v = kp.c1 * v + sig * pick(g);
+                }
+                const double dtsq = dt * dt;
+                px = A.x + dt * v + dtsq * (0.5 * a);
+                const double h = v + dt * (0.5 * a);
+                io.vh[k] = h;
+                tval = A.m * (h * h);
+            }
+        }
+    }
+    if (io.do_drift) mx_store_component(i, c, n, px, A, io, act);
+    return tval;
 }
 
 // Epilogue of a step kernel, called by every thread of every block (blockDim.x <= 256):

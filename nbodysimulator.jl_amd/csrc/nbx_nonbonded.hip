@@ -145,33 +145,54 @@ __device__ __forceinline__ double nb_finish(int64_t i, int64_t n, const double* 
 // Verlet-list force kernel: G lanes per atom
 // ---------------------------------------------------------------------------
 
+// End of the step by transposed lanes: the sums of the block's 256 / G atoms meet in LDS, and
+// three neighbouring lanes take the x, y, z of an atom, 16 atoms to a wavefront.  With the
+// first lane of every atom ending its step alone, a wavefront of 8 lanes per atom issued 26
+// loads and stores of 64 bytes and the FP64 tail for 8 active lanes (us per step, Lennard-
+// Jones: n = 32,000 15.9 -> 14.0 at 8 lanes, 18.6 -> 15.0 at 16; n = 864 7.0 -> 6.3 at 32).
+// Water stores three accelerations per atom from its first lane: the molecule kernel ends its
+// step, and the exchange would cost more than it saves (25.5 against 25.8).
 template <int G, bool LJ, int EL, bool WATER, typename IDX>
 __global__ void __launch_bounds__(NB_THREADS)
 k_nb_list(const double4* __restrict__ pos, const IDX* __restrict__ nbr,
           const int* __restrict__ nnb, int n, mx_pair_params pp, mx_kick_params kp, mx_io io) {
-    const int gid = mx_xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    constexpr int ATOMS = NB_THREADS / G;                    // atoms per block
+    constexpr int GROUPS = (ATOMS + MX_GROUP - 1) / MX_GROUP;
+    constexpr int ROUNDS = (GROUPS + 3) / 4;                 // groups per wavefront
+    constexpr int SUMS = (LJ ? 3 : 0) + (EL != 0 ? 3 : 0);
+    constexpr int E0 = LJ ? 3 : 0;                           // first electrostatic sum
+    __shared__ double fs[WATER ? 1 : ATOMS][SUMS];
+    const int first = mx_xcd_block(blockIdx.x, gridDim.x) * ATOMS;
     mx_resolve_step(kp);
-    const int i = gid / G;
-    const int lane = gid & (G - 1);
-    double tval = 0.0;
+    const int tid = threadIdx.x;
+    const int i = first + tid / G;
+    const int lane = tid & (G - 1);
+    // the component this lane ends the step of: atom g * 16 + (lane of the wavefront) / 3
+    const int wl = tid & 63, wave = tid >> 6;
+    const int ca = wl / 3, cc = wl - 3 * ca;
+    mx_component C[ROUNDS];
+    bool act[ROUNDS];
+    if constexpr (!WATER) {
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) {   // loaded while the pairs are summed
+            const int at = (wave + 4 * r) * MX_GROUP + ca;
+            act[r] = wl < 3 * MX_GROUP && at < ATOMS && first + at < n;
+            if (act[r]) mx_load_component(first + at, cc, n, io, C[r]);
+        }
+    }
     if (i < n) {
         const int cnt = nnb[i];
         const bool io_ = !WATER || (i % 3) == 0;
-        // the atom's inputs to the end of the step, loaded while the pairs are summed
-        mx_atom A;
-        if (lane == 0) {
-            if (WATER) {
-                A.m = io.ms[i];
-                A.q = EL != 0 ? io.qs[i] : 0.0;
-            } else {
-                mx_load_atom(i, n, io, A);
-            }
+        double mi = 1.0, qm = 0.0;
+        if (WATER && lane == 0) {
+            mi = io.ms[i];
+            qm = EL != 0 ? io.qs[i] : 0.0;
         }
         nbx_kahan acc[6];
 #pragma unroll
         for (int q = 0; q < 6; ++q) acc[q].init();
         const size_t stride = (size_t)n * G;
-        const IDX* p = nbr + gid;
+        const IDX* p = nbr + (size_t)i * G + lane;
         // NB_UNROLL slots per lane and pass: the position gathers of a pass are issued
         // together, and the slots of the next pass are loaded while this pass computes,
         // so a lane waits for about one gather per pass rather than two dependent loads
@@ -231,17 +252,44 @@ k_nb_list(const double4* __restrict__ pos, const IDX* __restrict__ nbr,
                 for (int q = 3; q < 6; ++q) acc[q].add(g[q]);
             }
         }
-        double F[6];
-#pragma unroll
-        for (int q = 0; q < 6; ++q) F[q] = lane_sum<G>(acc[q].value());
+        double F[SUMS];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-            F[q] *= iu;
-            F[3 + q] *= iu * iu;
+            if (LJ) F[q] = lane_sum<G>(acc[q].value()) * iu;
+            if (EL != 0) F[E0 + q] = lane_sum<G>(acc[3 + q].value()) * (iu * iu);
         }
-        if (lane == 0) tval = nb_finish<LJ, EL, WATER>(i, n, F, A, pp, kp, io);
+        if (lane == 0) {
+            if constexpr (WATER) {   // bonded terms and the end of the step: per molecule
+                const double cl = LJ ? pp.lj_c / mi : 0.0, ce = EL != 0 ? pp.el_k * qm / mi : 0.0;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    double a = 0.0;
+                    if (LJ) a += cl * F[k];
+                    if (EL != 0) a += ce * F[E0 + k];
+                    io.a[(size_t)k * n + i] = a;
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < SUMS; ++q) fs[tid / G][q] = F[q];
+            }
+        }
     }
-    if (!WATER) mx_epilogue(tval, io, n);
+    if constexpr (!WATER) {
+        __syncthreads();
+        double tval = 0.0;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) {
+            if ((wave + 4 * r) * MX_GROUP >= ATOMS) break;   // the whole wavefront
+            const int at = (wave + 4 * r) * MX_GROUP + ca;
+            double a = 0.0;
+            if (act[r]) {
+                if (LJ) a += pp.lj_c / C[r].m * fs[at][cc];
+                if (EL != 0) a += pp.el_k * C[r].q / C[r].m * fs[at][E0 + cc];
+            }
+            tval += mx_end_component(first + at, cc, n, a, C[r], kp, io, act[r]);
+        }
+        mx_epilogue(tval, io, n);
+    }
 }
 
 // ---------------------------------------------------------------------------
