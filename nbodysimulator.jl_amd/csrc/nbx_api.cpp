@@ -92,7 +92,10 @@ extern "C" int nbx_create(nbx_ctx** out, int64_t n, int32_t system_kind, const d
     c->h_ms.assign(masses, masses + n);
     c->equal_masses = n > 0 && std::all_of(masses, masses + n,
                                            [&](double m) { return m == masses[0]; });
-    if (n > 0) c->mass_wscale = 1.0 / *std::max_element(masses, masses + n);
+    if (n > 0) {
+        c->mass_wscale = 1.0 / *std::max_element(masses, masses + n);
+        c->mass_wmin = 1.0 / *std::min_element(masses, masses + n);
+    }
     if (charges) {
         c->h_qs.assign(charges, charges + n);
         c->has_q = true;
@@ -102,11 +105,17 @@ extern "C" int nbx_create(nbx_ctx** out, int64_t n, int32_t system_kind, const d
     if (const char* g = std::getenv("NBX_GRAPH_STEPS")) c->graph_steps = std::max(0, std::atoi(g));
     if (const char* g = std::getenv("NBX_BUILD_EVERY")) {
         const int m = std::atoi(g);
-        if (m == 1 || m == 2 || m == 5) c->build_every = m;
+        if (m == 1 || m == 2 || m == 5) {
+            c->build_every = m;
+            c->every_auto = false;
+        }
     }
     if (const char* g = std::getenv("NBX_LANES")) {
         const int l = std::atoi(g);
-        if (l == 1 || l == 2 || l == 4 || l == 8 || l == 16 || l == 32) c->nl.lanes = l;
+        if (l == 1 || l == 2 || l == 4 || l == 8 || l == 16 || l == 32) {
+            c->nl.lanes = l;
+            c->nl.lanes_auto = false;
+        }
     }
     // spatial re-sort of the mixed path's state every 10,000 steps from 8,192 atoms on
     // (NBX_SORT_EVERY: another interval for any size, 0 to never sort)
@@ -165,6 +174,7 @@ static void invalidate(nbx_ctx* c) {
     c->accel_valid = false;
     c->nl.ready = false;
     c->list_sorted = false;
+    c->every_chosen = false;
     ++c->version;
 }
 
@@ -388,6 +398,7 @@ extern "C" int nbx_set_state(nbx_ctx* c, const double* u, const double* v) {
     c->state_set = true;
     c->accel_valid = false;
     c->nl.ready = false;
+    c->every_chosen = false;
     c->steps_taken = 0;
     if ((rc = mx_reset_order(c))) return rc;
     return reset_nosehoover(c);

@@ -17,7 +17,7 @@
 // belongs to the drift of the step after the state when a run has ended)
 enum { NBX_SCAL_T = 0, NBX_SCAL_ZETA = 10, NBX_SCAL_XI = 11, NBX_SCAL_XI_SCRATCH = 15,
        NBX_SCAL_ZETA_PREV = 16, NBX_SCAL_XI_PREV = 17, NBX_SCAL_COUNT = 32 };
-enum { NBX_BINS_STEP = 0, NBX_BINS_FIXED = 1, NBX_BINS_BUILD = 2, NBX_FLAG_BINSET = 5 };
+enum { NBX_BINS_STEP = 0, NBX_BINS_FIXED = 1, NBX_BINS_BUILD = 2, NBX_FLAG_BINSET = 5, NBX_FLAG_SPEED = 8, NBX_FLAGS = 16 };
 
 enum { NBX_TERM_LJ = 1, NBX_TERM_ELEC = 2, NBX_TERM_GRAV = 3, NBX_TERM_RF = 4, NBX_TERM_MAG = 5 };
 
@@ -30,6 +30,8 @@ struct nbx_term {
 struct nbx_nlist {
     bool ready = false;
     int lanes = 8;            // lanes per atom in the force kernel (G)
+    bool lanes_auto = true;   // chosen by size when the lists are sized (not by NBX_LANES or
+                              // the autotuner)
     int cap = 0;              // neighbour slots per atom (multiple of lanes)
     int ncell = 0;            // cells per side (0: all-pairs neighbour search)
     int ccap = 0;             // atoms per cell bound
@@ -50,10 +52,11 @@ struct nbx_nlist {
                                   // NBX_BINS_BUILD: three sets rotating at each build)
     int* d_cell_atoms = nullptr;  // 3 x ncells x ccap
     double* d_xref = nullptr; // unwrapped positions at the last build (SoA)
-    int* d_flags = nullptr;   // [0] rebuild request, [1] overflow, [2] builds done,
+    int* d_flags = nullptr;   // NBX_FLAGS ints: [0] rebuild request, [1] overflow, [2] builds done,
                               // [4] block count of the temperature partials, [5] current bin set, [6] build
                               // finish counter, [7] a list went stale between two build
-                              // opportunities
+                              // opportunities, [8..9] bits of the largest squared speed
+                              // when the lists were made (a double)
     size_t cap_bytes = 0;
 };
 
@@ -115,6 +118,10 @@ struct nbx_ctx {
     // more than skin/2 between two opportunities invalidates the chunk, which is replayed
     // with a build opportunity at every step.
     int build_every = 1;
+    bool every_auto = true;     // chosen from the speeds of a new state (not by
+                                // NBX_BUILD_EVERY or the autotuner)
+    bool every_chosen = false;  // for the current state
+    double speed2 = 0.0;        // largest squared speed when its lists were made
     int64_t stale_replays = 0;  // chunks replayed because a list went stale (build_every -> 1)
     // device state
     double* d_x = nullptr;    // positions (unwrapped), 3n
@@ -149,6 +156,7 @@ struct nbx_ctx {
     // 1 / (largest mass): the FP32 gravity positions carry m / m_max, so that the self
     // term's finite 1/r^3 guard times the mass stays finite for any mass scale
     double mass_wscale = 1.0;
+    double mass_wmin = 1.0;     // 1 / (smallest mass)
     nbx_nlist nl;
     int64_t* d_step = nullptr;       // absolute step base read by replayed graphs
     hipGraphExec_t gexec = nullptr;  // captured block of mixed-path steps

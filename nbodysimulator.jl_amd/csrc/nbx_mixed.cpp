@@ -16,6 +16,7 @@
 #include <vector>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <string>
 
 #include "nbx_mixed.h"
@@ -126,18 +127,37 @@ void free_nl(nbx_nlist& nl) {
 int round_up(int x, int m) { return ((x + m - 1) / m) * m; }
 
 int alloc_flags(nbx_ctx* c) {
-    NBX_HIP(c, hipMalloc((void**)&c->nl.d_flags, sizeof(int) * 8));
-    NBX_HIP(c, hipMemsetAsync(c->nl.d_flags, 0, sizeof(int) * 8, c->stream));
+    NBX_HIP(c, hipMalloc((void**)&c->nl.d_flags, sizeof(int) * NBX_FLAGS));
+    NBX_HIP(c, hipMemsetAsync(c->nl.d_flags, 0, sizeof(int) * NBX_FLAGS, c->stream));
     return NBX_OK;
+}
+
+// Lanes per atom of the list force kernel for n atoms with `entries` list entries each: as
+// many as fill the chip (about 262,144 lanes, four wavefronts per SIMD), since fewer entries
+// per lane shorten its chain of dependent gathers, but not so many that a lane holds less than
+// one pass.  Measured us per step at 4 / 8 / 16 / 32 lanes -- Lennard-Jones (78 entries): n =
+// 864 9.7 / 7.4 / 6.5 / 6.3, 4,000 12.0 / 9.6 / 8.8 / 8.8, 8,000 12.3 / 10.0 / 9.5 / 10.0,
+// 32,000 15.0 / 14.0 / 15.0 / 17.9, 200,000 43.9 / 46.2 / 52.3 / 68.7; water (about 450
+// entries): 12,288 atoms 41 / 30 / 26.0 / 25.4, 24,000 47 / 37.5 / 35.5 / 36.4.
+int lanes_by_size(int64_t n, double entries) {
+    int g = n <= 4096 ? 32 : 16;
+    if (entries < 256.0)   // long lists keep 16 lanes busy at any size
+        while (g > 4 && n * g > 262144) g /= 2;
+    return g;
 }
 
 // size and allocate the lists for the current configuration (cap/ccap grown by `grow`)
 int alloc_lists(nbx_ctx* c, const mx_plan& p, double grow) {
     nbx_nlist& nl = c->nl;
+    const int64_t n = c->n;
+    {
+        const double L = c->bc.b[0], r = p.cutoff + (c->skin_set ? c->skin : 0.12 * p.cutoff);
+        if (nl.lanes_auto)
+            nl.lanes = lanes_by_size(n, 4.0 / 3.0 * M_PI * r * r * r * (double)n / (L * L * L));
+    }
     const int lanes = nl.lanes;
     free_nl(nl);
     nl.lanes = lanes;
-    const int64_t n = c->n;
     // the list kernels index one list row of n * lanes slots in 32 bits
     if (n * (int64_t)std::max(lanes, 1) >= (int64_t)1 << 32)
         return nbx_fail(c, NBX_ERR_CAPACITY, "n x lanes per atom must stay below 2^32");
@@ -451,6 +471,9 @@ static int prologue(nbx_ctx* c, mx_plan& p) {
     // the Berendsen term of the first evaluation uses v itself (vh := v)
     NBX_HIP(c, hipMemcpyAsync(c->d_vh, c->d_v, sizeof(double) * 3 * (size_t)c->n,
                               hipMemcpyDeviceToDevice, s));
+    if (p.kind != PLAN_GRAVITY && p.nb.mode_list)
+        mx_launch_max_speed(s, c->d_v, c->n,
+                            reinterpret_cast<unsigned long long*>(c->nl.d_flags + NBX_FLAG_SPEED));
     launch_build(c, p, 0);
     launch_step(c, p, kick_params(c, 0, 0.0, 0), 0, 0);
     NBX_HIP(c, hipGetLastError());
@@ -459,9 +482,32 @@ static int prologue(nbx_ctx* c, mx_plan& p) {
 }
 
 static int read_flags(nbx_ctx* c, int* h) {
-    NBX_HIP(c, hipMemcpyAsync(h, c->nl.d_flags, sizeof(int) * 8, hipMemcpyDeviceToHost, c->stream));
+    NBX_HIP(c, hipMemcpyAsync(h, c->nl.d_flags, sizeof(int) * NBX_FLAGS, hipMemcpyDeviceToHost, c->stream));
     NBX_HIP(c, hipStreamSynchronize(c->stream));
     return NBX_OK;
+}
+
+// Steps between build opportunities for a new state, from its largest speed (the thermostat's
+// five-sigma speed where that is larger): the largest interval M whose last M steps before
+// a build carry the fastest atom, with a quarter to spare, no further than the margin between
+// the build request and skin / 2 (make_io).  Each opportunity costs two gated launches of
+// 2 to 3 us; the earlier requests of M = 5 rebuild about half as often again (whole runs:
+// Lennard-Jones, n = 32,000, 250 steps of 0.002 4.13 -> 3.98 ms, n = 864 with the lanes by
+// size, 300 steps 2.82 -> 1.86 ms).  A state that speeds up past it marks a list stale and is
+// replayed with M = 1, as with any interval.
+static void choose_build_every(nbx_ctx* c, const mx_plan& p, double dt) {
+    if (!c->every_auto || c->every_chosen || p.kind == PLAN_GRAVITY || !p.nb.mode_list) return;
+    c->every_chosen = true;
+    double v2 = c->speed2;
+    if (c->therm != NBX_THERM_NONE && c->n > 0)
+        v2 = std::max(v2, 25.0 * c->kb * c->therm_T * c->mass_wmin);
+    const double reach = 1.25 * std::sqrt(v2) * dt;
+    c->build_every = 1;
+    for (int M : {5, 2})
+        if (reach * M <= 0.5 * c->nl.skin * (double)(M - 1) / (2.0 * M)) {
+            c->build_every = M;
+            break;
+        }
 }
 
 static int grow_lists(nbx_ctx* c, mx_plan& p, double& grow) {
@@ -491,13 +537,14 @@ static int ensure_ready(nbx_ctx* c, mx_plan& p, bool run = false) {
         c->list_sorted = false;   // the list made here is for the state's current order
         if ((rc = prepare(c, p, grow))) return rc;
         if ((rc = prologue(c, p))) return rc;
-        int h[8];
+        int h[NBX_FLAGS];
         if ((rc = read_flags(c, h))) return rc;
         while (h[1]) {
             if ((rc = grow_lists(c, p, grow))) return rc;
             if ((rc = prologue(c, p))) return rc;
             if ((rc = read_flags(c, h))) return rc;
         }
+        std::memcpy(&c->speed2, h + NBX_FLAG_SPEED, sizeof(double));
         return NBX_OK;
     }
     std::string why;
@@ -553,7 +600,7 @@ static int rebuild_list(nbx_ctx* c, mx_plan& p) {
         refresh_positions(c, p, true);
         launch_build(c, p, 0);
         NBX_HIP(c, hipGetLastError());
-        int h[8];
+        int h[NBX_FLAGS];
         if ((rc = read_flags(c, h))) return rc;
         if (!h[1]) return NBX_OK;
         if (attempt > 8) return nbx_fail(c, NBX_ERR_CAPACITY, "list overflow persists");
@@ -618,6 +665,7 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
     mx_plan p;
     int rc;
     if ((rc = ensure_ready(c, p, true))) return rc;
+    choose_build_every(c, p, dt);
     // the run keeps the state in the sorted order and returns it in the user's order
     const bool sorting = allow_sort && sort_enabled(c, p);
     struct order_guard {
@@ -784,7 +832,7 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
             if (chunk & 1)  // the state is in X[1]
                 NBX_HIP(c, hipMemcpyAsync(c->d_x, c->d_x2, sizeof(double) * n3,
                                           hipMemcpyDeviceToDevice, s));
-            int h[8];
+            int h[NBX_FLAGS];
             if ((rc = read_flags(c, h))) return rc;
             if (!h[1] && !h[7]) {
                 // the chunk stands: add its force-kernel times (the stream has drained)
@@ -983,7 +1031,7 @@ int fresh_list(nbx_ctx* c, mx_plan& p) {
         refresh_positions(c, p, true);
         launch_build(c, p, 0);
         NBX_HIP(c, hipGetLastError());
-        int h[8];
+        int h[NBX_FLAGS];
         if ((rc = read_flags(c, h))) return rc;
         if (!h[1]) return NBX_OK;
         if (attempt > 8) return nbx_fail(c, NBX_ERR_CAPACITY, "list overflow persists");
@@ -1172,7 +1220,7 @@ int mx_learned_run(nbx_ctx* c, const nbx_model* m, double dt, int stride, int64_
     double ke0, pe0;
     if ((rc = list_energy(c, 0, lj, epart, &ke0, &pe0))) return rc;
     const double E0 = ke0 + pe0;
-    int hflags[8];
+    int hflags[NBX_FLAGS];
     if ((rc = read_flags(c, hflags))) return rc;
     const int builds0 = hflags[2];
     const double D = dt * stride;
@@ -1414,6 +1462,7 @@ int mx_autotune(nbx_ctx* c, double dt, int trial, double* out, int nout) {
                 c->grav_chunks_set = (int)r.shape1;
             } else {
                 c->nl.lanes = (int)r.shape0;
+                c->nl.lanes_auto = c->every_auto = false;
                 c->skin = r.shape1;
                 c->skin_set = true;
                 c->build_every = (int)r.every;
@@ -1514,16 +1563,17 @@ int mx_autotune(nbx_ctx* c, double dt, int trial, double* out, int nout) {
         const int lanes0 = c->nl.lanes;
         const double skin0 = c->skin;
         const bool skin_set0 = c->skin_set;
-        const int every0 = c->build_every;
+        const bool lanes_auto0 = c->nl.lanes_auto, every_auto0 = c->every_auto;
         if ((rc = time_config(&base_ms))) return rc;
         best_ms = base_ms;
-        best0 = lanes0;
+        best0 = c->nl.lanes;
         best1 = c->nl.skin;
         best2 = build_every(c);
         const int lanes_c[5] = {2, 4, 8, 16, 32};
         const double skin_c[8] = {0.06, 0.09, 0.12, 0.15, 0.18, 0.24, 0.32, 0.40};
         const int every_c[3] = {1, 2, 5};
         bool set_best = false;
+        c->nl.lanes_auto = c->every_auto = false;
         for (int ei = 0; ei < 3; ++ei)
             for (int li = 0; li < 5; ++li)
                 for (int si = 0; si < 8; ++si) {
@@ -1555,9 +1605,12 @@ int mx_autotune(nbx_ctx* c, double dt, int trial, double* out, int nout) {
             c->build_every = (int)best2;
         } else {
             c->nl.lanes = lanes0;
+            c->nl.lanes_auto = lanes_auto0;
             c->skin = skin0;
             c->skin_set = skin_set0;
-            c->build_every = every0;
+            c->build_every = (int)best2;
+            c->every_auto = every_auto0;
+            c->every_chosen = false;
         }
     }
     if ((rc = restore())) return rc;

@@ -544,6 +544,8 @@ void mx_launch_magnetic(hipStream_t s, const nbx_ctx* c, const void* pos, double
                         const mx_kick_params& kp, const mx_io& io, int force_only_kernel);
 void mx_launch_step_advance(hipStream_t s, int64_t* step_base, int64_t delta, int set);
 void mx_launch_fill_int(hipStream_t s, int* p, int64_t count, int value);
+// *bits = max(*bits, bits of the largest |v|^2): the order of non-negative doubles
+void mx_launch_max_speed(hipStream_t s, const double* v, int64_t n, unsigned long long* bits);
 // bins of P (gated by *req; the bins were cleared by the build kernel that used them last)
 void mx_launch_bin(hipStream_t s, const nbx_ctx* c, const void* pos, const int* req,
                    int* bin_count, int* bin_atoms);

@@ -451,6 +451,24 @@ void mx_launch_fill_int(hipStream_t s, int* p, int64_t count, int value) {
     hipLaunchKernelGGL(k_fill_int, dim3(nbx_blocks(count, 256)), dim3(256), 0, s, p, count, value);
 }
 
+__global__ void __launch_bounds__(256)
+k_max_speed(const double* __restrict__ v, int n, unsigned long long* __restrict__ bits) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    double s = 0.0;
+    if (i < n) {
+        const double a = v[i], b = v[n + i], c = v[2 * (size_t)n + i];
+        s = a * a + b * b + c * c;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s = fmax(s, __shfl_xor(s, off, 64));
+    if ((threadIdx.x & 63) == 0) atomicMax(bits, (unsigned long long)__double_as_longlong(s));
+}
+
+void mx_launch_max_speed(hipStream_t s, const double* v, int64_t n, unsigned long long* bits) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_max_speed, dim3(nbx_blocks(n, 256)), dim3(256), 0, s, v, (int)n, bits);
+}
+
 // wrapped copy of x (after set_state), binned; requests a list build
 __global__ void k_mx_positions(const double* __restrict__ x, int n, int kind, void* pos,
                                double L, double wscale, const double* __restrict__ ms,
