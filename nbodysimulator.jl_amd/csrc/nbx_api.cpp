@@ -754,6 +754,41 @@ static int ref_vv_fused(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, in
     return NBX_OK;
 }
 
+// the small systems whose whole run is one workgroup's (ref64_small_run)
+static int ref_vv_small(nbx_ctx* c, double dt, int64_t nsteps, int64_t save_every,
+                        frame_sink* frames) {
+    std::vector<ref64_term> terms;
+    for (const nbx_term& t : c->terms) {
+        ref64_term r{};
+        if (!ref_pair_term(c, t, &r)) {   // magnetic dipoles
+            r.kind = t.kind;
+            for (int k = 0; k < 4; ++k) r.p[k] = t.p[k];
+        }
+        terms.push_back(r);
+    }
+    const int64_t n3 = 3 * c->n, step0 = c->steps_taken;
+    int64_t done = 0;
+    while (done < nsteps) {
+        // a launch ends after 20,000 steps (some 10 ms), or when the frames fill their buffer
+        int64_t m = std::min<int64_t>(nsteps - done, 20000);
+        if (frames) m = std::min(m, (frames->cap - frames->pending) * save_every - done % save_every);
+        double* const u = frames ? c->d_frames + frames->pending * n3 : nullptr;
+        double* const v = frames ? c->d_frames + (frames->cap + frames->pending) * n3 : nullptr;
+        ref64_small_run(c->stream, (int)c->n, c->d_x, c->d_v, c->d_a, c->d_ms, c->d_qs,
+                        c->mm_set ? c->d_mm : nullptr, terms.data(), (int)terms.size(), c->bc, dt, done,
+                        m, frames ? save_every : 0, u, v);
+        NBX_HIP(c, hipGetLastError());
+        if (frames) {
+            frames->pending += (done + m) / save_every - done / save_every;
+            if (frames->pending == frames->cap)
+                if (int rc = frames->flush()) return rc;
+        }
+        done += m;
+        c->steps_taken = step0 + done;
+    }
+    return NBX_OK;
+}
+
 static int ref_vv(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t save_every,
                   double* uf, double* vf) {
     hipStream_t s = c->stream;
@@ -774,6 +809,11 @@ static int ref_vv(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t 
         c->accel_valid = true;
     }
     const int water = c->sys == NBX_SYS_WATER;
+    if (nsteps > 0 && !water && c->n <= NBX_REF_SMALL && c->therm == NBX_THERM_NONE &&
+        !c->terms.empty()) {
+        if ((rc = ref_vv_small(c, dt, nsteps, save_every, frames))) return rc;
+        return frames ? sink.flush() : NBX_OK;
+    }
     if (nsteps > 0 && ref_fuses(c)) {
         if ((rc = ref_vv_fused(c, dt, nsteps, seed, save_every, frames))) return rc;
         return frames ? sink.flush() : NBX_OK;

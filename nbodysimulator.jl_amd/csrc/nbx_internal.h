@@ -263,6 +263,14 @@ void ref64_water_step(hipStream_t s, const ref64_term& el, const ref64_term& lj,
                       const double* ms, const double* qs, int64_t n, const nbx_bcv& bc,
                       double* elec, double* ljv, double rOH, double kbond, double aHOH, double ka,
                       const ref64_step& st);
+// up to NBX_REF_SMALL bodies of a potential system without a thermostat run all their steps in
+// one workgroup (its pair terms fill 56 KiB of LDS): nsteps steps after step0 from (x, v, a),
+// frames of the multiples of save_every from uf, vf on
+#define NBX_REF_SMALL 48
+void ref64_small_run(hipStream_t s, int n, double* x, double* v, double* a, const double* ms,
+                     const double* qs, const double* mm, const ref64_term* terms, int count,
+                     const nbx_bcv& bc, double dt, int64_t step0, int64_t nsteps, int64_t save_every,
+                     double* uf, double* vf);
 // up to this many bodies gravity gives each target a wavefront (n = 16,000: 2.0 ms per
 // evaluation against 2.9 with a thread per target; twice the bodies 8 against 5.3)
 #define NBX_REF_GRAV_WAVES 16384

@@ -494,6 +494,20 @@ __device__ __forceinline__ double ref_norm3(double x, double y, double z) {
 //   c_k = (((mi_k mij + mj_k mir) + r_k (mi.mj)) - ((5 r_k) mir) mij) / rij4
 // then dv += (3 mu_4pi / m_i) * sum_j c.  mm: moments SoA (component k at k*n + j).
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ void ref_mag_term(double rx, double ry, double rz, const double* mi,
+                                             const double* mj, double* t) {
+    const double d = (rx * rx + ry * ry) + rz * rz;
+    const double rij4 = d * d;
+    const double nr = ref_norm3(rx, ry, rz);
+    const double r1 = rx / nr, r2 = ry / nr, r3 = rz / nr;
+    const double mir = (mi[0] * r1 + mi[1] * r2) + mi[2] * r3;
+    const double mij = (mj[0] * r1 + mj[1] * r2) + mj[2] * r3;
+    const double dmm = (mi[0] * mj[0] + mi[1] * mj[1]) + mi[2] * mj[2];
+    t[0] = (((mi[0] * mij + mj[0] * mir) + r1 * dmm) - ((5.0 * r1) * mir) * mij) / rij4;
+    t[1] = (((mi[1] * mij + mj[1] * mir) + r2 * dmm) - ((5.0 * r2) * mir) * mij) / rij4;
+    t[2] = (((mi[2] * mij + mj[2] * mir) + r3 * dmm) - ((5.0 * r3) * mir) * mij) / rij4;
+}
+
 __global__ void __launch_bounds__(REF_TILE)
 k_ref_mag(const double* __restrict__ x, double* __restrict__ dv, const double* __restrict__ ms,
           const double* __restrict__ mm, int64_t n, int64_t ib, int64_t ie, double mu_4pi) {
@@ -518,18 +532,12 @@ k_ref_mag(const double* __restrict__ x, double* __restrict__ dv, const double* _
         if (active) {
             for (int q = 0; q < lim; ++q) {
                 if (base + q == i) continue;
-                const double rx = xi - sx[q], ry = yi - sy[q], rz = zi - sz[q];
-                const double d = (rx * rx + ry * ry) + rz * rz;
-                const double rij4 = d * d;
-                const double nr = ref_norm3(rx, ry, rz);
-                const double r1 = rx / nr, r2 = ry / nr, r3 = rz / nr;
-                const double mjx = smx[q], mjy = smy[q], mjz = smz[q];
-                const double mir = (mix * r1 + miy * r2) + miz * r3;
-                const double mij = (mjx * r1 + mjy * r2) + mjz * r3;
-                const double dmm = (mix * mjx + miy * mjy) + miz * mjz;
-                f1 += (((mix * mij + mjx * mir) + r1 * dmm) - ((5.0 * r1) * mir) * mij) / rij4;
-                f2 += (((miy * mij + mjy * mir) + r2 * dmm) - ((5.0 * r2) * mir) * mij) / rij4;
-                f3 += (((miz * mij + mjz * mir) + r3 * dmm) - ((5.0 * r3) * mir) * mij) / rij4;
+                const double mi[3] = {mix, miy, miz}, mj[3] = {smx[q], smy[q], smz[q]};
+                double t[3];
+                ref_mag_term(xi - sx[q], yi - sy[q], zi - sz[q], mi, mj, t);
+                f1 += t[0];
+                f2 += t[1];
+                f3 += t[2];
             }
         }
         __syncthreads();
@@ -547,6 +555,156 @@ void ref64_mag(hipStream_t s, const double* x, double* dv, const double* ms, con
     if (ie <= ib) return;
     hipLaunchKernelGGL(k_ref_mag, dim3(nbx_blocks(ie - ib, REF_TILE)), dim3(REF_TILE), 0, s, x,
                        dv, ms, mm, n, ib, ie, mu_4pi);
+}
+
+// ---------------------------------------------------------------------------
+// Few bodies: a whole run of velocity-Verlet steps in one workgroup
+// ---------------------------------------------------------------------------
+
+// With a few bodies a step is a handful of dependent FP64 operations, and launches are all
+// its cost (8 bodies: a force kernel and a frame kernel per step, 7.0 us; here 0.7).  The
+// state lives in LDS.  Per potential, every ordered pair's term is evaluated by a thread of
+// its own (phase A), then a thread per body and component adds its row in ascending j
+// (phase B) -- the sums of k_ref_pairs, bit for bit; a pair out of range or the body itself
+// contributes the +0.0 that leaves a sum unchanged.  Then the same thread kicks, writes the
+// frame if one is due, and drifts.  A latency chain of about 1,600 cycles and two barriers
+// per step, most of it the square root, the division and the ordered adds.
+struct ref_small_laws {
+    ref_law law[8];
+    int kind[8];
+    int count;
+};
+
+template <int KIND>
+__device__ __forceinline__ void ref_small_term(const ref_law& law, const double* x, const double* w,
+                                               const nbx_bcv& bc, int i, int j, double* t) {
+    t[0] = t[1] = t[2] = 0.0;
+    if (i != j)
+        (void)ref_pair_term<KIND>(law, x[3 * i], x[3 * i + 1], x[3 * i + 2], x[3 * j],
+                                  x[3 * j + 1], x[3 * j + 2], w[j], bc, t);
+}
+
+__global__ void __launch_bounds__(1024)
+k_ref_small(int n, double* __restrict__ gx, double* __restrict__ gv, double* __restrict__ ga,
+            const double* __restrict__ gms, const double* __restrict__ gqs,
+            const double* __restrict__ gmm, ref_small_laws laws, nbx_bcv bc, double dt, int64_t step0,
+            int64_t nsteps, int64_t save_every, double* __restrict__ uf, double* __restrict__ vf) {
+    constexpr int N = NBX_REF_SMALL;
+    __shared__ double term[3 * N * (N + 1)];
+    __shared__ double x[3 * N], mm[3 * N], ms[N], qs[N];
+    const int tid = threadIdx.x;
+    const int ld = n | 1;          // odd: the rows of phase B start in different banks
+    const int n3 = 3 * n;
+    if (tid < n) {
+        ms[tid] = gms[tid];
+        qs[tid] = gqs[tid];
+    }
+    // thread t < 3 n: component c of body b
+    const int b = tid / 3, c = tid - 3 * b;
+    const bool own = tid < n3;
+    double px = 0.0, v = 0.0, a = 0.0, vh = 0.0;
+    const double half = 0.5, dtsq = dt * dt;
+    if (own) {
+        px = gx[c * n + b];
+        v = gv[c * n + b];
+        a = ga[c * n + b];
+        if (gmm != nullptr) mm[tid] = gmm[c * n + b];
+    }
+    // the thread's pairs of phase A, and the frame that is due next
+    constexpr int PAIRS = (N * N + 1023) / 1024;
+    int pi[PAIRS], pj[PAIRS];
+#pragma unroll
+    for (int q = 0; q < PAIRS; ++q) {
+        const int p = tid + q * (int)blockDim.x;
+        pi[q] = p < n * n ? p / n : -1;
+        pj[q] = p - pi[q] * n;
+    }
+    int64_t due = save_every > 0 ? save_every - step0 % save_every : nsteps + 1;
+    double* fu = uf + tid;
+    double* fv = vf + tid;
+    __syncthreads();
+    for (int64_t s = 1; s <= nsteps; ++s) {
+        if (own) {   // drift
+            px = px + dt * v + dtsq * (half * a);
+            vh = v + dt * (half * a);
+            x[tid] = px;
+            a = 0.0;
+        }
+        __syncthreads();
+        for (int q = 0; q < laws.count; ++q) {
+            const ref_law& law = laws.law[q];
+            const int kind = laws.kind[q];
+#pragma unroll
+            for (int r = 0; r < PAIRS; ++r) {
+                const int i = pi[r], j = pj[r];
+                if (i < 0) break;
+                double t[3];
+                if (kind == NBX_TERM_LJ) ref_small_term<REF_LJ>(law, x, ms, bc, i, j, t);
+                else if (kind == NBX_TERM_ELEC) ref_small_term<REF_COULOMB>(law, x, qs, bc, i, j, t);
+                else if (kind == NBX_TERM_RF) ref_small_term<REF_RF>(law, x, qs, bc, i, j, t);
+                else if (kind == NBX_TERM_GRAV) ref_small_term<REF_GRAV>(law, x, ms, bc, i, j, t);
+                else if (i == j) t[0] = t[1] = t[2] = 0.0;
+                else ref_mag_term(x[3 * i] - x[3 * j], x[3 * i + 1] - x[3 * j + 1],
+                                  x[3 * i + 2] - x[3 * j + 2], mm + 3 * i, mm + 3 * j, t);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) term[(3 * i + k) * ld + j] = t[k];
+            }
+            __syncthreads();
+            if (own) {
+                const double* row = term + tid * ld;
+                double f = 0.0;
+                int j = 0;
+                for (; j + 8 <= n; j += 8) {
+                    double u[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) u[k] = row[j + k];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) f += u[k];
+                }
+                for (; j < n; ++j) f += row[j];
+                double add = f;
+                if (kind == NBX_TERM_LJ) add = 24.0 * law.c / ms[b] * f;
+                else if (kind == NBX_TERM_MAG) add = 3.0 * law.c / ms[b] * f;
+                else if (kind != NBX_TERM_GRAV) add = law.c * qs[b] / ms[b] * f;
+                a += add;
+            }
+            if (q + 1 < laws.count) __syncthreads();   // the rows are read before the next terms
+        }
+        if (own) {   // kick; the barrier after the next drift separates it from the terms
+            v = vh + dt * (0.5 * a);
+            if (s == due) {
+                *fu = px;
+                *fv = v;
+                fu += n3;
+                fv += n3;
+                due += save_every;
+            }
+        }
+    }
+    if (own) {
+        gx[c * n + b] = px;
+        gv[c * n + b] = v;
+        ga[c * n + b] = a;
+    }
+}
+
+void ref64_small_run(hipStream_t s, int n, double* x, double* v, double* a, const double* ms,
+                     const double* qs, const double* mm, const ref64_term* terms, int count,
+                     const nbx_bcv& bc, double dt, int64_t step0, int64_t nsteps, int64_t save_every,
+                     double* uf, double* vf) {
+    ref_small_laws laws{};
+    laws.count = count;
+    for (int q = 0; q < count; ++q) {
+        ref64_term t = terms[q];
+        t.filter = false;
+        laws.kind[q] = t.kind;
+        if (t.kind == NBX_TERM_MAG) laws.law[q].c = t.p[0];
+        else laws.law[q] = make_law(t, bc);
+    }
+    const int want = std::max(n * n, 3 * n);
+    const int threads = std::min(1024, (want + 63) / 64 * 64);
+    hipLaunchKernelGGL(k_ref_small, dim3(1), dim3(threads), 0, s, n, x, v, a, ms, qs, mm, laws, bc, dt,
+                       step0, nsteps, save_every, uf, vf);
 }
 
 // ---------------------------------------------------------------------------

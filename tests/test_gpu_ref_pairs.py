@@ -121,3 +121,41 @@ def test_water_runs_match_oracle(nbx, el, rc, therm):
     uo, vo, (ufo, vfo) = orc.vv_run(w.u, w.v, 0.0005, 15, seed=5, save_every=5)
     for a, b in ((u, uo), (v, vo), (uf, ufo), (vf, vfo)):      # acos in the angle: libm
         assert np.abs(a - b).max() <= 1e-11 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("law,bc", [("gravity", "infinite"), ("open", "infinite"), ("lj", "cubic"),
+                                    ("rf", "cubic"), ("lj", "lohi"), ("grav+el+lj", "infinite"),
+                                    ("magnetic", "infinite")])
+@pytest.mark.parametrize("n", [1, 2, 3, 8, 9, 21, 33, 47, 48, 49])
+def test_small_runs_bitwise(nbx, n, law, bc):
+    print(f"[case] fp64 small run n={n} law={law} bc={bc}", flush=True)
+    L = 1.2 * max(n, 8) ** (1.0 / 3.0)
+    if law == "magnetic":
+        rng = np.random.default_rng(n)
+        m, mm = rng.uniform(0.5, 2.0, n), 0.1 * rng.standard_normal((n, 3))
+        ctx, orc = _lib.Context(n, _lib.SYS_POTENTIAL, m), O.System(m).moments(mm)
+        ctx.set_moments(mm)
+        ctx.add_magnetostatic(0.3)
+        orc.add(O.TERM_MAG, 0.3)
+    else:
+        ctx, orc, rng = pair(n, law, bc, L, 2)
+    u, v = lattice(n, L, rng), 0.3 * rng.standard_normal((n, 3))
+    ctx.set_state(u, v)
+    uf, vf = ctx.vv_run(0.002, 25, save_every=3)
+    ctx.vv_run(0.002, 1)
+    ctx.vv_run(0.002, 14)
+    u1, v1 = ctx.get_state()
+    uo, vo, (ufo, vfo) = orc.vv_run(u, v, 0.002, 40, save_every=3)
+    assert np.array_equal(u1, uo) and np.array_equal(v1, vo) and ctx.steps_taken() == 40
+    assert np.array_equal(uf, ufo[:9]) and np.array_equal(vf, vfo[:9])
+
+
+def test_small_run_of_several_launches(nbx):
+    print("[case] fp64 small run, 45,000 steps", flush=True)
+    ctx, orc, rng = pair(2, "gravity", "infinite", 3.0)
+    u, v = np.array([[0.0, 0, 0], [1.0, 0, 0]]), np.array([[0.0, -0.3, 0], [0, 0.6, 0.1]])
+    ctx.set_state(u, v)
+    uf, vf = ctx.vv_run(1e-3, 45000, save_every=7)
+    uo, vo, (ufo, vfo) = orc.vv_run(u, v, 1e-3, 45000, save_every=7)
+    assert np.array_equal(uf, ufo) and np.array_equal(vf, vfo)
+    assert np.array_equal(ctx.get_state()[0], uo)
