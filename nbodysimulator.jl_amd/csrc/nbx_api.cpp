@@ -15,6 +15,7 @@
 #include "nbx_internal.h"
 
 static thread_local std::string g_create_error;
+void mx_launch_iota(hipStream_t s, int* p, int64_t n);   // nbx_sort.hip
 
 int nbx_fail(nbx_ctx* c, int code, const std::string& msg) {
     if (c) c->err = msg;
@@ -40,23 +41,14 @@ static void free_ptr(void* p) {
 
 static void release(nbx_ctx* c) {
     mx_release(c);
-    free_ptr(c->d_x); free_ptr(c->d_v); free_ptr(c->d_a); free_ptr(c->d_vh);
-    free_ptr(c->d_tmp); free_ptr(c->d_ms); free_ptr(c->d_qs); free_ptr(c->d_red);
-    free_ptr(c->d_scal);
-    free_ptr(c->d_rdf_work); free_ptr(c->d_frac); free_ptr(c->d_rhs); free_ptr(c->d_water);
-    free_ptr(c->d_frames);
-    c->d_rdf_work = c->d_rhs = c->d_water = c->d_frames = nullptr;
+    void* const own[] = {c->d_base, c->d_mm, c->d_mm4, c->d_rdf_work, c->d_frac, c->d_rhs, c->d_water,
+                         c->d_frames, c->d_backup, c->d_sortbuf, c->d_permbuf};
+    for (void* p : own) free_ptr(p);
+    c->d_base = nullptr;
+    c->d_rdf_work = c->d_rhs = c->d_water = c->d_frames = c->d_backup = c->d_permbuf = nullptr;
     c->d_frac = nullptr;
-    free_ptr(c->d_mm);
-    free_ptr(c->d_mm4);
-    if (c->d_perm) (void)hipFree(c->d_perm);
-    if (c->d_iperm) (void)hipFree(c->d_iperm);
-    if (c->d_pmap) (void)hipFree(c->d_pmap);
-    if (c->d_sortbuf) (void)hipFree(c->d_sortbuf);
-    if (c->d_permbuf) (void)hipFree(c->d_permbuf);
     c->d_perm = c->d_iperm = c->d_pmap = nullptr;
     c->d_sortbuf = nullptr;
-    c->d_permbuf = nullptr;
     c->sortbuf_bytes = 0;
     c->d_mm = nullptr;
     c->d_mm4 = nullptr;
@@ -126,32 +118,40 @@ extern "C" int nbx_create(nbx_ctx** out, int64_t n, int32_t system_kind, const d
     // set-up of nbx_rdf_noalloc: the device address of this GPU's histogram array
     if (e == hipSuccess && ref64_rdf_scratch(c->device, &c->d_rdf_hist) != 0)
         e = hipErrorInvalidSymbol;
-    const size_t b3 = sizeof(double) * (size_t)(3 * (n > 0 ? n : 1));
-    const size_t b1 = sizeof(double) * (size_t)(n > 0 ? n : 1);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_x, b3);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_v, b3);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_a, b3);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_vh, b3);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_tmp, b3);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_ms, b1);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_qs, b1);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_red, b1 + 8192 * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_scal, NBX_SCAL_COUNT * sizeof(double));
-    const size_t bi = sizeof(int) * (size_t)(n > 0 ? n : 1);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_perm, bi);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_iperm, bi);
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_pmap, bi);
-    if (e == hipSuccess && n > 0) {
-        std::vector<int> iota((size_t)n);
-        for (int64_t k = 0; k < n; ++k) iota[(size_t)k] = (int)k;
-        e = hipMemcpy(c->d_perm, iota.data(), bi, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMemcpy(c->d_iperm, iota.data(), bi, hipMemcpyHostToDevice);
+    // one allocation for the arrays every context needs, each at a 256-byte boundary
+    const size_t n1 = (size_t)(n > 0 ? n : 1);
+    size_t off = 0;
+    const auto part = [&off](size_t bytes) {
+        const size_t at = off;
+        off += (bytes + 255) / 256 * 256;
+        return at;
+    };
+    const size_t b1 = sizeof(double) * n1, b3 = 3 * b1, bi = sizeof(int) * n1;
+    const size_t at3[5] = {part(b3), part(b3), part(b3), part(b3), part(b3)};
+    const size_t at_ms = part(b1), at_qs = part(b1), at_red = part(b1 + 8192 * sizeof(double)),
+                 at_scal = part(NBX_SCAL_COUNT * sizeof(double)), at_p[3] = {part(bi), part(bi), part(bi)};
+    if (e == hipSuccess) e = hipMalloc((void**)&c->d_base, off);
+    if (e == hipSuccess) {
+        double** const p3[5] = {&c->d_x, &c->d_v, &c->d_a, &c->d_vh, &c->d_tmp};
+        int** const pi[3] = {&c->d_perm, &c->d_iperm, &c->d_pmap};
+        for (int k = 0; k < 5; ++k) *p3[k] = reinterpret_cast<double*>(c->d_base + at3[k]);
+        for (int k = 0; k < 3; ++k) *pi[k] = reinterpret_cast<int*>(c->d_base + at_p[k]);
+        c->d_ms = reinterpret_cast<double*>(c->d_base + at_ms);
+        c->d_qs = reinterpret_cast<double*>(c->d_base + at_qs);
+        c->d_red = reinterpret_cast<double*>(c->d_base + at_red);
+        c->d_scal = reinterpret_cast<double*>(c->d_base + at_scal);
+        // the finite flag and the Nose-Hoover state start at zero
+        ref64_fill(c->stream, c->d_scal, NBX_SCAL_COUNT, 0.0);
+        mx_launch_iota(c->stream, c->d_perm, n);
+        mx_launch_iota(c->stream, c->d_iperm, n);
+        if (n > 0 && !charges) ref64_fill(c->stream, c->d_qs, n, 0.0);
+        e = hipGetLastError();
     }
     if (e == hipSuccess && n > 0)
-        e = hipMemcpy(c->d_ms, masses, b1, hipMemcpyHostToDevice);
+        e = hipMemcpyAsync(c->d_ms, masses, b1, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess && n > 0 && charges)
-        e = hipMemcpy(c->d_qs, charges, b1, hipMemcpyHostToDevice);
-    if (e == hipSuccess && n > 0 && !charges) e = hipMemset(c->d_qs, 0, b1);
+        e = hipMemcpyAsync(c->d_qs, charges, b1, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
         std::string msg = std::string("nbx_create: ") + hipGetErrorString(e);
         release(c);
@@ -279,7 +279,6 @@ extern "C" int nbx_add_gravitational(nbx_ctx* c, double G) {
 }
 
 static int upload_aos(nbx_ctx* c, const double* host, double* d_soa);
-static bool all_finite(const double* p, int64_t count);
 
 extern "C" int nbx_add_magnetostatic(nbx_ctx* c, double mu_4pi) {
     if (!c) return NBX_ERR_INVALID;
@@ -293,7 +292,7 @@ extern "C" int nbx_add_magnetostatic(nbx_ctx* c, double mu_4pi) {
 extern "C" int nbx_set_moments(nbx_ctx* c, const double* mm) {
     if (!c || !mm) return NBX_ERR_INVALID;
     const int64_t n = c->n;
-    if (!all_finite(mm, 3 * n)) return nbx_fail(c, NBX_ERR_NONFINITE, "moments hold NaN or Inf");
+    if (!nbx_all_finite(mm, 3 * n)) return nbx_fail(c, NBX_ERR_NONFINITE, "moments hold NaN or Inf");
     if (!c->d_mm) NBX_HIP(c, hipMalloc((void**)&c->d_mm, sizeof(double) * 3 * (size_t)std::max<int64_t>(n, 1)));
     if (!c->d_mm4) NBX_HIP(c, hipMalloc(&c->d_mm4, sizeof(float) * 4 * (size_t)std::max<int64_t>(n, 1)));
     if (n > 0) {
@@ -331,8 +330,8 @@ extern "C" int nbx_set_spcfw(nbx_ctx* c, double rOH, double aHOH, double kbond, 
 // (gather_bodies_initial_coordinates, src/nbody_to_ode.jl:1-20)
 static int reset_nosehoover(nbx_ctx* c) {
     c->nh_advanced = false;
-    NBX_HIP(c, hipMemsetAsync(c->d_scal + NBX_SCAL_ZETA, 0, 2 * sizeof(double), c->stream));
-    NBX_HIP(c, hipStreamSynchronize(c->stream));
+    ref64_fill(c->stream, c->d_scal + NBX_SCAL_ZETA, 2, 0.0);
+    NBX_HIP(c, hipGetLastError());
     return NBX_OK;
 }
 
@@ -374,17 +373,40 @@ static int download_aos(const nbx_ctx* cc, const double* d_soa, double* host) {
     return NBX_OK;
 }
 
-static bool all_finite(const double* p, int64_t count) {
-    for (int64_t i = 0; i < count; ++i)
-        if (!std::isfinite(p[i])) return false;
-    return true;
+constexpr int64_t NBX_STAGING_DOUBLES = (int64_t)4 << 20;
+
+// staging of `doubles` doubles for frames on their way to the host
+static int frame_staging(nbx_ctx* c, size_t doubles) {
+    if (c->frames_doubles >= doubles) return NBX_OK;
+    free_ptr(c->d_frames);
+    c->d_frames = nullptr;
+    c->frames_doubles = 0;
+    NBX_HIP(c, hipMalloc((void**)&c->d_frames, sizeof(double) * doubles));
+    c->frames_doubles = doubles;
+    return NBX_OK;
+}
+
+// positions and velocities in the caller's layout: one kernel, two copies, one wait; states
+// above the staging's usual 32 MiB go one after the other through d_tmp
+static int download_state(nbx_ctx* c, double* u, double* v) {
+    const size_t n3 = 3 * (size_t)c->n;
+    if (2 * n3 > (size_t)NBX_STAGING_DOUBLES && c->frames_doubles < 2 * n3) {
+        int rc = download_aos(c, c->d_x, u);
+        return rc ? rc : download_aos(c, c->d_v, v);
+    }
+    if (int rc = frame_staging(c, 2 * n3)) return rc;
+    ref64_save_frame(c->stream, c->d_x, c->d_v, c->d_frames, c->d_frames + n3, c->n);
+    NBX_HIP(c, hipMemcpyAsync(u, c->d_frames, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
+    NBX_HIP(c, hipMemcpyAsync(v, c->d_frames + n3, sizeof(double) * n3, hipMemcpyDeviceToHost, c->stream));
+    NBX_HIP(c, hipStreamSynchronize(c->stream));
+    return NBX_OK;
 }
 
 extern "C" int nbx_set_state(nbx_ctx* c, const double* u, const double* v) {
     if (!c) return NBX_ERR_INVALID;
     if (c->n == 0) { c->state_set = true; c->steps_taken = 0; return NBX_OK; }
     if (!u) return nbx_fail(c, NBX_ERR_INVALID, "positions are NULL");
-    if (!all_finite(u, 3 * c->n) || (v && !all_finite(v, 3 * c->n)))
+    if (!nbx_all_finite(u, 3 * c->n) || (v && !nbx_all_finite(v, 3 * c->n)))
         return nbx_fail(c, NBX_ERR_NONFINITE, "state holds NaN or Inf");
     int rc = upload_aos(c, u, c->d_x);
     if (rc) return rc;
@@ -394,23 +416,25 @@ extern "C" int nbx_set_state(nbx_ctx* c, const double* u, const double* v) {
     } else {
         ref64_fill(c->stream, c->d_v, 3 * c->n, 0.0);
     }
-    NBX_HIP(c, hipStreamSynchronize(c->stream));
     c->state_set = true;
     c->accel_valid = false;
     c->nl.ready = false;
     c->every_chosen = false;
     c->steps_taken = 0;
     if ((rc = mx_reset_order(c))) return rc;
-    return reset_nosehoover(c);
+    if ((rc = reset_nosehoover(c))) return rc;
+    NBX_HIP(c, hipStreamSynchronize(c->stream));   // the caller's arrays are free again
+    return NBX_OK;
 }
 
 extern "C" int nbx_get_state(const nbx_ctx* c, double* u, double* v) {
     if (!c) return NBX_ERR_INVALID;
     if (!c->state_set) return nbx_fail(const_cast<nbx_ctx*>(c), NBX_ERR_INVALID, "no state set");
     if (c->n == 0) return NBX_OK;
-    if (u) { int rc = download_aos(c, c->d_x, u); if (rc) return rc; }
-    if (v) { int rc = download_aos(c, c->d_v, v); if (rc) return rc; }
-    return NBX_OK;
+    nbx_ctx* m = const_cast<nbx_ctx*>(c);
+    if (u && v) return download_state(m, u, v);
+    if (u) return download_aos(c, c->d_x, u);
+    return v ? download_aos(c, c->d_v, v) : NBX_OK;
 }
 
 extern "C" int64_t nbx_steps_taken(const nbx_ctx* c) { return c ? c->steps_taken : -1; }
@@ -554,7 +578,7 @@ extern "C" int nbx_rhs(nbx_ctx* c, const double* u, const double* v, double* dv)
     if (!u || !dv) return nbx_fail(c, NBX_ERR_INVALID, "u and dv are required");
     int rc = check_config(c);
     if (rc) return rc;
-    if (!all_finite(u, 3 * c->n)) return nbx_fail(c, NBX_ERR_NONFINITE, "u holds NaN or Inf");
+    if (!nbx_all_finite(u, 3 * c->n)) return nbx_fail(c, NBX_ERR_NONFINITE, "u holds NaN or Inf");
     if ((c->therm == NBX_THERM_BERENDSEN || c->therm == NBX_THERM_NOSEHOOVER) && !v)
         return nbx_fail(c, NBX_ERR_INVALID, "the Berendsen / Nose-Hoover term needs v");
     scratch3 s;
@@ -584,7 +608,7 @@ extern "C" int nbx_accelerations(nbx_ctx* c, int32_t term, const double* u, int6
             (term >= 2 && !c->spcfw_set))
             return nbx_fail(c, NBX_ERR_INVALID, "water term not configured");
     }
-    if (!all_finite(u, 3 * c->n)) return nbx_fail(c, NBX_ERR_NONFINITE, "u holds NaN or Inf");
+    if (!nbx_all_finite(u, 3 * c->n)) return nbx_fail(c, NBX_ERR_NONFINITE, "u holds NaN or Inf");
     scratch3 s;
     int rc;
     if ((rc = alloc_scratch(c, s))) return rc;
@@ -614,9 +638,7 @@ extern "C" int nbx_accelerations(nbx_ctx* c, int32_t term, const double* u, int6
 
 static int save_frame(nbx_ctx* c, int64_t f, double* uf, double* vf) {
     const int64_t n3 = 3 * c->n;
-    int rc = download_aos(c, c->d_x, uf + f * n3);
-    if (rc) return rc;
-    return download_aos(c, c->d_v, vf + f * n3);
+    return download_state(c, uf + f * n3, vf + f * n3);
 }
 
 // Frames of an FP64 run: collected on the device in the caller's layout and copied to the
@@ -629,16 +651,8 @@ struct frame_sink {
 
     int open(int64_t frames) {
         const int64_t n3 = 3 * c->n;
-        cap = std::max<int64_t>(1, std::min<int64_t>(frames, ((int64_t)2 << 20) / n3));
-        const size_t doubles = 2 * (size_t)(cap * n3);
-        if (c->frames_doubles < doubles) {
-            free_ptr(c->d_frames);
-            c->d_frames = nullptr;
-            c->frames_doubles = 0;
-            NBX_HIP(c, hipMalloc((void**)&c->d_frames, sizeof(double) * doubles));
-            c->frames_doubles = doubles;
-        }
-        return NBX_OK;
+        cap = std::max<int64_t>(1, std::min<int64_t>(frames, NBX_STAGING_DOUBLES / 2 / n3));
+        return frame_staging(c, 2 * (size_t)(cap * n3));
     }
     int add(const double* x, const double* v) {
         const int64_t n3 = 3 * c->n;
@@ -844,16 +858,17 @@ int mx_vv(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64_t save_eve
           double* vf, int64_t* nframes);
 int mx_supported(nbx_ctx* c, std::string* why);
 
+// The end of a run: waits for it and reports a state that became NaN or Inf.  The flag is zero
+// until a check sets it, and is cleared when it has been reported.
 static int check_finite_state(nbx_ctx* c) {
     int* d_flag = reinterpret_cast<int*>(c->d_scal + 8);
-    NBX_HIP(c, hipMemsetAsync(d_flag, 0, sizeof(int), c->stream));
-    ref64_check_finite(c->stream, c->d_x, 3 * c->n, d_flag);
-    ref64_check_finite(c->stream, c->d_v, 3 * c->n, d_flag);
+    ref64_check_finite(c->stream, c->d_x, c->d_v, 3 * c->n, d_flag);
     int h = 0;
     NBX_HIP(c, hipMemcpyAsync(&h, d_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     NBX_HIP(c, hipStreamSynchronize(c->stream));
-    if (h) return nbx_fail(c, NBX_ERR_NONFINITE, "the state became NaN or Inf during the run");
-    return NBX_OK;
+    if (!h) return NBX_OK;
+    NBX_HIP(c, hipMemsetAsync(d_flag, 0, sizeof(int), c->stream));
+    return nbx_fail(c, NBX_ERR_NONFINITE, "the state became NaN or Inf during the run");
 }
 
 extern "C" int nbx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed,
@@ -880,7 +895,6 @@ extern "C" int nbx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed,
         rc = ref_vv(c, dt, nsteps, seed, save_every, u_frames, v_frames);
     }
     if (rc) return rc;
-    NBX_HIP(c, hipStreamSynchronize(c->stream));
     return check_finite_state(c);
 }
 
@@ -943,7 +957,6 @@ extern "C" int nbx_em_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed,
         rc = ref_em(c, dt, nsteps, seed, save_every, u_frames, v_frames);
     }
     if (rc) return rc;
-    NBX_HIP(c, hipStreamSynchronize(c->stream));
     return check_finite_state(c);
 }
 

@@ -58,6 +58,7 @@ struct nbx_batch {
     int* d_flags = nullptr;   // [0] overflow, [1] list builds
     int* d_order = nullptr;
     int64_t* d_step = nullptr;
+    double* d_backup = nullptr;   // x, v and a at the start of a run
     void* d_reps = nullptr;
     void* h_params = nullptr;
     bool state_set = false, accel_valid = false;
@@ -90,7 +91,7 @@ static void batch_release(nbx_batch* b) {
     b->gexec = nullptr;
     bfree(b->d_x); bfree(b->d_v); bfree(b->d_a); bfree(b->d_vh); bfree(b->d_xref);
     bfree(b->d_ms); bfree(b->d_tmp); bfree(b->d_nbr); bfree(b->d_nnb); bfree(b->d_flags);
-    bfree(b->d_slot);
+    bfree(b->d_slot); bfree(b->d_backup);
     bfree(b->d_order); bfree(b->d_step); bfree(b->d_reps);
     if (b->h_params) free(b->h_params);
     b->h_params = nullptr;
@@ -266,9 +267,8 @@ static int down3(const nbx_batch* bc, const double* d, double* host) {
 extern "C" int nbx_batch_set_state(nbx_batch* b, const double* u, const double* v) {
     if (!b) return NBX_ERR_INVALID;
     if (!u) return bfail(b, NBX_ERR_INVALID, "positions are NULL");
-    for (int64_t k = 0; k < 3 * b->ntot; ++k)
-        if (!std::isfinite(u[k]) || (v && !std::isfinite(v[k])))
-            return bfail(b, NBX_ERR_NONFINITE, "state holds NaN or Inf");
+    if (!nbx_all_finite(u, 3 * b->ntot) || (v && !nbx_all_finite(v, 3 * b->ntot)))
+        return bfail(b, NBX_ERR_NONFINITE, "state holds NaN or Inf");
     int rc = up3(b, u, b->d_x);
     if (rc) return rc;
     if (v) { if ((rc = up3(b, v, b->d_v))) return rc; }
@@ -319,9 +319,8 @@ extern "C" int nbx_batch_run(nbx_batch* b, double dt, int64_t nsteps, uint64_t s
     if (K > (1 << 30)) return bfail(b, NBX_ERR_INVALID, "steps_per_launch too large");
     hipStream_t s = b->stream;
     const size_t b3 = sizeof(double) * 3 * (size_t)b->ntot;
-    double* bk = nullptr;
-    BHIP(b, hipMalloc((void**)&bk, 3 * b3));
-    struct guard { double* p; ~guard() { if (p) (void)hipFree(p); } } g{bk};
+    if (!b->d_backup) BHIP(b, hipMalloc((void**)&b->d_backup, 3 * b3));
+    double* const bk = b->d_backup;
     double grow = 1.0;
     const int64_t step0 = b->steps_taken;
     const bool had_accel = b->accel_valid;

@@ -57,7 +57,8 @@ struct nbx_nlist {
                               // finish counter, [7] a list went stale between two build
                               // opportunities, [8..9] bits of the largest squared speed
                               // when the lists were made (a double)
-    size_t cap_bytes = 0;
+    // bytes allocated for the buffers above: kept while they are large enough
+    size_t nbr_bytes = 0, nnb_bytes = 0, count_bytes = 0, atoms_bytes = 0, xref_bytes = 0;
 };
 
 // What a captured step graph depends on; a mismatch forces a new capture.  Every device
@@ -123,7 +124,8 @@ struct nbx_ctx {
     bool every_chosen = false;  // for the current state
     double speed2 = 0.0;        // largest squared speed when its lists were made
     int64_t stale_replays = 0;  // chunks replayed because a list went stale (build_every -> 1)
-    // device state
+    // device state: one allocation (d_base) holds d_x .. d_pmap
+    char* d_base = nullptr;
     double* d_x = nullptr;    // positions (unwrapped), 3n
     double* d_v = nullptr;    // velocities, 3n
     double* d_a = nullptr;    // accelerations at d_x, 3n
@@ -138,6 +140,7 @@ struct nbx_ctx {
     double* d_water = nullptr;     // water: electrostatic and Lennard-Jones sums (6n)
     double* d_frames = nullptr;    // saved frames on their way to the host
     size_t frames_doubles = 0;
+    double* d_backup = nullptr;    // mixed path: the state at the start of a chunk
     double* d_ms = nullptr;
     double* d_qs = nullptr;
     double* d_mm = nullptr;   // magnetic moments (SoA 3n), when set
@@ -336,7 +339,21 @@ void ref64_rdf_hist(hipStream_t s, const double* frames_aos, int64_t nframes, in
 #define NBX_MAX_DEVICES 64
 int ref64_rdf_scratch(int device, unsigned long long** out);
 void ref64_zero_u64(hipStream_t s, unsigned long long* p, int64_t count);
-int64_t ref64_check_finite(hipStream_t s, const double* p, int64_t count, int* d_flag);
+// sets d_flag[0] when a or b (count values each) holds NaN or Inf
+void ref64_check_finite(hipStream_t s, const double* a, const double* b, int64_t count, int* d_flag);
+// p[k] = value of five arrays in one launch: dst[0..3] of n3 doubles, dst[4] of nscal
+void ref64_copy_state(hipStream_t s, const double* const* src, double* const* dst, int64_t n3,
+                      int64_t nscal);
+
+// x * 0 is 0 for finite x and NaN otherwise; eight running sums, no branch per value
+inline bool nbx_all_finite(const double* p, int64_t count) {
+    double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    int64_t i = 0;
+    for (; i + 8 <= count; i += 8)
+        for (int k = 0; k < 8; ++k) s[k] += p[i + k] * 0.0;
+    for (; i < count; ++i) s[0] += p[i] * 0.0;
+    return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])) == 0.0;
+}
 
 // ---- mixed path (nbx_mixed.cpp driving nbx_nonbonded.hip and nbx_gravity.hip) ----
 int mx_time_force(nbx_ctx* c, int iters, double* avg_ms, const char** name);

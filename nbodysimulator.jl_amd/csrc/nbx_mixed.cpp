@@ -112,23 +112,33 @@ bool make_plan(const nbx_ctx* c, mx_plan& p, std::string* why) {
 }
 
 void free_nl(nbx_nlist& nl) {
-    if (nl.d_nbr) (void)hipFree(nl.d_nbr);
-    if (nl.d_nnb) (void)hipFree(nl.d_nnb);
-    if (nl.d_cell_count) (void)hipFree(nl.d_cell_count);
-    if (nl.d_cell_atoms) (void)hipFree(nl.d_cell_atoms);
-    if (nl.d_xref) (void)hipFree(nl.d_xref);
-    if (nl.d_flags) (void)hipFree(nl.d_flags);
+    void* const own[] = {nl.d_nbr, nl.d_nnb, nl.d_cell_count, nl.d_cell_atoms, nl.d_xref, nl.d_flags};
+    for (void* p : own)
+        if (p) (void)hipFree(p);
     nl.d_nbr = nullptr;
     nl.d_nnb = nl.d_cell_count = nl.d_cell_atoms = nl.d_flags = nullptr;
     nl.d_xref = nullptr;
+    nl.nbr_bytes = nl.nnb_bytes = nl.count_bytes = nl.atoms_bytes = nl.xref_bytes = 0;
     nl.ready = false;
 }
 
 int round_up(int x, int m) { return ((x + m - 1) / m) * m; }
 
-int alloc_flags(nbx_ctx* c) {
-    NBX_HIP(c, hipMalloc((void**)&c->nl.d_flags, sizeof(int) * NBX_FLAGS));
-    NBX_HIP(c, hipMemsetAsync(c->nl.d_flags, 0, sizeof(int) * NBX_FLAGS, c->stream));
+int reset_flags(nbx_ctx* c) {
+    if (!c->nl.d_flags) NBX_HIP(c, hipMalloc((void**)&c->nl.d_flags, sizeof(int) * NBX_FLAGS));
+    mx_launch_fill_int(c->stream, c->nl.d_flags, NBX_FLAGS, 0);
+    return NBX_OK;
+}
+
+// a list buffer of at least `bytes`: the one it has, or a new one
+template <class T>
+int list_buffer(nbx_ctx* c, T** p, size_t* have, size_t bytes) {
+    if (*p && *have >= bytes) return NBX_OK;
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+    *have = 0;
+    NBX_HIP(c, hipMalloc((void**)p, bytes));
+    *have = bytes;
     return NBX_OK;
 }
 
@@ -156,8 +166,7 @@ int alloc_lists(nbx_ctx* c, const mx_plan& p, double grow) {
             nl.lanes = lanes_by_size(n, 4.0 / 3.0 * M_PI * r * r * r * (double)n / (L * L * L));
     }
     const int lanes = nl.lanes;
-    free_nl(nl);
-    nl.lanes = lanes;
+    nl.ready = false;
     // the list kernels index one list row of n * lanes slots in 32 bits
     if (n * (int64_t)std::max(lanes, 1) >= (int64_t)1 << 32)
         return nbx_fail(c, NBX_ERR_CAPACITY, "n x lanes per atom must stay below 2^32");
@@ -196,19 +205,21 @@ int alloc_lists(nbx_ctx* c, const mx_plan& p, double grow) {
         return nbx_fail(c, NBX_ERR_CAPACITY, "cell occupancy above 1024 atoms (box too dense)");
     const size_t ncells = (size_t)nc * nc * nc;
     nl.nbr_wide = n > 65536 ? 1 : 0;
-    NBX_HIP(c, hipMalloc(&nl.d_nbr, (nl.nbr_wide ? sizeof(int) : sizeof(uint16_t)) *
-                                        (size_t)nl.cap * (size_t)n));
-    NBX_HIP(c, hipMalloc((void**)&nl.d_nnb, sizeof(int) * (size_t)n));
-    NBX_HIP(c, hipMalloc((void**)&nl.d_cell_count, sizeof(int) * 3 * std::max<size_t>(ncells, 1)));
-    NBX_HIP(c, hipMalloc((void**)&nl.d_cell_atoms,
-                         sizeof(int) * 3 * std::max<size_t>(ncells * (size_t)nl.ccap, 1)));
-    NBX_HIP(c, hipMalloc((void**)&nl.d_xref, sizeof(double) * 3 * (size_t)n));
-    int rc = alloc_flags(c);
-    if (rc) return rc;
-    NBX_HIP(c, hipMemsetAsync(nl.d_nnb, 0, sizeof(int) * (size_t)n, c->stream));
-    NBX_HIP(c, hipMemsetAsync(nl.d_cell_count, 0, sizeof(int) * 3 * std::max<size_t>(ncells, 1),
-                              c->stream));
-    nl.cap_bytes = sizeof(int) * (size_t)nl.cap * (size_t)n;
+    // a new state of the same system finds its buffers, and the captured step graph that
+    // holds their addresses, as they are
+    int rc;
+    const size_t nb = (nl.nbr_wide ? sizeof(int) : sizeof(uint16_t)) * (size_t)nl.cap * (size_t)n;
+    if ((rc = list_buffer(c, &nl.d_nbr, &nl.nbr_bytes, nb)) ||
+        (rc = list_buffer(c, &nl.d_nnb, &nl.nnb_bytes, sizeof(int) * (size_t)n)) ||
+        (rc = list_buffer(c, &nl.d_cell_count, &nl.count_bytes, sizeof(int) * 3 * std::max<size_t>(ncells, 1))) ||
+        (rc = list_buffer(c, &nl.d_cell_atoms, &nl.atoms_bytes,
+                          sizeof(int) * 3 * std::max<size_t>(ncells * (size_t)nl.ccap, 1))) ||
+        (rc = list_buffer(c, &nl.d_xref, &nl.xref_bytes, sizeof(double) * 3 * (size_t)n)) ||
+        (rc = reset_flags(c)))
+        return rc;
+    mx_launch_fill_int(c->stream, nl.d_nnb, n, 0);
+    mx_launch_fill_int(c->stream, nl.d_cell_count, (int64_t)(3 * std::max<size_t>(ncells, 1)), 0);
+    NBX_HIP(c, hipGetLastError());
     nl.ready = true;
     return NBX_OK;
 }
@@ -402,11 +413,6 @@ void launch_build(nbx_ctx* c, const mx_plan& p, int par) {
                     bin_count(c), bin_atoms(c), clear);
 }
 
-struct backup4 {
-    double* p = nullptr;
-    ~backup4() { if (p) (void)hipFree(p); }
-};
-
 }  // namespace
 
 int mx_supported(nbx_ctx* c, std::string* why) {
@@ -435,8 +441,8 @@ static int prepare(nbx_ctx* c, mx_plan& p, double grow) {
         }
     }
     if (p.kind == PLAN_GRAVITY || !p.nb.mode_list) {
-        free_nl(c->nl);
-        int rc = alloc_flags(c);
+        if (c->nl.d_nbr) free_nl(c->nl);   // the lists of an earlier configuration
+        int rc = reset_flags(c);
         if (rc) return rc;
         c->nl.ready = true;
         return NBX_OK;
@@ -562,10 +568,11 @@ static bool sort_enabled(const nbx_ctx* c, const mx_plan& p) {
 }
 
 int mx_reset_order(nbx_ctx* c) {
-    mx_launch_iota(c->stream, c->d_perm, c->n);
-    mx_launch_iota(c->stream, c->d_iperm, c->n);
-    NBX_HIP(c, hipGetLastError());
-    NBX_HIP(c, hipStreamSynchronize(c->stream));
+    if (!c->perm_identity) {
+        mx_launch_iota(c->stream, c->d_perm, c->n);
+        mx_launch_iota(c->stream, c->d_iperm, c->n);
+        NBX_HIP(c, hipGetLastError());
+    }
     c->perm_identity = true;
     c->list_sorted = false;
     c->last_sort_step = -1;
@@ -673,7 +680,6 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
         ~order_guard() {
             if (!c || c->perm_identity) return;
             (void)permute_state(c, c->d_iperm);
-            (void)hipStreamSynchronize(c->stream);
             c->list_sorted = true;
         }
     } og;
@@ -695,8 +701,14 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
     hipStream_t s = c->stream;
     const int64_t n = c->n;
     const size_t n3 = 3 * (size_t)n;
-    backup4 bk;
-    NBX_HIP(c, hipMalloc((void**)&bk.p, sizeof(double) * (4 * n3 + NBX_SCAL_COUNT)));
+    // the chunk's start is kept for a replay where a list can overflow or go stale (the plans
+    // without lists never replay)
+    const bool lists = !all_pairs_tiled(p) && p.nb.mode_list;
+    if (lists && !c->d_backup)
+        NBX_HIP(c, hipMalloc((void**)&c->d_backup, sizeof(double) * (4 * n3 + NBX_SCAL_COUNT)));
+    double* const bk = c->d_backup;
+    double* const bkp[5] = {bk, bk + n3, bk + 2 * n3, bk + 3 * n3, bk + 4 * n3};
+    double* const live[5] = {c->d_x, c->d_v, c->d_a, c->d_vh, c->d_scal};
     const int64_t chunk_max = 500;
     while (c->kt_on && c->kt_ev.size() < 2 * (size_t)chunk_max) {
         hipEvent_t e = nullptr;
@@ -784,13 +796,7 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
             }
             chunk = std::min(chunk, S - t0 % S);
         }
-        // device-side backup of the state for an overflow replay
-        const double* src[4] = {c->d_x, c->d_v, c->d_a, c->d_vh};
-        for (int k = 0; k < 4; ++k)
-            NBX_HIP(c, hipMemcpyAsync(bk.p + k * n3, src[k], sizeof(double) * n3,
-                                      hipMemcpyDeviceToDevice, s));
-        NBX_HIP(c, hipMemcpyAsync(bk.p + 4 * n3, c->d_scal, sizeof(double) * NBX_SCAL_COUNT,
-                                  hipMemcpyDeviceToDevice, s));
+        if (lists) ref64_copy_state(s, live, bkp, (int64_t)n3, NBX_SCAL_COUNT);
         const int64_t step0 = c->steps_taken;
         for (int attempt = 0;; ++attempt) {
             mx_launch_step_advance(s, c->d_step, step0, 1);
@@ -832,8 +838,10 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
             if (chunk & 1)  // the state is in X[1]
                 NBX_HIP(c, hipMemcpyAsync(c->d_x, c->d_x2, sizeof(double) * n3,
                                           hipMemcpyDeviceToDevice, s));
-            int h[NBX_FLAGS];
-            if ((rc = read_flags(c, h))) return rc;
+            int h[NBX_FLAGS] = {0};
+            if (lists || c->kt_on) {   // kernel timing reads its events next
+                if ((rc = read_flags(c, h))) return rc;
+            }
             if (!h[1] && !h[7]) {
                 // the chunk stands: add its force-kernel times (the stream has drained)
                 for (size_t k = 0; k + 1 < c->kt_used; k += 2) {
@@ -850,12 +858,7 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
             c->kt_used = 0;   // replayed: its timings are dropped
             // overflow: restore and replay with larger lists; a list that went stale between
             // two build opportunities: restore and replay with an opportunity at every step
-            double* dst[4] = {c->d_x, c->d_v, c->d_a, c->d_vh};
-            for (int k = 0; k < 4; ++k)
-                NBX_HIP(c, hipMemcpyAsync(dst[k], bk.p + k * n3, sizeof(double) * n3,
-                                          hipMemcpyDeviceToDevice, s));
-            NBX_HIP(c, hipMemcpyAsync(c->d_scal, bk.p + 4 * n3, sizeof(double) * NBX_SCAL_COUNT,
-                                      hipMemcpyDeviceToDevice, s));
+            ref64_copy_state(s, bkp, live, (int64_t)n3, NBX_SCAL_COUNT);
             if (h[1]) {
                 if ((rc = grow_lists(c, p, grow))) return rc;
             } else {
@@ -874,10 +877,10 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
             const double* fx = c->d_x;
             const double* fv = c->d_v;
             if (sorting && !c->perm_identity) {
-                mx_launch_gather(s, c->d_x, bk.p, c->d_iperm, n, 3);
-                mx_launch_gather(s, c->d_v, bk.p + n3, c->d_iperm, n, 3);
-                fx = bk.p;
-                fv = bk.p + n3;
+                mx_launch_gather(s, c->d_x, bkp[0], c->d_iperm, n, 3);
+                mx_launch_gather(s, c->d_v, bkp[1], c->d_iperm, n, 3);
+                fx = bkp[0];
+                fv = bkp[1];
             }
             ref64_soa_to_aos(s, fx, c->d_tmp, n);
             NBX_HIP(c, hipMemcpyAsync(uf + *nframes * n3, c->d_tmp, sizeof(double) * n3,

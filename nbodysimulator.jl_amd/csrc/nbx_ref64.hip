@@ -1474,16 +1474,39 @@ void ref64_zero_u64(hipStream_t s, unsigned long long* p, int64_t count) {
     hipLaunchKernelGGL(k_fill_u64, dim3(nbx_blocks(count, 256)), dim3(256), 0, s, p, count);
 }
 
-__global__ void k_check_finite(const double* __restrict__ p, int64_t count, int* flag) {
+__global__ void k_check_finite(const double* __restrict__ a, const double* __restrict__ b,
+                               int64_t count, int* flag) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < count && !isfinite(p[t])) flag[0] = 1;
+    if (t < count && !(isfinite(a[t]) && isfinite(b[t]))) flag[0] = 1;
 }
 
-int64_t ref64_check_finite(hipStream_t s, const double* p, int64_t count, int* d_flag) {
-    if (count <= 0) return 0;
-    hipLaunchKernelGGL(k_check_finite, dim3(nbx_blocks(count, 256)), dim3(256), 0, s, p, count,
+void ref64_check_finite(hipStream_t s, const double* a, const double* b, int64_t count, int* d_flag) {
+    if (count <= 0) return;
+    hipLaunchKernelGGL(k_check_finite, dim3(nbx_blocks(count, 256)), dim3(256), 0, s, a, b, count,
                        d_flag);
-    return 0;
+}
+
+struct ref_copies {
+    const double* src[5];
+    double* dst[5];
+};
+
+__global__ void __launch_bounds__(256)
+k_copy_state(ref_copies c, int64_t n3, int64_t nscal) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n3) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) c.dst[k][t] = c.src[k][t];
+    }
+    if (t < nscal) c.dst[4][t] = c.src[4][t];
+}
+
+void ref64_copy_state(hipStream_t s, const double* const* src, double* const* dst, int64_t n3,
+                      int64_t nscal) {
+    ref_copies c{};
+    for (int k = 0; k < 5; ++k) { c.src[k] = src[k]; c.dst[k] = dst[k]; }
+    hipLaunchKernelGGL(k_copy_state, dim3(nbx_blocks(std::max(n3, nscal), 256)), dim3(256), 0, s, c,
+                       n3, nscal);
 }
 
 // ---------------------------------------------------------------------------

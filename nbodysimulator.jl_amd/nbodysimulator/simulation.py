@@ -230,23 +230,23 @@ def run_simulation(s: NBodySimulation, alg=None, *, dt: float = None,
     step = ctx.em_run if isinstance(alg, EM) else ctx.vv_run
     save = True if save_everystep is None else bool(save_everystep)
     ts = [t1]
-    us = [u0.copy()]
-    vs = [v0.copy()]
     if save:
-        if nsteps:
-            uf, vf = step(dt, nsteps, rng_seed, save_every=1)
-            us.extend(uf[1:]); vs.extend(vf[1:])
+        us, vs = u0[None].copy(), v0[None].copy()
+        if nsteps:   # frame 0 is the initial state
+            us, vs = step(dt, nsteps, rng_seed, save_every=1)
             ts.extend(t1 + dt * np.arange(1, nsteps + 1))
         if last:
             uf, vf = step(last, 1, rng_seed, save_every=1)
-            us.append(uf[1]); vs.append(vf[1]); ts.append(t2)
+            us, vs = np.concatenate([us, uf[1:]]), np.concatenate([vs, vf[1:]])
+            ts.append(t2)
     else:
         if nsteps:
             step(dt, nsteps, rng_seed)
         if last:
             step(last, 1, rng_seed)
         u, v = ctx.get_state()
-        us.append(u); vs.append(v); ts.append(t2)
+        us, vs = [u0.copy(), u], [v0.copy(), v]
+        ts.append(t2)
     steps = nsteps + (1 if last else 0)
     sol = Solution(np.asarray(ts), np.asarray(us), np.asarray(vs), _Stats(steps))
     return SimulationResult(sol, s, ctx)
