@@ -17,7 +17,10 @@
 // belongs to the drift of the step after the state when a run has ended)
 enum { NBX_SCAL_T = 0, NBX_SCAL_ZETA = 10, NBX_SCAL_XI = 11, NBX_SCAL_XI_SCRATCH = 15,
        NBX_SCAL_ZETA_PREV = 16, NBX_SCAL_XI_PREV = 17, NBX_SCAL_COUNT = 32 };
-enum { NBX_BINS_STEP = 0, NBX_BINS_FIXED = 1, NBX_BINS_BUILD = 2, NBX_FLAG_BINSET = 5, NBX_FLAG_SPEED = 8, NBX_FLAGS = 16 };
+enum { NBX_BINS_STEP = 0, NBX_BINS_FIXED = 1, NBX_BINS_BUILD = 2, NBX_FLAG_BINSET = 5, NBX_FLAG_SPEED = 8, NBX_FLAGS = 16,
+       // the flags' allocation: their line, then a line per group of the list build's blocks
+       NBX_FLAGS_LINE = 32, NBX_BUILD_GROUPS = 32,
+       NBX_FLAGS_INTS = NBX_FLAGS_LINE * (1 + NBX_BUILD_GROUPS) };
 
 enum { NBX_TERM_LJ = 1, NBX_TERM_ELEC = 2, NBX_TERM_GRAV = 3, NBX_TERM_RF = 4, NBX_TERM_MAG = 5 };
 

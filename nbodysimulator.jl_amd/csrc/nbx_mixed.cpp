@@ -125,8 +125,8 @@ void free_nl(nbx_nlist& nl) {
 int round_up(int x, int m) { return ((x + m - 1) / m) * m; }
 
 int reset_flags(nbx_ctx* c) {
-    if (!c->nl.d_flags) NBX_HIP(c, hipMalloc((void**)&c->nl.d_flags, sizeof(int) * NBX_FLAGS));
-    mx_launch_fill_int(c->stream, c->nl.d_flags, NBX_FLAGS, 0);
+    if (!c->nl.d_flags) NBX_HIP(c, hipMalloc((void**)&c->nl.d_flags, sizeof(int) * NBX_FLAGS_INTS));
+    mx_launch_fill_int(c->stream, c->nl.d_flags, NBX_FLAGS_INTS, 0);
     return NBX_OK;
 }
 

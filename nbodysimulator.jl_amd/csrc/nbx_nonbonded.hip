@@ -619,34 +619,41 @@ void mx_launch_gather(hipStream_t s, const double* src, double* dst, const int* 
 }
 
 // ---------------------------------------------------------------------------
-// Verlet list build (gated by *req): one block of 4 wavefronts per cell.
-//   1. the cell's own atoms (<= 256 per pass) are staged in LDS (rotate: and binned by
-//      their current positions into the next bin set);
+// Verlet list build (gated by *req): one block per cell.
+//   1. the cell's own atoms (<= 128 per pass) are staged in LDS;
 //   2. the atoms of the stencil cells -- the 27 neighbour cells, or with rotate the 125
-//      cells within two half-size cells (fixed order; in batches of <= 1024) -- are
-//      staged in LDS -- indices, then FP32 positions (with per-step bins: at the periodic
-//      image of their cell next to the home cell), every load independent -- and sorted
+//      cells within two half-size cells (fixed order; in batches of THREADS x QN) -- are
+//      staged in LDS -- indices, then positions, every load independent -- and sorted
 //      by index within each cell, so every list comes out in a reproducible order (cell
-//      order, then index order);
+//      order, then index order).  Positions are FP32 differences of the fixed-point box
+//      fractions from the home cell's centre: the integer wrap-around places every
+//      candidate at its image next to the cell, so a test is three FP32 subtractions.
+//      With three cells per side that image need not be the nearest to each own atom:
+//      the integers themselves are staged and subtracted (WRAP);
 //   3. wave w takes own atoms 8 at a time; its 64 lanes read 64 candidates at a time and
-//      test each against the 8 (per-step bins: a plain FP32 difference, the images being
-//      the near ones; other bins: the difference of the fixed-point box fractions, whose
-//      integer wrap-around is the minimum image), appending every atom's hits in
-//      candidate order (ballot + prefix count).
+//      test each against the 8, appending every atom's hits in candidate order (ballot +
+//      prefix count);
+//   4. rotate: the own atoms are binned by their current positions into the next bin set.
 //   The squared list radius carries a 1e-4 relative margin so that the FP32 test never
 //   drops a pair that the FP64 distance puts inside the list radius.
+// All blocks of a launch run at once and in step, so the chain of each block's loads adds to
+// its tests, which bound it (VALU: about 70 cycles a wavefront test).  Us per build: 32,000
+// Lennard-Jones atoms (1,331 cells) 38 -> 30, of which 4 by six blocks per CU instead of five
+// (80 registers, 21 KB) -- with five, 51 blocks ran in a round of their own; 4,096 water
+// molecules (512 cells of 24 atoms, 3,000 candidates each) 72 -> 50 with eight waves a block
+// (two batches instead of three), FP32 differences and 32-bit list addresses.  Blocks mapped
+// to the XCDs by runs of cells changed nothing for Lennard-Jones and cost water 10 %.
 // Per-step bins: every block also clears its cell in the other bin set (used by the next
 // step).  Rotate (bins made by the builds): the build reads set b % 3 (the bins of the
 // previous build; every atom has since moved at most 3/4 skin, which the drift enforces,
 // and two half cells reach list radius + 1.5 skin), fills set (b + 1) % 3 (cleared by the
 // previous build) and clears set (b + 2) % 3; the last block to finish (device-scope
-// counter) advances b, which every block read at its start.
+// counters) advances b, which every block read at its start.
 // ---------------------------------------------------------------------------
 
-#define BUILD_THREADS 256
-#define BUILD_SLOTS 1024
-#define BUILD_OWN 256
+#define BUILD_OWN 128
 #define BUILD_OWN_BATCH 8
+#define BUILD_SMALL_CELL 768   // most atoms of a cell in the small layout (3 x 256 slots)
 
 __device__ __forceinline__ int build_segment(const int* seg, int nseg, int t) {
     int lo = 0, hi = nseg - 1;   // last s with seg[s] <= t
@@ -658,31 +665,39 @@ __device__ __forceinline__ int build_segment(const int* seg, int nseg, int t) {
     return lo;
 }
 
-#define BUILD_STENCIL 125
+// Counts this block as finished with the bins; true for the last block of the grid.  Blocks
+// count in groups, each on a cache line of its own, and the last of a group in the grid's
+// counter: one counter for all 1,331 blocks of 32,000 atoms took their additions one after
+// the other, about 10 ns each
+__device__ __forceinline__ bool build_finished(int* flags) {
+    const unsigned k = blockIdx.x % NBX_BUILD_GROUPS, blocks = gridDim.x;
+    const unsigned members = (blocks - k + NBX_BUILD_GROUPS - 1) / NBX_BUILD_GROUPS;
+    unsigned* const group = reinterpret_cast<unsigned*>(flags) + NBX_FLAGS_LINE * (1 + k);
+    if (atomicAdd(group, 1u) != members - 1) return false;
+    *group = 0;
+    const unsigned groups = blocks < NBX_BUILD_GROUPS ? blocks : NBX_BUILD_GROUPS;
+    return atomicAdd(reinterpret_cast<unsigned*>(flags) + NBX_FLAG_BINSET + 1, 1u) == groups - 1;
+}
 
-template <bool WATER, bool SHIFT>
-__global__ void __launch_bounds__(BUILD_THREADS)
+template <bool WATER, bool WRAP, int THREADS, int QN>
+__global__ void __launch_bounds__(THREADS, THREADS == 256 ? 6 : 3)
 k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int n, int nc,
-              double Ld, int* __restrict__ bin_count, int* __restrict__ bin_atoms,
-              int ccap, double inv_cs, float rlist2f, int G, int cap,
+              int* __restrict__ bin_count, int* __restrict__ bin_atoms,
+              int ccap, double inv_cs, float r2test, int G, int cap, int near,
               void* __restrict__ nbr, int nbr_wide, int* __restrict__ nnb,
               double* __restrict__ xref, int* __restrict__ flags, int* __restrict__ req,
               int clear_bins, int rotate, int parts) {
+    constexpr int BUILD_SLOTS = THREADS * QN, BUILD_STENCIL = 125;
     __shared__ __attribute__((aligned(16))) int skey[BUILD_SLOTS];
-    __shared__ float4 spos[BUILD_SLOTS];
+    __shared__ float4 spos[BUILD_SLOTS];      // position, and the index's bits
     __shared__ int seg[BUILD_STENCIL + 1], segcell[BUILD_STENCIL];
     __shared__ int ncnt[BUILD_STENCIL], ncell[BUILD_STENCIL];
-    __shared__ float4 nshift[BUILD_STENCIL], segshift[BUILD_STENCIL];
     __shared__ int npre[BUILD_STENCIL + 1];   // exclusive prefix sums of ncnt
     __shared__ int okey[BUILD_OWN], ocnt[BUILD_OWN];
     __shared__ float4 opos[BUILD_OWN];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    // the squared list radius in the units of the test: length, or L / 2^32 for the
-    // fixed-point positions
-    const float r2test = SHIFT ? rlist2f
-                               : (float)((double)rlist2f * (4294967296.0 / Ld) * (4294967296.0 / Ld));
     // `parts` blocks share a home cell, each taking a contiguous slice of its atoms (more
     // blocks in flight when the cells are few and large, as for water)
     const int cid = blockIdx.x / parts, part = blockIdx.x % parts;
@@ -707,15 +722,12 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
         const int m2 = count[nid];
         ncell[tid] = nid;
         ncnt[tid] = m2 < ccap ? m2 : ccap;
-        // the periodic image of the stencil cell next to the home cell: -1, 0 or +1 box
-        // sides per axis
-        const auto img = [nc](int c) { return c < 0 ? -1.0f : (c >= nc ? 1.0f : 0.0f); };
-        nshift[tid] = make_float4(img(cx + ox), img(cy + oy), img(cz + oz), 0.0f);
     }
     int m = count[cid];
     m = m < ccap ? m : ccap;
     const int per = (m + parts - 1) / parts;
     const int hb = part * per, he = (hb + per) < m ? (hb + per) : m;
+    bool all_read = false;
     if (hb < he) {   // uniform over the block
     __syncthreads();
     if (wave == 0) {   // prefix sums of the stencil counts (nst <= 128: two per lane)
@@ -731,30 +743,31 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
         if (2 * lane + 1 <= nst) npre[2 * lane + 1] = ex + a0;
     }
     __syncthreads();
+    // box fractions are read as FP32 differences from the home cell's centre, whose integer
+    // wrap-around takes every candidate at its image next to the cell
+    const auto centre = [nc](int c) { return (uint32_t)((c + 0.5) / nc * 4294967296.0); };
+    const uint32_t hx = centre(cx), hy = centre(cy), hz = centre(cz);
+    const uint4* const posq = mx_posq(pos, n);
+    const auto place = [&](const uint4 q, int i) {
+        if constexpr (WRAP)
+            return make_float4(__uint_as_float(q.x), __uint_as_float(q.y), __uint_as_float(q.z),
+                               __int_as_float(i));
+        else
+            return make_float4((float)(int)(q.x - hx), (float)(int)(q.y - hy),
+                               (float)(int)(q.z - hz), __int_as_float(i));
+    };
     // G is a power of two: slot r of atom i is at (r >> lgG) n G + i G + r % G
     const uint32_t stride32 = (uint32_t)n * (uint32_t)G;
     const int lgG = __builtin_ctz((unsigned)G);
     for (int own0 = hb; own0 < he; own0 += BUILD_OWN) {
         const int mo = (he - own0) < BUILD_OWN ? (he - own0) : BUILD_OWN;
-        for (int t = tid; t < mo; t += BUILD_THREADS) {
-            const int i = atoms[(size_t)cid * ccap + own0 + t];
-            const double4 p = pos[i];
-            okey[t] = i;
-            if (SHIFT) {
-                opos[t] = make_float4((float)p.x, (float)p.y, (float)p.z, 0.0f);
-            } else {   // the fixed-point box fractions (their bits), minimum image by integers
-                const uint4 qv = mx_posq(pos, n)[i];
-                opos[t] = make_float4(__uint_as_float(qv.x), __uint_as_float(qv.y),
-                                      __uint_as_float(qv.z), 0.0f);
-            }
-            ocnt[t] = 0;
-            if (rotate) {   // the bin of the atom's current position, for the next build
-                const int c2 = (mx_cell_coord(p.z, inv_cs, nc) * nc +
-                                mx_cell_coord(p.y, inv_cs, nc)) * nc + mx_cell_coord(p.x, inv_cs, nc);
-                const int slot = atomicAdd(&next_count[c2], 1);
-                if (slot < ccap) next_atoms[(size_t)c2 * ccap + slot] = i;
-                else flags[1] = 1;
-            }
+        int own = 0;
+        if (tid < mo) {
+            own = atoms[(size_t)cid * ccap + own0 + tid];
+            okey[tid] = own;
+            const uint4 q = posq[own];
+            opos[tid] = place(q, own);
+            ocnt[tid] = 0;
         }
         int nb = 0;
         while (nb < nst) {
@@ -771,26 +784,18 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
             if (tid < nseg) {
                 seg[tid] = npre[nb + tid] - npre[nb];
                 segcell[tid] = ncell[nb + tid];
-                segshift[tid] = nshift[nb + tid];
             }
             if (tid == 0) seg[nseg] = M;
             nb = lo;
             __syncthreads();
-            // candidate t = tid + q BUILD_THREADS: its stencil cell (segment), index and
-            // position; the position gathers are issued here and stay in flight through
-            // the barrier and the rank counts below
-            constexpr int QN = BUILD_SLOTS / BUILD_THREADS;
+            // candidate t = tid + q THREADS: its stencil cell (segment), index and position;
+            // the position gathers are issued here and stay in flight through the barrier
+            // and the rank counts below
             int ck[QN], cs[QN], cr[QN];
-            // per-step bins: FP64 positions shifted to the image next to the home cell;
-            // other bins: the 16-byte fixed-point positions
-            using gather_t = typename std::conditional<SHIFT, double4, uint4>::type;
-            const gather_t* gsrc;
-            if constexpr (SHIFT) gsrc = pos;
-            else gsrc = mx_posq(pos, n);
-            gather_t pg[QN];
+            uint4 pg[QN];
 #pragma unroll
             for (int q = 0; q < QN; ++q) {
-                const int t = tid + q * BUILD_THREADS;
+                const int t = tid + q * THREADS;
                 ck[q] = -1;
                 cs[q] = 0;
                 if (t < M) {
@@ -802,7 +807,7 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
             }
 #pragma unroll
             for (int q = 0; q < QN; ++q)
-                if (ck[q] >= 0) pg[q] = gsrc[ck[q]];
+                if (ck[q] >= 0) pg[q] = posq[ck[q]];
             __syncthreads();
             // rank by index within the candidate's cell (the cell's indices read four at
             // a time where aligned), so that candidates are stored in list order
@@ -821,38 +826,19 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
                     cr[q] = b + r;
                 }
             }
-            // positions at the candidate's image next to the home cell (FP64 sum, one FP32
-            // rounding), or the fixed-point fractions' bits
-            float4 cp[QN];
 #pragma unroll
-            for (int q = 0; q < QN; ++q) {
-                if (ck[q] >= 0) {
-                    if constexpr (SHIFT) {
-                        const float4 sh = segshift[cs[q]];
-                        cp[q] = make_float4((float)(pg[q].x + (double)sh.x * Ld),
-                                            (float)(pg[q].y + (double)sh.y * Ld),
-                                            (float)(pg[q].z + (double)sh.z * Ld), 0.0f);
-                    } else {
-                        cp[q] = make_float4(__uint_as_float(pg[q].x), __uint_as_float(pg[q].y),
-                                            __uint_as_float(pg[q].z), 0.0f);
-                    }
-                }
-            }
+            for (int q = 0; q < QN; ++q)
+                if (ck[q] >= 0) spos[cr[q]] = place(pg[q], ck[q]);
             __syncthreads();
-#pragma unroll
-            for (int q = 0; q < QN; ++q) {
-                if (ck[q] >= 0) {
-                    skey[cr[q]] = ck[q];
-                    spos[cr[q]] = cp[q];
-                }
-            }
-            __syncthreads();
+            // nothing of the bins is read any more: the block counts as finished, and the
+            // counter's answer arrives during the tests
+            if (tid == 0 && nb >= nst && own0 + BUILD_OWN >= he) all_read = build_finished(flags);
             // wave w tests the candidates against `per` of its own atoms at a time (own
-            // atoms per*w .. per*w+per-1, then per*(w+4) ..; per = ceil(own / 4) up to 8, so
+            // atoms per*w .. per*w+per-1, then the next; per = ceil(own / waves) up to 8, so
             // every wave has work): each candidate is read from LDS once per `per` tests,
             // and those tests are independent
-            const int per = min(BUILD_OWN_BATCH, (mo + BUILD_THREADS / 64 - 1) / (BUILD_THREADS / 64));
-            for (int o0 = wave * per; o0 < mo; o0 += BUILD_THREADS / 64 * per) {
+            const int per = min(BUILD_OWN_BATCH, (mo + THREADS / 64 - 1) / (THREADS / 64));
+            for (int o0 = wave * per; o0 < mo; o0 += THREADS / 64 * per) {
                 // the batch's own atoms are the same for the whole wave: their index and list
                 // count are held in scalar registers
                 const int no = __builtin_amdgcn_readfirstlane(min(per, mo - o0));
@@ -869,14 +855,14 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
                 for (int tb = 0; tb < M; tb += 64) {
                     const int t = tb + lane;
                     const bool v = t < M;
-                    const int j = skey[v ? t : 0];
                     const float4 pj = spos[v ? t : 0];
+                    const int j = __float_as_int(pj.w);
                     const int jm = WATER ? j / 3 : 0;
 #pragma unroll
                     for (int k = 0; k < BUILD_OWN_BATCH; ++k) {
                         if (k >= no) break;   // scalar
                         float dx, dy, dz;
-                        if constexpr (SHIFT) {
+                        if constexpr (!WRAP) {
                             dx = pi[k].x - pj.x;
                             dy = pi[k].y - pj.y;
                             dz = pi[k].z - pj.z;
@@ -887,19 +873,25 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
                         }
                         // every term evaluated (no short-circuit branches)
                         const bool hit = v & (dx * dx + dy * dy + dz * dz < r2test) &
-                                         (j != ii[k]) & !(WATER && jm == im[k]);
+                                         (WATER ? jm != im[k] : j != ii[k]);
                         const unsigned long long mask = __ballot(hit);
                         if (mask == 0ull) continue;   // scalar
                         // slot r of a hit: the hits before this lane in the wave, after
                         // the atom's earlier hits (slots past the capacity are counted, not
                         // stored: the count flags the overflow)
                         const unsigned lo = (unsigned)mask, hi = (unsigned)(mask >> 32);
-                        const int r = cc[k] + (int)__builtin_amdgcn_mbcnt_hi(
-                                                  hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
-                        if (hit & (r < cap))
-                            mx_nbr_store(nbr, nbr_wide,
-                                         (uint64_t)(uint32_t)(r >> lgG) * stride32 +
-                                             (uint32_t)(ii[k] * G + (r & (G - 1))), j);
+                        const int r = (int)__builtin_amdgcn_mbcnt_hi(
+                            hi, __builtin_amdgcn_mbcnt_lo(lo, (unsigned)cc[k]));
+                        if (hit & (r < cap)) {
+                            const uint32_t row = (uint32_t)(r >> lgG), col = (uint32_t)(r & (G - 1));
+                            const uint32_t first = (uint32_t)(ii[k] * G);   // scalar
+                            if (near) {   // 16-bit entries, 32-bit offsets
+                                const uint32_t at = (__umul24(row, stride32) + first + col) * 2u;
+                                *reinterpret_cast<uint16_t*>(static_cast<char*>(nbr) + at) = (uint16_t)j;
+                            } else {
+                                mx_nbr_store(nbr, nbr_wide, (uint64_t)row * stride32 + first + col, j);
+                            }
+                        }
                         cc[k] += __popcll(mask);
                     }
                 }
@@ -911,14 +903,22 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
             }
             __syncthreads();
         }
-        for (int t = tid; t < mo; t += BUILD_THREADS) {
-            const int i = okey[t];
-            int c = ocnt[t];
+        if (tid < mo) {
+            int c = ocnt[tid];
             if (c > cap) { flags[1] = 1; c = cap; }
-            nnb[i] = c;
-            xref[i] = x[i];
-            xref[n + i] = x[n + i];
-            xref[2 * n + i] = x[2 * n + i];
+            nnb[own] = c;
+        }
+        if (tid < mo)
+            for (int k = 0; k < 3; ++k) xref[(size_t)k * n + own] = x[(size_t)k * n + own];
+        const int rt = THREADS - 1 - tid;   // other waves than those above
+        if (rotate && rt < mo) {   // the bin of the atom's current position, for the next build
+            const int i = okey[rt];
+            const double4 p = pos[i];
+            const int c2 = (mx_cell_coord(p.z, inv_cs, nc) * nc +
+                            mx_cell_coord(p.y, inv_cs, nc)) * nc + mx_cell_coord(p.x, inv_cs, nc);
+            const int slot = atomicAdd(&next_count[c2], 1);
+            if (slot < ccap) next_atoms[(size_t)c2 * ccap + slot] = i;
+            else flags[1] = 1;
         }
         __syncthreads();
     }
@@ -931,11 +931,11 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
     // here would write back the L2 of the block's XCD once per cell
     __shared__ int last;
     __syncthreads();
-    if (tid == 0) last = atomicAdd(reinterpret_cast<unsigned*>(&state[1]), 1u) == gridDim.x - 1;
+    if (tid == 0) last = hb < he ? all_read : build_finished(flags);
     __syncthreads();
     if (!last) return;
     if (clear_bins)
-        for (int c = tid; c < ncells; c += BUILD_THREADS) bin_count[c] = 0;
+        for (int c = tid; c < ncells; c += THREADS) bin_count[c] = 0;
     if (tid == 0) {
         state[1] = 0;
         if (rotate) state[0] = (bset + 1) % 3;
@@ -1018,22 +1018,24 @@ static void launch_build_t(hipStream_t s, const nbx_ctx* c, const void* pos, con
         int parts = (512 + ncells - 1) / ncells;
         parts = parts < 1 ? 1 : (parts > 8 ? 8 : parts);
         const dim3 grid(ncells * parts);
-        // per-step bins hold every atom in the cell of its current position, so a stencil
-        // cell's atoms are shifted once to their image next to the home cell; bins made
-        // earlier (set-up bins of 3 cells per side, bins of the previous build) need the
-        // minimum image per candidate
-        if (nl.bin_mode == NBX_BINS_STEP)
-            hipLaunchKernelGGL((k_build_cells<WATER, true>), grid, dim3(BUILD_THREADS), 0, s,
-                               (const double4*)pos, x, n, nc, L, bin_count,
-                               bin_atoms, nl.ccap, (double)nc / L, r2f, nl.lanes, nl.cap, nbr,
-                               nl.nbr_wide, nl.d_nnb, nl.d_xref, nl.d_flags, req, clear_bins,
-                               rotate, parts);
+        // The small layout keeps six blocks on a CU and takes a cell's stencil in one batch
+        // where 27 cells hold up to 768 atoms; the half-size cells' stencils (about 3,000
+        // atoms for water) and denser cells take eight waves and 2,048 slots.
+        // the squared list radius in the units of the tests, L / 2^32
+        const float r2t = (float)((double)r2f * (4294967296.0 / L) * (4294967296.0 / L));
+        // 32-bit addresses of the entries: rows x (n x lanes) by a 24-bit product
+        const int near = !nl.nbr_wide && c->n * (int64_t)nl.lanes < (int64_t)1 << 24 &&
+                         c->n * (int64_t)nl.cap < (int64_t)1 << 31;
+#define BUILD_ARGS(threads) grid, dim3(threads), 0, s, (const double4*)pos, x, n, nc, bin_count, \
+                   bin_atoms, nl.ccap, (double)nc / L, r2t, nl.lanes, nl.cap, near, nbr, \
+                   nl.nbr_wide, nl.d_nnb, nl.d_xref, nl.d_flags, req, clear_bins, rotate, parts
+        if (nc == 3)
+            hipLaunchKernelGGL((k_build_cells<WATER, true, 512, 4>), BUILD_ARGS(512));
+        else if (rotate || nl.ccap > BUILD_SMALL_CELL)
+            hipLaunchKernelGGL((k_build_cells<WATER, false, 512, 4>), BUILD_ARGS(512));
         else
-            hipLaunchKernelGGL((k_build_cells<WATER, false>), grid, dim3(BUILD_THREADS), 0, s,
-                               (const double4*)pos, x, n, nc, L, bin_count,
-                               bin_atoms, nl.ccap, (double)nc / L, r2f, nl.lanes, nl.cap, nbr,
-                               nl.nbr_wide, nl.d_nnb, nl.d_xref, nl.d_flags, req, clear_bins,
-                               rotate, parts);
+            hipLaunchKernelGGL((k_build_cells<WATER, false, 256, 3>), BUILD_ARGS(256));
+#undef BUILD_ARGS
     } else {
         hipLaunchKernelGGL((k_build_allpairs<WATER>), dim3(nbx_blocks(n, 128)), dim3(128), 0,
                            s, (const double4*)pos, x, n, L, 1.0 / L, r2, nl.lanes, nl.cap, nbr,
