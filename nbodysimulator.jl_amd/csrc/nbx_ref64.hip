@@ -1345,6 +1345,20 @@ void ref64_bonded_pe(hipStream_t s, const double* x, int64_t n, double rOH, doub
 // Above RDF_LDS_BINS bins (64 KiB of LDS with the staged atoms) the counts go to memory
 // directly.
 #define RDF_LDS_BINS 8000
+
+// box fractions in units of 2^-32; false where the coordinate is more than 1,024 boxes away (or
+// no number), too far for the bound on the difference to the FP64 distance
+__device__ __forceinline__ bool rdf_fixed(double x, double y, double z, double invL, uint32_t* q) {
+    const double t[3] = {x * invL, y * invL, z * invL};
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        ok = ok && fabs(t[k]) < 1024.0;
+        q[k] = ok ? (uint32_t)(uint64_t)((t[k] - floor(t[k])) * 4294967296.0) : 0u;
+    }
+    return ok;
+}
+
 template <bool LDS>
 __global__ void __launch_bounds__(1024)
 k_ref_rdf(const double* __restrict__ f, int64_t n, int jstride, int64_t nj, int64_t nframes,
@@ -1368,7 +1382,9 @@ k_ref_rdf(const double* __restrict__ f, int64_t n, int jstride, int64_t nj, int6
         }
         __syncthreads();
     };
-    const double radius = 0.5 * L, lim = (0.5 * L) * (0.5 * L);
+    const double radius = 0.5 * L, lim = (0.5 * L) * (0.5 * L), invL = 1.0 / L;
+    const float per_bin = (float)((double)maxbin * 0x1p-32), half = 0.5f * (float)maxbin;
+    const float open_abs = (float)maxbin * 2e-9f;
     const int64_t T = (nj + 63) >> 6, per_frame = T * (T + 1) / 2, items = per_frame * nframes;
     const int64_t stride = (int64_t)gridDim.x * waves;
     // 2^19 tiles of 2^12 pairs at most between two flushes: a counter stays below 2^32
@@ -1396,7 +1412,7 @@ k_ref_rdf(const double* __restrict__ f, int64_t n, int jstride, int64_t nj, int6
                 sb[4 * lane] = p[0]; sb[4 * lane + 1] = p[1]; sb[4 * lane + 2] = p[2];
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            for (int k = 0; k < nb; ++k) {
+            const auto exact = [&](int k) {   // atom k of the staged against the lane's
                 const double rx = nbx_wrap_cubic(xi - sb[4 * k], L, radius);
                 const double ry = nbx_wrap_cubic(yi - sb[4 * k + 1], L, radius);
                 const double rz = nbx_wrap_cubic(zi - sb[4 * k + 2], L, radius);
@@ -1408,6 +1424,30 @@ k_ref_rdf(const double* __restrict__ f, int64_t n, int jstride, int64_t nj, int6
                         if (LDS) atomicAdd(&cnt[(unsigned)fb], 1u);
                         else atomicAdd(&hist[(int64_t)fb], 2ull);
                     }
+                }
+            };
+            uint32_t qi[3] = {0u, 0u, 0u}, qj[3] = {0u, 0u, 0u};
+            bool ok = true;
+            if (LDS) {
+                if (a < nj) ok = rdf_fixed(xi, yi, zi, invL, qi);
+                if (lane < nb)
+                    ok = rdf_fixed(sb[4 * lane], sb[4 * lane + 1], sb[4 * lane + 2], invL, qj) && ok;
+            }
+            if (!LDS || __any(!ok)) {
+                for (int k = 0; k < nb; ++k) exact(k);
+            } else {
+                const bool diagonal = I == J;   // off it every lane holds an atom, a < b
+                for (int k = 0; k < nb; ++k) {
+                    const float dx = (float)(int)(qi[0] - __builtin_amdgcn_readlane(qj[0], k));
+                    const float dy = (float)(int)(qi[1] - __builtin_amdgcn_readlane(qj[1], k));
+                    const float dz = (float)(int)(qi[2] - __builtin_amdgcn_readlane(qj[2], k));
+                    const float g = __builtin_amdgcn_sqrtf(fmaf(dz, dz, fmaf(dy, dy, dx * dx))) * per_bin;
+                    const float open = fmaf(g, 6e-7f, open_abs);
+                    const bool pair = !diagonal || k > lane;
+                    if (__any(pair && (fabsf(g - rintf(g)) <= open || fabsf(g - half) <= open)))
+                        exact(k);
+                    else if (pair && g < half && g > 1.0f)
+                        atomicAdd(&cnt[(unsigned)ceilf(g)], 1u);
                 }
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

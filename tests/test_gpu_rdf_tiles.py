@@ -36,3 +36,22 @@ def test_water_counts_oxygens(nbx):
     ctx.set_boundary(_lib.BC_CUBIC, [L, 0, 0, 0, 0, 0])
     gr = ctx.rdf(frames, 200)[1]
     assert np.array_equal(gr, O.rdf(frames, L, indxs=np.arange(0, n, 3), maxbin=200)[1])
+
+
+@pytest.mark.parametrize("L,maxbin", [(8.0, 64), (8.0, 1000), (7.3, 73), (7.3, 4001)])
+def test_distances_on_bin_edges_and_far_images(nbx, L, maxbin):
+    # distances that are whole multiples of a bin or of half the box, whose bin only the FP64
+    # square root and division decide, and atoms too far away for the FP32 estimate
+    print(f"[case] rdf edges L={L} maxbin={maxbin}", flush=True)
+    rng = np.random.default_rng(maxbin)
+    n = 300
+    grid = rng.integers(0, 16, (n, 3)) * (L / 16)            # on multiples of L / 16
+    line = np.zeros((n, 3))
+    line[:, 0] = rng.integers(0, maxbin, n) * (L / maxbin)   # on bin edges along x
+    far = rng.uniform(0, L, (n, 3))
+    far[::7] += L * 2000
+    far[1::7] -= L * 1023.5
+    frames = np.stack([grid, line, far])
+    ctx = _lib.Context(n, _lib.SYS_POTENTIAL, np.ones(n))
+    ctx.set_boundary(_lib.BC_CUBIC, [L, 0, 0, 0, 0, 0])
+    assert np.array_equal(ctx.rdf(frames, maxbin)[1], O.rdf(frames, L, maxbin=maxbin)[1])
