@@ -1123,22 +1123,42 @@ void ref64_kinetic(hipStream_t s, const double* v, const double* ms, int64_t n,
     hipLaunchKernelGGL(k_seq_mv2, dim3(1), dim3(256), 0, s, v, ms, n, 1, 0, 0.0, d_out);
 }
 
+// box fractions in units of 2^-32; false where the coordinate is more than 1,024 boxes away (or
+// no number), too far for the bound on the difference to the FP64 distance
+__device__ __forceinline__ bool box_fixed(double x, double y, double z, double invL, uint32_t* q) {
+    const double t[3] = {x * invL, y * invL, z * invL};
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        ok = ok && fabs(t[k]) < 1024.0;
+        q[k] = ok ? (uint32_t)(uint64_t)((t[k] - floor(t[k])) * 4294967296.0) : 0u;
+    }
+    return ok;
+}
+
 // Pair energies of the pairs i < j of nj atoms: a wavefront takes 64 x 64 tiles of the upper
 // triangle (64 atoms i in its lanes, 64 atoms j from LDS), adds per lane in FP64, and the
 // lanes, wavefronts and blocks are added in a fixed order (k_ref_pe_sum).  Bound by FP64
 // VALU work; one thread per atom i with the triangle's long and short rows took 5,300 us for
-// 10,976 Lennard-Jones atoms, this takes 108.
+// 10,976 Lennard-Jones atoms, this took 108 with every pair in FP64.
 //   LJ (:293-319): 4 (s12 - s6), a pair beyond the cutoff at the cutoff's value; those are
-//   counted and their constant is added once per lane.
+//   counted and their constant is added once per lane.  In a cubic box wider than four cutoffs
+//   (FILTER) an FP32 distance of fixed-point box fractions, off by less than 1e-6 and 4e-9 of
+//   the box, finds the few pairs that can be in range; they queue in LDS, and 64 at a time are
+//   taken in FP64.  The same atoms then take 71 us, 62 of them block 0's ordered sum (leaving
+//   out only the atoms j that no lane has in range: 81).  A tile with an atom more than 1,024
+//   boxes away takes every pair in FP64.
 //   Coulomb (:321-351): q_j / r, beyond the cutoff q_j / R; reaction field: in the cutoff only.
 // Block 0 of the launch adds the kinetic energy in index order meanwhile (ke_out).
 enum { REF_PE_LJ = 0, REF_PE_COULOMB = 1, REF_PE_RF = 2 };
 struct ref_pe_law {
     double s2, R, R2, krf, crf;
+    double invL;     // FILTER: 1 / L
+    float near2;     // FILTER: above the cutoff's square in the units of the box fractions
     int jstride, water;
 };
 
-template <int KIND>
+template <int KIND, bool FILTER>
 __global__ void __launch_bounds__(256)
 k_ref_pair_pe(const double* __restrict__ x, const double* __restrict__ qs, int64_t n, int64_t nj,
               ref_pe_law law, nbx_bcv bc, double* __restrict__ part,
@@ -1151,6 +1171,7 @@ k_ref_pair_pe(const double* __restrict__ x, const double* __restrict__ qs, int64
         return;
     }
     __shared__ double sj[4][64][4];
+    __shared__ uint16_t queue[FILTER ? 4 : 1][128];
     __shared__ double red[4];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1178,8 +1199,16 @@ k_ref_pair_pe(const double* __restrict__ x, const double* __restrict__ qs, int64
             sj[wave][lane][3] = KIND != REF_PE_LJ ? qs[j] : 0.0;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        uint32_t ui[3] = {0u, 0u, 0u}, uj[3] = {0u, 0u, 0u};
+        bool ok = FILTER;
+        if (FILTER) {
+            if (a < nj) ok = box_fixed(xi, yi, zi, law.invL, ui);
+            if (lane < nb)
+                ok = box_fixed(sj[wave][lane][0], sj[wave][lane][1], sj[wave][lane][2], law.invL,
+                               uj) && ok;
+        }
         double ei = 0.0;
-        for (int k = 0; k < nb; ++k) {
+        const auto exact = [&](int k) {
             double rx, ry, rz, r2;
             nbx_displacement(xi, yi, zi, sj[wave][k][0], sj[wave][k][1], sj[wave][k][2], bc, rx, ry,
                              rz, r2);
@@ -1199,6 +1228,52 @@ k_ref_pair_pe(const double* __restrict__ x, const double* __restrict__ qs, int64
             } else if (pair) {
                 ei += sj[wave][k][3] / (in ? sqrt(r2) : law.R);
             }
+        };
+        if (FILTER && !__any(!ok)) {   // off the diagonal every lane holds an atom, a < b
+            const bool diagonal = I == J;
+            int queued = 0, found = 0;
+            // the term of a queued pair: a source lane's atom and a staged atom
+            const auto term = [&](int slot, bool live) {
+                const int w = live ? queue[wave][slot] : 0;
+                const double x0 = __shfl(xi, w >> 6, 64), y0 = __shfl(yi, w >> 6, 64),
+                             z0 = __shfl(zi, w >> 6, 64);
+                const double* const q = sj[wave][w & 63];
+                double rx, ry, rz, r2;
+                nbx_displacement(x0, y0, z0, q[0], q[1], q[2], bc, rx, ry, rz, r2);
+                if (live && r2 < law.R2) {
+                    const double q2 = law.s2 / r2;
+                    const double s6 = q2 * q2 * q2;
+                    const double s12 = s6 * s6;
+                    ei += s12 - s6;
+                    ++found;
+                }
+            };
+            for (int k = 0; k < nb; ++k) {
+                const float dx = (float)(int)(ui[0] - __builtin_amdgcn_readlane(uj[0], k));
+                const float dy = (float)(int)(ui[1] - __builtin_amdgcn_readlane(uj[1], k));
+                const float dz = (float)(int)(ui[2] - __builtin_amdgcn_readlane(uj[2], k));
+                const bool pair = !diagonal || k > lane;
+                const bool near = pair && fmaf(dz, dz, fmaf(dy, dy, dx * dx)) < law.near2;
+                const unsigned long long mask = __ballot(near);
+                if (mask == 0ull) continue;
+                const int at = (int)__builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, (unsigned)queued));
+                if (near) queue[wave][at] = (uint16_t)(lane << 6 | k);
+                queued += __popcll(mask);
+                if (queued >= 64) {
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    queued -= 64;
+                    term(queued + lane, true);   // the newest: the older stay where they are
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                }
+            }
+            if (queued > 0) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                term(lane, lane < queued);
+            }
+            far += (diagonal ? (lane < nb ? nb - 1 - lane : 0) : nb) - found;
+        } else {
+            for (int k = 0; k < nb; ++k) exact(k);
         }
         e += KIND == REF_PE_LJ ? ei : ei * qi;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1236,8 +1311,12 @@ static void pair_pe(hipStream_t s, const double* x, const double* qs, int64_t n,
     const int64_t T = (nj + 63) >> 6;
     // 2,048 blocks of four wavefronts fill the chip (d_part holds 8,192 doubles at least)
     const int blocks = (int)std::min<int64_t>((T * (T + 1) / 2 + 3) / 4, 2048);
-    hipLaunchKernelGGL(k_ref_pair_pe<KIND>, dim3(blocks + 1), dim3(256), 0, s, x, qs, n, nj, law,
-                       bc, d_part, ke.v, ke.ms, ke.out);
+    if (law.near2 > 0.0f)
+        hipLaunchKernelGGL((k_ref_pair_pe<KIND, KIND == REF_PE_LJ>), dim3(blocks + 1), dim3(256), 0,
+                           s, x, qs, n, nj, law, bc, d_part, ke.v, ke.ms, ke.out);
+    else
+        hipLaunchKernelGGL((k_ref_pair_pe<KIND, false>), dim3(blocks + 1), dim3(256), 0, s, x, qs, n,
+                           nj, law, bc, d_part, ke.v, ke.ms, ke.out);
     hipLaunchKernelGGL(k_ref_pe_sum, dim3(1), dim3(256), 0, s, d_part, blocks, d_out);
 }
 
@@ -1248,6 +1327,11 @@ void ref64_lj_pe(hipStream_t s, const double* x, int64_t n, int jstride, int64_t
     law.s2 = sigma * sigma;
     law.R2 = R * R;
     law.jstride = jstride;
+    if (bc.kind == NBX_BC_CUBIC && R < 0.25 * bc.b[0]) {
+        law.invL = 1.0 / bc.b[0];
+        const double near = (R * law.invL * (1.0 + 1e-6) + 4e-9) * 4294967296.0;
+        law.near2 = (float)(near * near);
+    }
     pair_pe<REF_PE_LJ>(s, x, nullptr, n, nj, law, bc, d_part, d_out, ke);
 }
 
@@ -1335,29 +1419,19 @@ void ref64_bonded_pe(hipStream_t s, const double* x, int64_t n, double rOH, doub
 // RDF histogram (src/nbody_simulation_result.jl:664-693): frames in AoS (3 x n each)
 // ---------------------------------------------------------------------------
 
-// Bound by FP64 VALU work (about 100 instructions per pair: the wrapped displacement, the
-// square root and the division that the bin's rounding needs).  A wavefront takes 64 atoms
-// a (one per lane) against 64 atoms b from LDS, pairs b > a; wavefronts stride over the
-// upper triangle of 64 x 64 tiles of all frames, so few atoms or frames still spread over
-// the chip.  Counts go to a histogram in LDS shared by the block (one ds_add_u32 per pair
-// in range) and reach memory once per block.  Device-scope 64-bit atomics per pair from
-// n / 128 blocks took 3,170 us per frame of 4,000 atoms; this takes 23 (10 frames at once).
+// Bound by VALU work.  A wavefront takes 64 atoms a (one per lane) against 64 atoms b, pairs
+// b > a; wavefronts stride over the upper triangle of 64 x 64 tiles of all frames, so few
+// atoms or frames still spread over the chip.  The bin is estimated in FP32 from fixed-point
+// box fractions (the integer wrap-around is the minimum image); only where a lane's estimate
+// lies so near the edge of a bin or of the range that FP64 may put it on the other side
+// (6e-7 of the distance for the FP32 operations, 2e-9 of the box for the fractions) does the
+// wavefront take the FP64 displacement, square root and division: one iteration in 20 with
+// 1,000 bins.  Counts go to a histogram in LDS shared by the block (one ds_add_u32 per pair
+// in range) and reach memory once per block.  10 frames of 4,000 atoms: 99 us, all pairs in
+// FP64 220; device-scope 64-bit atomics per pair from n / 128 blocks took 3,170 a frame.
 // Above RDF_LDS_BINS bins (64 KiB of LDS with the staged atoms) the counts go to memory
-// directly.
+// directly, and every pair takes FP64 (the estimate is open too often to pay).
 #define RDF_LDS_BINS 8000
-
-// box fractions in units of 2^-32; false where the coordinate is more than 1,024 boxes away (or
-// no number), too far for the bound on the difference to the FP64 distance
-__device__ __forceinline__ bool rdf_fixed(double x, double y, double z, double invL, uint32_t* q) {
-    const double t[3] = {x * invL, y * invL, z * invL};
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        ok = ok && fabs(t[k]) < 1024.0;
-        q[k] = ok ? (uint32_t)(uint64_t)((t[k] - floor(t[k])) * 4294967296.0) : 0u;
-    }
-    return ok;
-}
 
 template <bool LDS>
 __global__ void __launch_bounds__(1024)
@@ -1429,9 +1503,9 @@ k_ref_rdf(const double* __restrict__ f, int64_t n, int jstride, int64_t nj, int6
             uint32_t qi[3] = {0u, 0u, 0u}, qj[3] = {0u, 0u, 0u};
             bool ok = true;
             if (LDS) {
-                if (a < nj) ok = rdf_fixed(xi, yi, zi, invL, qi);
+                if (a < nj) ok = box_fixed(xi, yi, zi, invL, qi);
                 if (lane < nb)
-                    ok = rdf_fixed(sb[4 * lane], sb[4 * lane + 1], sb[4 * lane + 2], invL, qj) && ok;
+                    ok = box_fixed(sb[4 * lane], sb[4 * lane + 1], sb[4 * lane + 2], invL, qj) && ok;
             }
             if (!LDS || __any(!ok)) {
                 for (int k = 0; k < nb; ++k) exact(k);

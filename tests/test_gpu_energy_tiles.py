@@ -49,3 +49,29 @@ def test_energies_match_oracle(nbx, n, el, bc):
     assert ke == orc.kinetic_energy(v) and pg == 0.0
     assert pe == pytest.approx(orc.potential_energy(u), rel=1e-11, abs=1e-300)
     assert ctx.temperature() == O.load().orc_md_temperature(O.dp(v), O.dp(m), 1.0, n, 0)
+
+
+@pytest.mark.parametrize("shift", [1000, 3000])
+def test_energies_with_atoms_many_boxes_away(nbx, shift):
+    # on either side of the distance up to which pairs are found in FP32; the images differ
+    # from the atoms in the box by the rounding of shift * L only (1e-12 of a distance, 1e-11
+    # of a close pair's energy)
+    print(f"[case] energies, atoms {shift} boxes away", flush=True)
+    n = 1025
+    rng = np.random.default_rng(shift)
+    L = 16.0   # shift * L is exact
+    g = np.stack(np.meshgrid(*[np.arange(11)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    u = g * (L / 11) + rng.uniform(0, 0.3, (n, 3))
+    w = u.copy()
+    w[::50] += shift * L * rng.integers(-1, 2, w[::50].shape)
+    pes = []
+    for x in (u, w):
+        ctx = _lib.Context(n, _lib.SYS_POTENTIAL, np.ones(n))
+        ctx.set_boundary(_lib.BC_CUBIC, [L, 0, 0, 0, 0, 0])
+        ctx.add_lennard_jones(1.0, 1.0, 2.5)
+        ctx.set_state(x, np.zeros_like(x))
+        pes.append(ctx.energies()[1])
+    orc = O.System(np.ones(n), bc=O.make_bc(O.BC_CUBIC, L)).add(O.TERM_LJ, 1.0, 1.0, 2.5)
+    assert pes[0] == pytest.approx(orc.potential_energy(u), rel=1e-11)
+    assert pes[1] == pytest.approx(orc.potential_energy(w), rel=1e-11)
+    assert pes[1] == pytest.approx(pes[0], rel=1e-9)
