@@ -142,17 +142,19 @@ def mixed_accel(ctx, u):
 
 def gravity_issue_model(ctx, pairs, kernel_ms, equal_masses):
     """Issue-limited time of k_grav_tiled from the measured issue rates of its
-    instruction kinds (nbx_valu_probe, wave64 instructions per SIMD per ns): per pair
-    3 v_sub + 3 v_mul (2 when every body has the same mass: the kernel then leaves the
-    mass out of the pair term) at the v_mul rate, 6 FMA at the v_fmac rate, one
-    v_rsq_f32."""
+    instruction kinds (nbx_valu_probe, wave64 instructions per SIMD per ns).  The kernel
+    evaluates each unordered pair once and adds it to both bodies: 3 v_sub, 2 v_mul (4 with
+    unequal masses: each side takes the other's) at the v_mul rate, 9 FMA at the v_fmac
+    rate, one v_rsq_f32, and with four targets per lane three quarters of a lane rotation
+    of the source sums, counted at the v_mul rate."""
     r_fma, r_mul, r_rsq = (ctx.valu_probe(k, 5) for k in (0, 1, 2))
     simds = 4 * 256
-    muls = 2 if equal_masses else 3
-    ns_per_wave_pair = (3.0 + muls) / r_mul + 6.0 / r_fma + 1.0 / r_rsq  # per 64 pairs, per SIMD
-    bound_ms = pairs / 64.0 * ns_per_wave_pair / simds * 1e-6
+    muls = 2 if equal_masses else 4
+    ns_per_wave_pair = (3.0 + muls + 0.75) / r_mul + 9.0 / r_fma + 1.0 / r_rsq  # per 64, per SIMD
+    bound_ms = pairs / 2.0 / 64.0 * ns_per_wave_pair / simds * 1e-6
     return {"fmac_per_simd_ns": r_fma, "mul_per_simd_ns": r_mul, "rsq_per_simd_ns": r_rsq,
-            "instructions_per_pair": f"3 sub, {muls} mul, 6 fma, 1 v_rsq_f32",
+            "instructions_per_unordered_pair": f"3 sub, {muls} mul, 9 fma, 1 v_rsq_f32, "
+                                               "0.75 lane rotations",
             "issue_bound_ms": bound_ms, "frac_of_issue_bound": bound_ms / kernel_ms}
 
 
