@@ -1519,6 +1519,7 @@ int mx_autotune(nbx_ctx* c, double dt, int trial, double* out, int nout) {
         NBX_HIP(c, hipStreamSynchronize(s));
         const auto t0 = std::chrono::steady_clock::now();
         if ((r = mx_vv(c, dt, trial, 0, 0, nullptr, nullptr, &nf))) return r;
+        NBX_HIP(c, hipStreamSynchronize(s));   // a plan without lists only enqueues its steps
         const auto t1 = std::chrono::steady_clock::now();
         *ms = std::chrono::duration<double, std::milli>(t1 - t0).count() / trial;
         return NBX_OK;

@@ -48,3 +48,18 @@ def test_every_pair_once(nbx, n, equal):
     # every pair enters both bodies: the total momentum stays at rest
     f = (m[:, None] * a)
     assert np.abs(f.sum(axis=0)).max() <= 1e-5 * np.abs(f).sum()
+
+
+def test_autotuner_times_the_steps_not_their_launches(nbx):
+    # a step takes at least its force kernel; half of it leaves room for the clock
+    print("[case] gravity autotuner n=40000", flush=True)
+    n = 40000
+    u, v, m = gen.plummer(n, seed=3)
+    ctx = _lib.Context(n, _lib.SYS_POTENTIAL, m)
+    ctx.add_gravitational(1.0)
+    ctx.set_precision(_lib.PREC_MIXED)
+    ctx.set_state(u, v)
+    tuned = ctx.autotune(1e-3, 10)
+    ctx.set_state(u, v)
+    kernel_ms, _ = ctx.time_force_kernel(5)
+    assert tuned["entry_ms_per_step"] >= 0.5 * kernel_ms
