@@ -89,8 +89,16 @@ void ref64_soa_to_aos(hipStream_t s, const double* soa, double* aos, int64_t n) 
 // chunk through v_readlane: n = 864 36.6 -> 7.9 (the fused step included), n = 4,000
 // 341 -> 22; water's Coulomb and Lennard-Jones terms (1,029 atoms, cutoff 0.45 L) 71 -> 13.6.
 // A few targets per SIMD make it a latency chain: one wavefront's fractions, gathers, pair
-// terms and about 13 cycles per ordered add.
+// terms and about 13 cycles per ordered add; up to REF_SPLIT_TARGETS targets share it among
+// four wavefronts each (ref_block_sum; n = 864 7.7 -> 6.5).
 #define REF_WAVES 4   // targets (wavefronts) per block
+// Targets that get a block of four wavefronts each (filtered sums): as many as run at once,
+// six blocks (27 KB of LDS each) on each of 256 CUs.  us per step with one / four
+// wavefronts: Lennard-Jones n = 256 5.4 / 5.2, 500 6.3 / 5.5, 864 7.7 / 6.3, 1,372 9.7 / 9.5,
+// 2,048 11.2 / 13.1, 4,000 20 / 33; water (4/3 targets an atom) 375 atoms 13.1 / 10.9, 1,029
+// 17.9 / 17.1, 1,536 19.4 / 19.2, 2,187 24.1 / 28.2.
+#define REF_SPLIT_BLOCKS 6
+#define REF_SPLIT_TARGETS (256 * REF_SPLIT_BLOCKS)
 enum { REF_LJ = 0, REF_COULOMB = 1, REF_RF = 2, REF_GRAV = 3 };
 
 struct ref_law {
@@ -157,6 +165,27 @@ __device__ __forceinline__ bool ref_pair_term(const ref_law& law, double xi, dou
 }
 
 // the whole wavefront's sum over the sources of target i: component min(lane, 2) in each lane
+// component c of cnt terms added to f one after another
+__device__ __forceinline__ double ref_add_terms(double f, const double* term, int cnt, int c) {
+    int q = 0;
+    for (; q + 16 <= cnt; q += 16) {
+        double u[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) u[k] = term[3 * (q + k) + c];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) f += u[k];
+    }
+    for (; q + 4 <= cnt; q += 4) {
+        double u[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) u[k] = term[3 * (q + k) + c];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) f += u[k];
+    }
+    for (; q < cnt; ++q) f += term[3 * q + c];
+    return f;
+}
+
 template <int KIND, bool FILTER>
 __device__ __forceinline__ double ref_wave_sum(const ref_atoms& A, const ref_law& law,
                                                const nbx_bcv& bc, int64_t i, int* cand,
@@ -181,23 +210,7 @@ __device__ __forceinline__ double ref_wave_sum(const ref_atoms& A, const ref_law
             term[3 * at + 2] = t[2];
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        const int cnt = __popcll(mask);
-        int q = 0;
-        for (; q + 16 <= cnt; q += 16) {
-            double u[16];
-#pragma unroll
-            for (int k = 0; k < 16; ++k) u[k] = term[3 * (q + k) + c];
-#pragma unroll
-            for (int k = 0; k < 16; ++k) f += u[k];
-        }
-        for (; q + 4 <= cnt; q += 4) {
-            double u[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) u[k] = term[3 * (q + k) + c];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) f += u[k];
-        }
-        for (; q < cnt; ++q) f += term[3 * q + c];
+        f = ref_add_terms(f, term, __popcll(mask), c);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     };
     if constexpr (FILTER) {
@@ -258,6 +271,85 @@ __device__ __forceinline__ double ref_wave_sum(const ref_atoms& A, const ref_law
             const int64_t jj = base + lane;
             add(jj < law.nj && !ref_excluded(i, jj * law.jstride, law.water), px, py, pz, pw);
         }
+    }
+    return f;
+}
+
+// The filtered sum of one target by a block of four wavefronts: in a round of at most 1,024
+// sources each takes up to 256 consecutive ones, filters them and leaves its terms in LDS in
+// ascending j; the first wavefront then adds the four runs of terms in order, so the sum is
+// that of ref_wave_sum bit for bit.  With few targets the sum is a latency chain, and a
+// wavefront alone spends most of it in the filter (n = 864, us: filter 3.3, terms and adds
+// 1.5, end of the step 0.6).  The result is valid in wavefront 0.
+struct ref_block_lds {
+    uint16_t cand[4][256];
+    double term[4][3 * 256];
+    int count[4];
+};
+
+template <int KIND>
+__device__ __forceinline__ double ref_block_sum(const ref_atoms& A, const ref_law& law,
+                                                const nbx_bcv& bc, int64_t i, ref_block_lds& S) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane < 2 ? lane : 2;
+    const int64_t n = A.n;
+    const double xi = A.x[i], yi = A.x[n + i], zi = A.x[2 * n + i];
+    const float4 fi = A.frac[i];
+    const double* const w = KIND == REF_LJ ? nullptr : A.qs;
+    const int64_t chunks = (law.nj + 63) >> 6;
+    // rounds of equal size, at most four chunks per wavefront
+    const int64_t rounds = (chunks + 15) >> 4;
+    const int u = (int)((chunks + 4 * rounds - 1) / (4 * rounds));
+    double f = 0.0;
+    for (int64_t first = 0; first < chunks;) {   // the same for the whole block
+        const int64_t base = 64 * (first + wave * u);
+        float4 fj[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t jj = base + 64 * q + lane;
+            fj[q] = A.frac[q < u && jj < law.nj ? jj * law.jstride : i];
+        }
+        int pending = 0;   // uniform over the wavefront
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t jj = base + 64 * q + lane;
+            float dx = fi.x - fj[q].x, dy = fi.y - fj[q].y, dz = fi.z - fj[q].z;
+            dx -= rintf(dx);
+            dy -= rintf(dy);
+            dz -= rintf(dz);
+            const bool near = q < u && jj < law.nj && !ref_excluded(i, jj * law.jstride, law.water) &&
+                              !(dx * dx + dy * dy + dz * dz >= law.lim);
+            const unsigned long long mask = __ballot(near);
+            const int at = pending + (int)__builtin_amdgcn_mbcnt_hi(
+                (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+            if (near) S.cand[wave][at] = (uint16_t)(64 * q + lane);
+            pending += __popcll(mask);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        int got = 0;
+        for (int p = 0; p < pending; p += 64) {
+            const bool ok = p + lane < pending;
+            const int64_t j = ok ? (base + S.cand[wave][p + lane]) * law.jstride : i;
+            double t[3] = {0.0, 0.0, 0.0};
+            const bool hit = ok && ref_pair_term<KIND>(law, xi, yi, zi, A.x[j], A.x[n + j],
+                                                       A.x[2 * n + j], w != nullptr ? w[j] : 0.0,
+                                                       bc, t);
+            const unsigned long long mask = __ballot(hit);
+            const int at = got + (int)__builtin_amdgcn_mbcnt_hi(
+                (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+            if (hit) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) S.term[wave][3 * at + k] = t[k];
+            }
+            got += __popcll(mask);
+        }
+        if (lane == 0) S.count[wave] = got;
+        first += 4 * u;
+        __syncthreads();
+        if (wave == 0)
+            for (int v = 0; v < 4; ++v) f = ref_add_terms(f, S.term[v], S.count[v], c);
+        if (first < chunks) __syncthreads();   // read before the next round writes
     }
     return f;
 }
@@ -342,6 +434,26 @@ k_ref_pairs(ref_atoms A, ref_law law, nbx_bcv bc, int64_t ib, int64_t cnt, int i
     }
 }
 
+// a block per target: few targets (REF_SPLIT_TARGETS)
+template <int KIND, bool STEP>
+__global__ void __launch_bounds__(256, REF_SPLIT_BLOCKS)
+k_ref_pairs_split(ref_atoms A, ref_law law, nbx_bcv bc, int64_t ib, int istride,
+                  double* __restrict__ dv, ref64_step st) {
+    __shared__ ref_block_lds S;
+    const int64_t i = ib + (int64_t)blockIdx.x * istride;
+    const double f = ref_block_sum<KIND>(A, law, bc, i, S);
+    if (threadIdx.x >= 3) return;
+    const int c = threadIdx.x;
+    const double add = ref_contribution<KIND>(A, law, i, f);
+    const int64_t k = c * A.n + i;
+    if constexpr (STEP) {
+        ref_end_step(st, A.n, i, c, (st.a_in != nullptr ? st.a_in[k] : 0.0) + add, A.ms[i], i,
+                     A.ms[0]);
+    } else {
+        dv[k] += add;
+    }
+}
+
 static double rf_krf(double R, double eps_rf) {
     if (__builtin_isinf(eps_rf)) return 1.0 / (2.0 * R * R * R);
     return (eps_rf - 1.0) / ((2.0 * eps_rf + 1.0) * (R * R * R));
@@ -385,6 +497,11 @@ static void launch_pairs(hipStream_t s, const ref64_term& t, const ref_atoms& A,
     const int64_t cnt = (ie - ib + t.istride - 1) / t.istride;
     const dim3 grid(nbx_blocks(cnt, REF_WAVES)), block(64 * REF_WAVES);
     if constexpr (KIND != REF_GRAV) {
+        if (t.filter && cnt <= REF_SPLIT_TARGETS) {
+            hipLaunchKernelGGL((k_ref_pairs_split<KIND, STEP>), dim3((unsigned)cnt), dim3(256), 0, s,
+                               A, law, bc, ib, t.istride, dv, st);
+            return;
+        }
         if (t.filter) {
             hipLaunchKernelGGL((k_ref_pairs<KIND, true, STEP>), grid, block, 0, s, A, law, bc, ib,
                                cnt, t.istride, dv, st);
@@ -837,6 +954,23 @@ k_ref_water_pairs(ref_atoms A, ref_law el, ref_law lj, nbx_bcv bc, double* __res
     }
 }
 
+template <int KIND>
+__global__ void __launch_bounds__(256, REF_SPLIT_BLOCKS)
+k_ref_water_pairs_split(ref_atoms A, ref_law el, ref_law lj, nbx_bcv bc, double* __restrict__ elec,
+                        double* __restrict__ ljv) {
+    __shared__ ref_block_lds S;
+    const int64_t n = A.n, t = blockIdx.x;
+    const int c = threadIdx.x;
+    if (t < n) {
+        const double f = ref_block_sum<KIND>(A, el, bc, t, S);
+        if (c < 3) elec[c * n + t] = ref_contribution<KIND>(A, el, t, f);
+    } else {
+        const int64_t i = 3 * (t - n);
+        const double f = ref_block_sum<REF_LJ>(A, lj, bc, i, S);
+        if (c < 3) ljv[c * n + i] = ref_contribution<REF_LJ>(A, lj, i, f);
+    }
+}
+
 // one thread per component of an atom (thread t: atom t / 3, component t % 3)
 __global__ void __launch_bounds__(192)
 k_ref_water_step(const double* __restrict__ ms, int64_t n, const double* __restrict__ elec,
@@ -874,7 +1008,11 @@ void ref64_water_step(hipStream_t s, const ref64_term& el, const ref64_term& lj,
     const dim3 grid(nbx_blocks(n + n / 3, REF_WAVES)), block(64 * REF_WAVES);
     const bool rf = el.kind == NBX_TERM_RF;
     // both laws filter, or neither (el.filter == lj.filter)
-    if (el.filter) {
+    if (el.filter && n + n / 3 <= REF_SPLIT_TARGETS) {
+        const dim3 each((unsigned)(n + n / 3)), four(256);
+        if (rf) hipLaunchKernelGGL((k_ref_water_pairs_split<REF_RF>), each, four, 0, s, A, le, ll, bc, elec, ljv);
+        else hipLaunchKernelGGL((k_ref_water_pairs_split<REF_COULOMB>), each, four, 0, s, A, le, ll, bc, elec, ljv);
+    } else if (el.filter) {
         if (rf) hipLaunchKernelGGL((k_ref_water_pairs<REF_RF, true>), grid, block, 0, s, A, le, ll, bc, elec, ljv);
         else hipLaunchKernelGGL((k_ref_water_pairs<REF_COULOMB, true>), grid, block, 0, s, A, le, ll, bc, elec, ljv);
     } else {

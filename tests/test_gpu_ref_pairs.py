@@ -159,3 +159,24 @@ def test_small_run_of_several_launches(nbx):
     uo, vo, (ufo, vfo) = orc.vv_run(u, v, 1e-3, 45000, save_every=7)
     assert np.array_equal(uf, ufo) and np.array_equal(vf, vfo)
     assert np.array_equal(ctx.get_state()[0], uo)
+
+
+# Four wavefronts per target up to 1,536 targets, in rounds of at most 1,024 sources: a round's
+# edge, the last targets of the rule and the first past it, and a cutoff of nearly half the
+# box, with about half of a wavefront's 256 sources in range
+@pytest.mark.parametrize("law", ["lj", "rf", "wide"])
+@pytest.mark.parametrize("n", [255, 257, 1024, 1025, 1536, 1537, 2049])
+def test_forces_by_four_wavefronts_bitwise(nbx, monkeypatch, n, law):
+    print(f"[case] fp64 pairs by four wavefronts n={n} law={law}", flush=True)
+    L = 1.2 * n ** (1.0 / 3.0)
+    monkeypatch.setitem(LAWS, "wide", [("el", 1.3, 0.49 * L)])
+    ctx, orc, rng = pair(n, law, "cubic", L)
+    u = lattice(n, L, rng)
+    u[::5] += L * rng.integers(-40, 41, (len(u[::5]), 3))
+    assert np.array_equal(ctx.rhs(u), orc.rhs(u))
+    v = rng.standard_normal((n, 3))
+    ctx.set_state(u, v)
+    ctx.vv_run(0.001, 2)
+    uo, vo, _ = orc.vv_run(u, v, 0.001, 2)
+    u1, v1 = ctx.get_state()
+    assert np.array_equal(u1, uo) and np.array_equal(v1, vo)
