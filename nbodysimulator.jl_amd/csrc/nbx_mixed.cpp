@@ -500,15 +500,20 @@ static int read_flags(nbx_ctx* c, int* h) {
 // 2 to 3 us; the earlier requests of M = 5 rebuild about half as often again (whole runs:
 // Lennard-Jones, n = 32,000, 250 steps of 0.002 4.13 -> 3.98 ms, n = 864 with the lanes by
 // size, 300 steps 2.82 -> 1.86 ms).  A state that speeds up past it marks a list stale and is
-// replayed with M = 1, as with any interval.
+// replayed with M = 1, as with any interval, at twice the cost: water without a thermostat,
+// whose bonds do that to many a state (519 molecules, 102 steps 7.3 ms with M = 1, 15.5
+// replayed), takes M = 1.
 static void choose_build_every(nbx_ctx* c, const mx_plan& p, double dt) {
     if (!c->every_auto || c->every_chosen || p.kind == PLAN_GRAVITY || !p.nb.mode_list) return;
     c->every_chosen = true;
+    c->build_every = 1;
+    // strained bonds speed up atoms that nothing cools; a context that had a list go stale
+    // keeps M = 1
+    if ((p.nb.water && c->therm == NBX_THERM_NONE) || c->stale_replays > 0) return;
     double v2 = c->speed2;
     if (c->therm != NBX_THERM_NONE && c->n > 0)
         v2 = std::max(v2, 25.0 * c->kb * c->therm_T * c->mass_wmin);
     const double reach = 1.25 * std::sqrt(v2) * dt;
-    c->build_every = 1;
     for (int M : {5, 2})
         if (reach * M <= 0.5 * c->nl.skin * (double)(M - 1) / (2.0 * M)) {
             c->build_every = M;
