@@ -943,57 +943,56 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
     }
 }
 
-// small boxes (fewer than 3 cells per side): every atom scans all atoms
-template <bool WATER>
-__device__ __forceinline__ void build_allpairs_atom(const double4* __restrict__ pos,
-                                                    const double* __restrict__ x, int i, int n,
-                                                    double L, double invL, double rlist2, int G,
-                                                    int cap, void* __restrict__ nbr,
-                                                    int nbr_wide, int* __restrict__ nnb,
-                                                    double* __restrict__ xref,
-                                                    int* __restrict__ flags) {
-    if (i == 0) atomicAdd(&flags[2], 1);
-    const double4 pi = pos[i];
-    const size_t stride = (size_t)n * G;
-    const int lgG = __builtin_ctz((unsigned)G);
-    int c = 0;
-    for (int j = 0; j < n; ++j) {
-        if (j == i) continue;
-        if (WATER && (j / 3) == (i / 3)) continue;
-        const double4 pj = pos[j];
-        double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
-        dx -= L * rint(dx * invL);
-        dy -= L * rint(dy * invL);
-        dz -= L * rint(dz * invL);
-        if (dx * dx + dy * dy + dz * dz < rlist2) {
-            if (c < cap)
-                mx_nbr_store(nbr, nbr_wide, (size_t)(c >> lgG) * stride + (size_t)i * G + (c & (G - 1)), j);
-            ++c;
-        }
-    }
-    if (c > cap) { flags[1] = 1; c = cap; }
-    nnb[i] = c;
-    xref[i] = x[i];
-    xref[n + i] = x[n + i];
-    xref[2 * n + i] = x[2 * n + i];
-}
+// Small boxes (fewer than 3 cells per side): every atom against all atoms, a wavefront per
+// atom whose lanes test 64 others at a time and append the hits in index order (ballot +
+// prefix count).  One thread per atom took 600 us a build for 795 water molecules, a chain
+// of 2,385 dependent tests (a pass of 136 steps with 15 builds 11,300 -> 2,300 us).
+#define ALLPAIRS_WAVES 4
 
 template <bool WATER>
-__global__ void k_build_allpairs(const double4* __restrict__ pos, const double* __restrict__ x,
-                                 int n, double L, double invL, double rlist2, int G, int cap,
-                                 void* __restrict__ nbr, int nbr_wide, int* __restrict__ nnb,
-                                 double* __restrict__ xref, int* __restrict__ flags,
-                                 int* __restrict__ req) {
+__global__ void __launch_bounds__(64 * ALLPAIRS_WAVES)
+k_build_allpairs(const double4* __restrict__ pos, const double* __restrict__ x, int n, double L,
+                 double invL, double rlist2, int G, int cap, void* __restrict__ nbr, int nbr_wide,
+                 int* __restrict__ nnb, double* __restrict__ xref, int* __restrict__ flags,
+                 int* __restrict__ req) {
     if (req[0] == 0) return;   // uniform: only this kernel's last block clears the request
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        build_allpairs_atom<WATER>(pos, x, i, n, L, invL, rlist2, G, cap, nbr, nbr_wide, nnb,
-                                   xref, flags);
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&flags[2], 1);
+    const int lane = threadIdx.x & 63;
+    const int i = __builtin_amdgcn_readfirstlane(blockIdx.x * ALLPAIRS_WAVES + (threadIdx.x >> 6));
+    if (i < n) {
+        const double4 pi = pos[i];
+        const size_t stride = (size_t)n * G;
+        const int lgG = __builtin_ctz((unsigned)G);
+        int c = 0;   // uniform
+        double4 nx = pos[lane < n ? lane : i];
+        for (int j0 = 0; j0 < n; j0 += 64) {
+            const int j = j0 + lane;
+            const double4 pj = nx;
+            nx = pos[j + 64 < n ? j + 64 : i];
+            double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
+            dx -= L * rint(dx * invL);
+            dy -= L * rint(dy * invL);
+            dz -= L * rint(dz * invL);
+            const bool hit = j < n && (WATER ? j / 3 != i / 3 : j != i) &&
+                             dx * dx + dy * dy + dz * dz < rlist2;
+            const unsigned long long mask = __ballot(hit);
+            const int r = (int)__builtin_amdgcn_mbcnt_hi(
+                (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, (unsigned)c));
+            if (hit && r < cap)
+                mx_nbr_store(nbr, nbr_wide,
+                             (size_t)(r >> lgG) * stride + (size_t)i * G + (r & (G - 1)), j);
+            c += __popcll(mask);
+        }
+        if (lane == 0) {
+            if (c > cap) { flags[1] = 1; c = cap; }
+            nnb[i] = c;
+        }
+        if (lane < 3) xref[(size_t)lane * n + i] = x[(size_t)lane * n + i];
+    }
     __shared__ int last;
     __syncthreads();
-    if (threadIdx.x == 0)   // no fence: the last block only clears what every block read
-        last = atomicAdd(reinterpret_cast<unsigned*>(&flags[NBX_FLAG_BINSET + 1]), 1u) ==
-               gridDim.x - 1;
+    // no fence: the last block only clears what every block read
+    if (threadIdx.x == 0) last = build_finished(flags);
     __syncthreads();
     if (last && threadIdx.x == 0) {
         flags[NBX_FLAG_BINSET + 1] = 0;
@@ -1037,8 +1036,8 @@ static void launch_build_t(hipStream_t s, const nbx_ctx* c, const void* pos, con
             hipLaunchKernelGGL((k_build_cells<WATER, false, 256, 3>), BUILD_ARGS(256));
 #undef BUILD_ARGS
     } else {
-        hipLaunchKernelGGL((k_build_allpairs<WATER>), dim3(nbx_blocks(n, 128)), dim3(128), 0,
-                           s, (const double4*)pos, x, n, L, 1.0 / L, r2, nl.lanes, nl.cap, nbr,
+        hipLaunchKernelGGL((k_build_allpairs<WATER>), dim3(nbx_blocks(n, ALLPAIRS_WAVES)),
+                           dim3(64 * ALLPAIRS_WAVES), 0, s, (const double4*)pos, x, n, L, 1.0 / L, r2, nl.lanes, nl.cap, nbr,
                            nl.nbr_wide, nl.d_nnb, nl.d_xref, nl.d_flags, req);
     }
 }

@@ -18,6 +18,9 @@ def pairs_within(u, L, r):
 
 
 @pytest.mark.parametrize("cells,rho,R,skin", [
+    (2, 0.8442, 1.5, 0.3),     # all pairs, fewer atoms than lanes
+    (4, 0.8442, 2.5, 0.3),     # all pairs, 256 atoms
+    (5, 0.8442, 2.7, 0.3),     # all pairs, 500
     (6, 0.8442, 2.5, 0.3),     # 3 cells per side
     (8, 0.8442, 2.5, 0.3),     # 4
     (9, 0.8442, 2.5, 0.2),     # 5
