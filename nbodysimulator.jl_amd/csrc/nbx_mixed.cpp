@@ -861,15 +861,18 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
                 break;
             }
             c->kt_used = 0;   // replayed: its timings are dropped
-            // overflow: restore and replay with larger lists; a list that went stale between
-            // two build opportunities: restore and replay with an opportunity at every step
+            // a list that went stale between two build opportunities: restore and replay with
+            // an opportunity at every step; overflow: restore and replay with larger lists.
+            // Stale first: the steps after it ran on a list that misses pairs, and what they
+            // overflowed (the builds' bins are flagged past 3/4 skin) larger lists do not mend
             ref64_copy_state(s, bkp, live, (int64_t)n3, NBX_SCAL_COUNT);
-            if (h[1]) {
-                if ((rc = grow_lists(c, p, grow))) return rc;
-            } else {
+            if (h[7]) {
                 c->build_every = 1;
                 ++c->stale_replays;
                 mx_launch_fill_int(s, c->nl.d_flags + 7, 1, 0);
+                mx_launch_fill_int(s, c->nl.d_flags + 1, 1, 0);
+            } else if ((rc = grow_lists(c, p, grow))) {
+                return rc;
             }
             if ((rc = prologue(c, p))) return rc;
             if (attempt > 8)
