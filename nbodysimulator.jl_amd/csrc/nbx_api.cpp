@@ -42,11 +42,12 @@ static void free_ptr(void* p) {
 static void release(nbx_ctx* c) {
     mx_release(c);
     void* const own[] = {c->d_base, c->d_mm, c->d_mm4, c->d_rdf_work, c->d_frac, c->d_rhs, c->d_water,
-                         c->d_frames, c->d_backup, c->d_sortbuf, c->d_permbuf};
+                         c->d_frames, c->d_backup, c->d_bins, c->d_sortbuf, c->d_permbuf};
     for (void* p : own) free_ptr(p);
     c->d_base = nullptr;
     c->d_rdf_work = c->d_rhs = c->d_water = c->d_frames = c->d_backup = c->d_permbuf = nullptr;
     c->d_frac = nullptr;
+    c->d_bins = nullptr;
     c->d_perm = c->d_iperm = c->d_pmap = nullptr;
     c->d_sortbuf = nullptr;
     c->sortbuf_bytes = 0;
@@ -175,6 +176,7 @@ static void invalidate(nbx_ctx* c) {
     c->nl.ready = false;
     c->list_sorted = false;
     c->every_chosen = false;
+    c->guarded = false;
     ++c->version;
 }
 
@@ -1255,8 +1257,9 @@ extern "C" int nbx_autotune(nbx_ctx* c, double dt, int32_t trial_steps, double* 
 
 extern "C" int nbx_get_stats(nbx_ctx* c, int64_t* out, int32_t nout) {
     if (!c || !out || nout < 0 || nout > 8) return NBX_ERR_INVALID;
-    int64_t v[8] = {0, c->nl.cap, c->nl.ncell, c->nl.lanes, c->graph_steps, c->build_every,
-                    c->stale_replays, c->sorts_applied};
+    int64_t v[8] = {0, c->nl.cap, c->nl.ncell, c->nl.lanes, c->graph_steps,
+                    c->every_auto && c->guarded ? 1 : c->build_every, c->stale_replays,
+                    c->sorts_applied};
     if (c->nl.d_flags) {
         int h[8] = {0};
         NBX_HIP(c, hipMemcpyAsync(h, c->nl.d_flags, sizeof(h), hipMemcpyDeviceToHost, c->stream));

@@ -17,7 +17,8 @@
 // belongs to the drift of the step after the state when a run has ended)
 enum { NBX_SCAL_T = 0, NBX_SCAL_ZETA = 10, NBX_SCAL_XI = 11, NBX_SCAL_XI_SCRATCH = 15,
        NBX_SCAL_ZETA_PREV = 16, NBX_SCAL_XI_PREV = 17, NBX_SCAL_COUNT = 32 };
-enum { NBX_BINS_STEP = 0, NBX_BINS_FIXED = 1, NBX_BINS_BUILD = 2, NBX_FLAG_BINSET = 5, NBX_FLAG_SPEED = 8, NBX_FLAGS = 16,
+enum { NBX_BINS_STEP = 0, NBX_BINS_FIXED = 1, NBX_BINS_BUILD = 2,
+       NBX_FLAG_BINSET = 5, NBX_FLAG_STALE = 7, NBX_FLAG_SPEED = 8, NBX_FLAGS = 16,
        // the flags' allocation: their line, then a line per group of the list build's blocks
        NBX_FLAGS_LINE = 32, NBX_BUILD_GROUPS = 32,
        NBX_FLAGS_INTS = NBX_FLAGS_LINE * (1 + NBX_BUILD_GROUPS) };
@@ -83,6 +84,7 @@ struct nbx_graph_key {
     const void* part = nullptr;
     int cap = 0, ccap = 0, ncell = 0, lanes = 0, steps = 0, chunks = 0, tpt = 0;
     int build_every = 1;      // steps between build opportunities
+    int guarded = 0;          // builds launched between them too
     int par_off = 0;          // buffer parity of the chunk step a replay starts after
     int em = 0;               // Euler-Maruyama steps instead of velocity Verlet
     const void* ids = nullptr;  // slot -> user atom map of a sorted state (nullptr: none)
@@ -92,7 +94,8 @@ struct nbx_graph_key {
                cell_atoms == o.cell_atoms && xref == o.xref && flags == o.flags && pos == o.pos &&
                part == o.part && cap == o.cap && ccap == o.ccap && ncell == o.ncell &&
                lanes == o.lanes && steps == o.steps && chunks == o.chunks && tpt == o.tpt &&
-               em == o.em && build_every == o.build_every && par_off == o.par_off &&
+               em == o.em && build_every == o.build_every && guarded == o.guarded &&
+               par_off == o.par_off &&
                ids == o.ids;
     }
 };
@@ -119,14 +122,17 @@ struct nbx_ctx {
     bool skin_set = false;
     // Verlet-list build opportunities every build_every steps (1, 2 or 5; the autotuner's
     // choice): the steps in between launch no build or binning kernel.  An atom that moves
-    // more than skin/2 between two opportunities invalidates the chunk, which is replayed
-    // with a build opportunity at every step.
+    // more than skin/2 between two opportunities invalidates the chunk, which is replayed:
+    // with build_every = 1 where the interval was set, guarded where it was chosen.
     int build_every = 1;
     bool every_auto = true;     // chosen from the speeds of a new state (not by
                                 // NBX_BUILD_EVERY or the autotuner)
     bool every_chosen = false;  // for the current state
     double speed2 = 0.0;        // largest squared speed when its lists were made
-    int64_t stale_replays = 0;  // chunks replayed because a list went stale (build_every -> 1)
+    // chosen interval: a list went stale in this configuration, and the steps between two
+    // opportunities launch builds too, which run where an atom has moved past skin/2
+    bool guarded = false;
+    int64_t stale_replays = 0;  // chunks replayed because a list went stale
     // device state: one allocation (d_base) holds d_x .. d_pmap
     char* d_base = nullptr;
     double* d_x = nullptr;    // positions (unwrapped), 3n
@@ -144,6 +150,8 @@ struct nbx_ctx {
     double* d_frames = nullptr;    // saved frames on their way to the host
     size_t frames_doubles = 0;
     double* d_backup = nullptr;    // mixed path: the state at the start of a chunk
+    uint64_t* d_bins = nullptr;    // and the bins made by the builds
+    size_t bins_bytes = 0;
     double* d_ms = nullptr;
     double* d_qs = nullptr;
     double* d_mm = nullptr;   // magnetic moments (SoA 3n), when set
@@ -344,9 +352,14 @@ int ref64_rdf_scratch(int device, unsigned long long** out);
 void ref64_zero_u64(hipStream_t s, unsigned long long* p, int64_t count);
 // sets d_flag[0] when a or b (count values each) holds NaN or Inf
 void ref64_check_finite(hipStream_t s, const double* a, const double* b, int64_t count, int* d_flag);
-// p[k] = value of five arrays in one launch: dst[0..3] of n3 doubles, dst[4] of nscal
-void ref64_copy_state(hipStream_t s, const double* const* src, double* const* dst, int64_t n3,
-                      int64_t nscal);
+// up to nine arrays of 8-byte words in one launch
+#define REF64_COPIES 9
+struct ref64_copies {
+    const uint64_t* src[REF64_COPIES];
+    uint64_t* dst[REF64_COPIES];
+    int64_t words[REF64_COPIES];   // 0: none
+};
+void ref64_copy_words(hipStream_t s, const ref64_copies& c);
 
 // x * 0 is 0 for finite x and NaN otherwise; eight running sums, no branch per value
 inline bool nbx_all_finite(const double* p, int64_t count) {

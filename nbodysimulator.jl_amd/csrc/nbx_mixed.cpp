@@ -124,6 +124,8 @@ void free_nl(nbx_nlist& nl) {
 
 int round_up(int x, int m) { return ((x + m - 1) / m) * m; }
 
+size_t int_pairs(size_t ints) { return (ints + 1) / 2; }
+
 int reset_flags(nbx_ctx* c) {
     if (!c->nl.d_flags) NBX_HIP(c, hipMalloc((void**)&c->nl.d_flags, sizeof(int) * NBX_FLAGS_INTS));
     mx_launch_fill_int(c->stream, c->nl.d_flags, NBX_FLAGS_INTS, 0);
@@ -211,9 +213,10 @@ int alloc_lists(nbx_ctx* c, const mx_plan& p, double grow) {
     const size_t nb = (nl.nbr_wide ? sizeof(int) : sizeof(uint16_t)) * (size_t)nl.cap * (size_t)n;
     if ((rc = list_buffer(c, &nl.d_nbr, &nl.nbr_bytes, nb)) ||
         (rc = list_buffer(c, &nl.d_nnb, &nl.nnb_bytes, sizeof(int) * (size_t)n)) ||
-        (rc = list_buffer(c, &nl.d_cell_count, &nl.count_bytes, sizeof(int) * 3 * std::max<size_t>(ncells, 1))) ||
+        // (the bins are copied by words of two ints)
+        (rc = list_buffer(c, &nl.d_cell_count, &nl.count_bytes, 8 * int_pairs(3 * std::max<size_t>(ncells, 1)))) ||
         (rc = list_buffer(c, &nl.d_cell_atoms, &nl.atoms_bytes,
-                          sizeof(int) * 3 * std::max<size_t>(ncells * (size_t)nl.ccap, 1))) ||
+                          8 * int_pairs(3 * std::max<size_t>(ncells * (size_t)nl.ccap, 1)))) ||
         (rc = list_buffer(c, &nl.d_xref, &nl.xref_bytes, sizeof(double) * 3 * (size_t)n)) ||
         (rc = reset_flags(c)))
         return rc;
@@ -270,12 +273,17 @@ double* xbuf(nbx_ctx* c, int par) { return par ? c->d_x2 : c->d_x; }
 void* pbuf(nbx_ctx* c, int par) { return par ? c->d_pos2 : c->d_pos; }
 // the rebuild request: set by the drift, consumed (and cleared) by the next build
 int* req_flag(nbx_ctx* c) { return c->nl.d_flags; }
+// set by the drift before a step without a build opportunity where an atom moved past skin/2
+int* stale_flag(nbx_ctx* c) { return c->nl.d_flags + NBX_FLAG_STALE; }
 // bins of the per-step and fixed modes (set 0; the rotating mode uses all three sets)
 int* bin_count(nbx_ctx* c) { return c->nl.d_cell_count; }
 int* bin_atoms(nbx_ctx* c) { return c->nl.d_cell_atoms; }
 
 // steps between list-build opportunities
 int build_every(const nbx_ctx* c) { return std::max(1, c->build_every); }
+
+// builds are launched on the steps between two opportunities too, gated by the stale flag
+bool guards(const nbx_ctx* c) { return c->every_auto && c->guarded && build_every(c) > 1; }
 
 mx_nh_params nh_params(const nbx_ctx* c, double dt, int advance) {
     mx_nh_params nh{};
@@ -350,14 +358,15 @@ mx_io make_io(nbx_ctx* c, const mx_plan& p, int par, int do_drift, double dt = 0
 }
 
 
-// after a kernel that wrote x into X[par_out]: bins for a requested list build (the
-// thermostat temperature of vh, and the Nose-Hoover update, are finished by the last
-// block of that kernel: mx_epilogue)
-void after_drift(nbx_ctx* c, const mx_plan& p, int par_out) {
+// after a kernel that wrote x into X[par_out]: bins for a requested list build, or for one
+// that the stale flag asks for (the thermostat temperature of vh, and the Nose-Hoover update,
+// are finished by the last block of that kernel: mx_epilogue)
+void after_drift(nbx_ctx* c, const mx_plan& p, int par_out, bool next_opp) {
     hipStream_t s = c->stream;
     if (p.kind != PLAN_GRAVITY && p.nb.mode_list && c->nl.ncell >= 3 &&
-        c->nl.bin_mode == NBX_BINS_STEP)
-        mx_launch_bin(s, c, pbuf(c, par_out), req_flag(c), bin_count(c), bin_atoms(c));
+        c->nl.bin_mode == NBX_BINS_STEP && (next_opp || guards(c)))
+        mx_launch_bin(s, c, pbuf(c, par_out), next_opp ? req_flag(c) : stale_flag(c), bin_count(c),
+                      bin_atoms(c));
 }
 
 // the next pair of force-kernel timing events, when timing is on and the pool has room
@@ -399,17 +408,18 @@ void launch_step(nbx_ctx* c, const mx_plan& p, const mx_kick_params& kp, int par
         }
     }
     if (io.need_T && !fold) mx_launch_temperature_finish(s, io);
-    if (do_drift && next_opp) after_drift(c, p, par ^ 1);
+    if (do_drift) after_drift(c, p, par ^ 1, next_opp);
 }
 
-void launch_build(nbx_ctx* c, const mx_plan& p, int par) {
+// gate: the request, or the stale flag on the steps between two opportunities
+void launch_build(nbx_ctx* c, const mx_plan& p, int par, int* gate) {
     if (p.kind == PLAN_GRAVITY || !p.nb.mode_list) return;
     // 3 cells per side: the 27 neighbour cells are the whole box, so any partition of
     // the atoms into home cells finds every neighbour -- the bins made at set-up serve
     // every build and no step bins
     // per-step bins are cleared by the build that used them, ready for the next binning
     const int clear = c->nl.bin_mode == NBX_BINS_STEP && c->nl.ncell >= 3 ? 1 : 0;
-    mx_launch_build(c->stream, c, p.nb.water, pbuf(c, par), xbuf(c, par), req_flag(c),
+    mx_launch_build(c->stream, c, p.nb.water, pbuf(c, par), xbuf(c, par), gate,
                     bin_count(c), bin_atoms(c), clear);
 }
 
@@ -480,7 +490,7 @@ static int prologue(nbx_ctx* c, mx_plan& p) {
     if (p.kind != PLAN_GRAVITY && p.nb.mode_list)
         mx_launch_max_speed(s, c->d_v, c->n,
                             reinterpret_cast<unsigned long long*>(c->nl.d_flags + NBX_FLAG_SPEED));
-    launch_build(c, p, 0);
+    launch_build(c, p, 0, req_flag(c));
     launch_step(c, p, kick_params(c, 0, 0.0, 0), 0, 0);
     NBX_HIP(c, hipGetLastError());
     c->accel_valid = true;
@@ -500,16 +510,16 @@ static int read_flags(nbx_ctx* c, int* h) {
 // 2 to 3 us; the earlier requests of M = 5 rebuild about half as often again (whole runs:
 // Lennard-Jones, n = 32,000, 250 steps of 0.002 4.13 -> 3.98 ms, n = 864 with the lanes by
 // size, 300 steps 2.82 -> 1.86 ms).  A state that speeds up past it marks a list stale and is
-// replayed with M = 1, as with any interval, at twice the cost: water without a thermostat,
-// whose bonds do that to many a state (519 molecules, 102 steps 7.3 ms with M = 1, 15.5
-// replayed), takes M = 1.
+// replayed guarded (mx_vv_run), at twice the cost: water without a thermostat, whose bonds do
+// that to many a state (519 molecules, 102 steps 7.3 ms with M = 1, 15.5 replayed), takes
+// M = 1.  M follows from the state, the time step and the configuration alone, so equal
+// calls run equal steps.
 static void choose_build_every(nbx_ctx* c, const mx_plan& p, double dt) {
     if (!c->every_auto || c->every_chosen || p.kind == PLAN_GRAVITY || !p.nb.mode_list) return;
     c->every_chosen = true;
     c->build_every = 1;
-    // strained bonds speed up atoms that nothing cools; a context that had a list go stale
-    // keeps M = 1
-    if ((p.nb.water && c->therm == NBX_THERM_NONE) || c->stale_replays > 0) return;
+    // strained bonds speed up atoms that nothing cools
+    if (p.nb.water && c->therm == NBX_THERM_NONE) return;
     double v2 = c->speed2;
     if (c->therm != NBX_THERM_NONE && c->n > 0)
         v2 = std::max(v2, 25.0 * c->kb * c->therm_T * c->mass_wmin);
@@ -610,7 +620,7 @@ static int rebuild_list(nbx_ctx* c, mx_plan& p) {
     double grow = 1.0;
     for (int attempt = 0;; ++attempt) {
         refresh_positions(c, p, true);
-        launch_build(c, p, 0);
+        launch_build(c, p, 0, req_flag(c));
         NBX_HIP(c, hipGetLastError());
         int h[NBX_FLAGS];
         if ((rc = read_flags(c, h))) return rc;
@@ -618,6 +628,34 @@ static int rebuild_list(nbx_ctx* c, mx_plan& p) {
         if (attempt > 8) return nbx_fail(c, NBX_ERR_CAPACITY, "list overflow persists");
         if ((rc = grow_lists(c, p, grow))) return rc;
     }
+}
+
+// The list of a chunk's start once more, from the positions xref that it was built for: the
+// same entries, since a build is a function of its positions and bins.  Per-step bins are made
+// of the positions, fixed bins stay; bins made by the builds (restored with the flags) step
+// back to the set that the list's build read, and that build fills the current set again.  The
+// caller restores the flags afterwards.
+static int remake_list(nbx_ctx* c, const mx_plan& p, const double* xref) {
+    hipStream_t s = c->stream;
+    nbx_nlist& nl = c->nl;
+    const size_t ncells = (size_t)nl.ncell * nl.ncell * nl.ncell;
+    const bool step_bins = nl.ncell >= 3 && nl.bin_mode == NBX_BINS_STEP;
+    if (step_bins) {
+        mx_launch_fill_int(s, nl.d_cell_count, (int64_t)(3 * ncells), 0);
+    } else if (nl.bin_mode == NBX_BINS_BUILD) {
+        int h[NBX_FLAGS], rc;
+        if ((rc = read_flags(c, h))) return rc;
+        const int set = h[NBX_FLAG_BINSET];
+        mx_launch_fill_int(s, nl.d_cell_count + (size_t)set * ncells, (int64_t)ncells, 0);
+        mx_launch_fill_int(s, nl.d_flags + NBX_FLAG_BINSET, 1, (set + 2) % 3);
+    }
+    mx_launch_positions(s, c, xref, c->d_pos, pos_kind(p), mass_wscale(c, p),
+                        step_bins ? bin_count(c) : nullptr, step_bins ? bin_atoms(c) : nullptr,
+                        req_flag(c));
+    mx_launch_build(s, c, p.nb.water, c->d_pos, xref, req_flag(c), bin_count(c), bin_atoms(c),
+                    step_bins ? 1 : 0);
+    NBX_HIP(c, hipGetLastError());
+    return NBX_OK;
 }
 
 // a new sorted order from the current positions: slots by cell of the list grid
@@ -709,11 +747,41 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
     // the chunk's start is kept for a replay where a list can overflow or go stale (the plans
     // without lists never replay)
     const bool lists = !all_pairs_tiled(p) && p.nb.mode_list;
+    constexpr int64_t flag_words = NBX_FLAGS / 2;
     if (lists && !c->d_backup)
-        NBX_HIP(c, hipMalloc((void**)&c->d_backup, sizeof(double) * (4 * n3 + NBX_SCAL_COUNT)));
+        NBX_HIP(c, hipMalloc((void**)&c->d_backup,
+                             sizeof(double) * (5 * n3 + NBX_SCAL_COUNT + flag_words)));
     double* const bk = c->d_backup;
-    double* const bkp[5] = {bk, bk + n3, bk + 2 * n3, bk + 3 * n3, bk + 4 * n3};
-    double* const live[5] = {c->d_x, c->d_v, c->d_a, c->d_vh, c->d_scal};
+    double* const bkp[7] = {bk, bk + n3, bk + 2 * n3, bk + 3 * n3, bk + 4 * n3, bk + 5 * n3,
+                            bk + 5 * n3 + NBX_SCAL_COUNT};   // x v a vh xref scalars flags
+    // the chunk's start into the backup, or back.  With a chosen interval (whose replay
+    // continues from the list of the chunk's start) also what that list was made from: the
+    // positions it was built for, the flags, and the bins that the builds made
+    const auto copy_chunk = [&](bool save, bool with_list) -> int {
+        ref64_copies cp{};
+        int k = 0;
+        const auto add = [&](void* live, void* kept, size_t words) {
+            cp.src[k] = static_cast<const uint64_t*>(save ? live : kept);
+            cp.dst[k] = static_cast<uint64_t*>(save ? kept : live);
+            cp.words[k++] = (int64_t)words;
+        };
+        double* const live[4] = {c->d_x, c->d_v, c->d_a, c->d_vh};
+        for (int q = 0; q < 4; ++q) add(live[q], bkp[q], n3);
+        add(c->d_scal, bkp[5], NBX_SCAL_COUNT);
+        if (with_list) {
+            add(c->nl.d_xref, bkp[4], n3);
+            add(c->nl.d_flags, bkp[6], flag_words);
+            if (c->nl.bin_mode == NBX_BINS_BUILD) {
+                const size_t ncells = (size_t)c->nl.ncell * c->nl.ncell * c->nl.ncell;
+                const size_t wc = int_pairs(3 * ncells), wa = int_pairs(3 * ncells * (size_t)c->nl.ccap);
+                if (int e = list_buffer(c, &c->d_bins, &c->bins_bytes, 8 * (wc + wa))) return e;
+                add(c->nl.d_cell_count, c->d_bins, wc);
+                add(c->nl.d_cell_atoms, c->d_bins + wc, wa);
+            }
+        }
+        ref64_copy_words(s, cp);
+        return NBX_OK;
+    };
     const int64_t chunk_max = 500;
     while (c->kt_on && c->kt_ev.size() < 2 * (size_t)chunk_max) {
         hipEvent_t e = nullptr;
@@ -739,7 +807,8 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
             kp.step_base = c->d_step;
             kp.step_off = k - k0;
             kp.ids = sorting ? c->d_perm : nullptr;
-            if ((base + k - 1) % M == 0) launch_build(c, p, par);
+            if ((base + k - 1) % M == 0) launch_build(c, p, par, req_flag(c));
+            else if (guards(c)) launch_build(c, p, par, stale_flag(c));
             launch_step(c, p, kp, par, 1, true, ((base + k) % M == 0 || k == last) ? 1 : 0);
         }
         mx_launch_step_advance(s, c->d_step, count, 0);
@@ -767,6 +836,7 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
         key.lanes = c->nl.lanes;
         key.steps = gsteps;
         key.build_every = build_every(c);
+        key.guarded = guards(c) ? 1 : 0;
         key.par_off = par_off;
         key.ids = sorting ? c->d_perm : nullptr;
         if (c->gexec && key == c->gkey) { *out = c->gexec; return NBX_OK; }
@@ -801,7 +871,9 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
             }
             chunk = std::min(chunk, S - t0 % S);
         }
-        if (lists) ref64_copy_state(s, live, bkp, (int64_t)n3, NBX_SCAL_COUNT);
+        // a guarded run needs no list to go back to: it is never stale
+        const bool keep_list = lists && c->every_auto && build_every(c) > 1 && !guards(c);
+        if (lists && (rc = copy_chunk(true, keep_list))) return rc;
         const int64_t step0 = c->steps_taken;
         for (int attempt = 0;; ++attempt) {
             mx_launch_step_advance(s, c->d_step, step0, 1);
@@ -825,7 +897,7 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
                 if (c->nh_advanced) io0.nh.advance = 0;
                 mx_launch_drift(s, c, kp, io0);
                 if (io0.need_T && !folds_temperature(c, p)) mx_launch_temperature_finish(s, io0);
-                if (first_opp) after_drift(c, p, 1);
+                after_drift(c, p, 1, first_opp);
             }
             const int gs = c->graph_steps;
             const int64_t M = build_every(c);
@@ -847,7 +919,7 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
             if (lists || c->kt_on) {   // kernel timing reads its events next
                 if ((rc = read_flags(c, h))) return rc;
             }
-            if (!h[1] && !h[7]) {
+            if (!h[1] && !h[NBX_FLAG_STALE]) {
                 // the chunk stands: add its force-kernel times (the stream has drained)
                 for (size_t k = 0; k + 1 < c->kt_used; k += 2) {
                     float ms = 0.f;
@@ -861,20 +933,37 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
                 break;
             }
             c->kt_used = 0;   // replayed: its timings are dropped
-            // a list that went stale between two build opportunities: restore and replay with
-            // an opportunity at every step; overflow: restore and replay with larger lists.
-            // Stale first: the steps after it ran on a list that misses pairs, and what they
-            // overflowed (the builds' bins are flagged past 3/4 skin) larger lists do not mend
-            ref64_copy_state(s, bkp, live, (int64_t)n3, NBX_SCAL_COUNT);
-            if (h[7]) {
+            // a list that went stale between two build opportunities: restore and replay;
+            // overflow: restore and replay with larger lists.  Stale first: the steps after it
+            // ran on a list that misses pairs, and what they overflowed (the builds' bins are
+            // flagged past 3/4 skin) larger lists do not mend
+            if (h[NBX_FLAG_STALE] && keep_list && !c->guarded) {
+                // chosen interval: the chunk again from its own list, guarded.  Up to the step
+                // before the list went stale these are the steps just taken, bit for bit, and
+                // from there on those of any other chunk that holds that step: where runs are
+                // split and frames are saved leaves no trace
+                if ((rc = copy_chunk(false, true)) || (rc = remake_list(c, p, bkp[4]))) return rc;
+                ref64_copies fl{};
+                fl.src[0] = reinterpret_cast<const uint64_t*>(bkp[6]);
+                fl.dst[0] = reinterpret_cast<uint64_t*>(c->nl.d_flags);
+                fl.words[0] = flag_words;
+                ref64_copy_words(s, fl);
+                c->guarded = true;
+                ++c->stale_replays;
+                continue;
+            }
+            if ((rc = copy_chunk(false, false))) return rc;
+            if (h[NBX_FLAG_STALE]) {
+                // set interval: an opportunity at every step from the chunk's start
                 c->build_every = 1;
                 ++c->stale_replays;
-                mx_launch_fill_int(s, c->nl.d_flags + 7, 1, 0);
+                mx_launch_fill_int(s, stale_flag(c), 1, 0);
                 mx_launch_fill_int(s, c->nl.d_flags + 1, 1, 0);
             } else if ((rc = grow_lists(c, p, grow))) {
                 return rc;
             }
             if ((rc = prologue(c, p))) return rc;
+            if (keep_list && (rc = copy_chunk(true, true))) return rc;   // the larger lists
             if (attempt > 8)
                 return nbx_fail(c, NBX_ERR_CAPACITY, "list overflow replay did not converge");
         }
@@ -1040,7 +1129,7 @@ int fresh_list(nbx_ctx* c, mx_plan& p) {
     if ((rc = ensure_ready(c, p))) return rc;
     for (int attempt = 0;; ++attempt) {
         refresh_positions(c, p, true);
-        launch_build(c, p, 0);
+        launch_build(c, p, 0, req_flag(c));
         NBX_HIP(c, hipGetLastError());
         int h[NBX_FLAGS];
         if ((rc = read_flags(c, h))) return rc;
@@ -1255,7 +1344,7 @@ int mx_learned_run(nbx_ctx* c, const nbx_model* m, double dt, int stride, int64_
         ip.part = mpart.as<double>();
         lr_launch_mlp_infer(s, ip);
         lr_launch_drift(s, mpart.as<double>(), nblk, dlab.as<float>(), D, make_io(c, p, par, 1, D), n);
-        after_drift(c, p, par ^ 1);
+        after_drift(c, p, par ^ 1, true);
     };
     auto run_chunk = [&](int64_t msteps) -> int {
         int rc2;
@@ -1265,7 +1354,7 @@ int mx_learned_run(nbx_ctx* c, const nbx_model* m, double dt, int stride, int64_
         const mx_kick_params kp = kick_params(c, 1, D, 0);
         for (int64_t k = 1; k <= msteps; ++k) {
             const int par = (int)(k & 1);
-            launch_build(c, p, par);
+            launch_build(c, p, par, req_flag(c));
             launch_step(c, p, kp, par, 0);
             start_step(par);
         }
@@ -1576,11 +1665,13 @@ int mx_autotune(nbx_ctx* c, double dt, int trial, double* out, int nout) {
         const double skin0 = c->skin;
         const bool skin_set0 = c->skin_set;
         const bool lanes_auto0 = c->nl.lanes_auto, every_auto0 = c->every_auto;
+        c->guarded = false;
         if ((rc = time_config(&base_ms))) return rc;
         best_ms = base_ms;
         best0 = c->nl.lanes;
         best1 = c->nl.skin;
-        best2 = build_every(c);
+        best2 = guards(c) ? 1 : build_every(c);
+        c->guarded = false;
         const int lanes_c[5] = {2, 4, 8, 16, 32};
         const double skin_c[8] = {0.06, 0.09, 0.12, 0.15, 0.18, 0.24, 0.32, 0.40};
         const int every_c[3] = {1, 2, 5};

@@ -237,7 +237,7 @@ __device__ __forceinline__ void mx_store_position(int64_t i, int64_t n, double p
         const double e2 = ex * ex + ey * ey + ez * ez;
         if (e2 > io.half_skin2) io.req_out[0] = 1;
         if (e2 > io.guard2) io.flags[1] = 1;
-        if (!io.next_opp && e2 > io.stale2) io.flags[7] = 1;
+        if (!io.next_opp && e2 > io.stale2) io.flags[NBX_FLAG_STALE] = 1;
     }
 }
 
@@ -348,7 +348,7 @@ __device__ __forceinline__ void mx_store_component(int64_t i, int c, int64_t n, 
         if (act && c == 0) {
             if (r2 > io.half_skin2) io.req_out[0] = 1;
             if (r2 > io.guard2) io.flags[1] = 1;
-            if (!io.next_opp && r2 > io.stale2) io.flags[7] = 1;
+            if (!io.next_opp && r2 > io.stale2) io.flags[NBX_FLAG_STALE] = 1;
         }
     }
 }

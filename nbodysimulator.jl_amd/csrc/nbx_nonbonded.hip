@@ -939,7 +939,8 @@ k_build_cells(const double4* __restrict__ pos, const double* __restrict__ x, int
     if (tid == 0) {
         state[1] = 0;
         if (rotate) state[0] = (bset + 1) % 3;
-        req[0] = 0;
+        req[0] = 0;     // the request, or the stale flag of a build between two opportunities,
+        flags[0] = 0;   // which serves the request as well
     }
 }
 
@@ -997,6 +998,7 @@ k_build_allpairs(const double4* __restrict__ pos, const double* __restrict__ x, 
     if (last && threadIdx.x == 0) {
         flags[NBX_FLAG_BINSET + 1] = 0;
         req[0] = 0;
+        flags[0] = 0;   // as in k_build_cells
     }
 }
 

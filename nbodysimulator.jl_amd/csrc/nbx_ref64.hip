@@ -1738,27 +1738,18 @@ void ref64_check_finite(hipStream_t s, const double* a, const double* b, int64_t
                        d_flag);
 }
 
-struct ref_copies {
-    const double* src[5];
-    double* dst[5];
-};
-
 __global__ void __launch_bounds__(256)
-k_copy_state(ref_copies c, int64_t n3, int64_t nscal) {
+k_copy_words(ref64_copies c) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n3) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) c.dst[k][t] = c.src[k][t];
-    }
-    if (t < nscal) c.dst[4][t] = c.src[4][t];
+    for (int k = 0; k < REF64_COPIES; ++k)
+        if (t < c.words[k]) c.dst[k][t] = c.src[k][t];
 }
 
-void ref64_copy_state(hipStream_t s, const double* const* src, double* const* dst, int64_t n3,
-                      int64_t nscal) {
-    ref_copies c{};
-    for (int k = 0; k < 5; ++k) { c.src[k] = src[k]; c.dst[k] = dst[k]; }
-    hipLaunchKernelGGL(k_copy_state, dim3(nbx_blocks(std::max(n3, nscal), 256)), dim3(256), 0, s, c,
-                       n3, nscal);
+void ref64_copy_words(hipStream_t s, const ref64_copies& c) {
+    const int64_t most = *std::max_element(c.words, c.words + REF64_COPIES);
+    if (most <= 0) return;
+    hipLaunchKernelGGL(k_copy_words, dim3(nbx_blocks(most, 256)), dim3(256), 0, s, c);
 }
 
 // ---------------------------------------------------------------------------
