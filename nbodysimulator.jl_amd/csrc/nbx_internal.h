@@ -127,8 +127,10 @@ struct nbx_ctx {
     int build_every = 1;
     bool every_auto = true;     // chosen from the speeds of a new state (not by
                                 // NBX_BUILD_EVERY or the autotuner)
-    bool every_chosen = false;  // for the current state
-    double speed2 = 0.0;        // largest squared speed when its lists were made
+    bool every_chosen = false;  // for the current state and the time step every_dt
+    double every_dt = 0.0;
+    double speed2 = 0.0;        // largest squared speed, and the step it was measured at
+    int64_t speed_step = 0;
     // chosen interval: a list went stale in this configuration, and the steps between two
     // opportunities launch builds too, which run where an atom has moved past skin/2
     bool guarded = false;

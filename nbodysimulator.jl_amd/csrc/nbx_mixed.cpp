@@ -477,6 +477,12 @@ static void refresh_positions(nbx_ctx* c, const mx_plan& p, bool bins) {
                         (pk == 1 && bins) ? req_flag(c) : nullptr);
 }
 
+// the largest squared speed into the flags (over what they hold)
+static void measure_speed(nbx_ctx* c) {
+    mx_launch_max_speed(c->stream, c->d_v, c->n,
+                        reinterpret_cast<unsigned long long*>(c->nl.d_flags + NBX_FLAG_SPEED));
+}
+
 // a = f(x, v) at the current state (no step taken)
 static int prologue(nbx_ctx* c, mx_plan& p) {
     hipStream_t s = c->stream;
@@ -487,9 +493,7 @@ static int prologue(nbx_ctx* c, mx_plan& p) {
     // the Berendsen term of the first evaluation uses v itself (vh := v)
     NBX_HIP(c, hipMemcpyAsync(c->d_vh, c->d_v, sizeof(double) * 3 * (size_t)c->n,
                               hipMemcpyDeviceToDevice, s));
-    if (p.kind != PLAN_GRAVITY && p.nb.mode_list)
-        mx_launch_max_speed(s, c->d_v, c->n,
-                            reinterpret_cast<unsigned long long*>(c->nl.d_flags + NBX_FLAG_SPEED));
+    if (p.kind != PLAN_GRAVITY && p.nb.mode_list) measure_speed(c);
     launch_build(c, p, 0, req_flag(c));
     launch_step(c, p, kick_params(c, 0, 0.0, 0), 0, 0);
     NBX_HIP(c, hipGetLastError());
@@ -514,12 +518,29 @@ static int read_flags(nbx_ctx* c, int* h) {
 // that to many a state (519 molecules, 102 steps 7.3 ms with M = 1, 15.5 replayed), takes
 // M = 1.  M follows from the state, the time step and the configuration alone, so equal
 // calls run equal steps.
-static void choose_build_every(nbx_ctx* c, const mx_plan& p, double dt) {
-    if (!c->every_auto || c->every_chosen || p.kind == PLAN_GRAVITY || !p.nb.mode_list) return;
+// Another time step chooses again; speeds older than 100 steps are measured again (a kernel
+// and a wait, which a caller that changes the step on every call does not pay each time).
+// *relist: the interval has grown, and a list made for a shorter one may hold atoms nearly
+// skin/2 away, with no opportunity for some steps.
+static int choose_build_every(nbx_ctx* c, const mx_plan& p, double dt, bool* relist) {
+    *relist = false;
+    if (!c->every_auto || p.kind == PLAN_GRAVITY || !p.nb.mode_list) return NBX_OK;
+    if (c->every_chosen && c->every_dt == dt) return NBX_OK;
+    const bool again = c->every_chosen;
+    const int before = build_every(c);
     c->every_chosen = true;
+    c->every_dt = dt;
     c->build_every = 1;
     // strained bonds speed up atoms that nothing cools
-    if (p.nb.water && c->therm == NBX_THERM_NONE) return;
+    if (p.nb.water && c->therm == NBX_THERM_NONE) return NBX_OK;
+    if (again && c->steps_taken - c->speed_step >= 100) {
+        int h[NBX_FLAGS], rc;
+        mx_launch_fill_int(c->stream, c->nl.d_flags + NBX_FLAG_SPEED, 2, 0);
+        measure_speed(c);
+        if ((rc = read_flags(c, h))) return rc;
+        std::memcpy(&c->speed2, h + NBX_FLAG_SPEED, sizeof(double));
+        c->speed_step = c->steps_taken;
+    }
     double v2 = c->speed2;
     if (c->therm != NBX_THERM_NONE && c->n > 0)
         v2 = std::max(v2, 25.0 * c->kb * c->therm_T * c->mass_wmin);
@@ -529,6 +550,8 @@ static void choose_build_every(nbx_ctx* c, const mx_plan& p, double dt) {
             c->build_every = M;
             break;
         }
+    *relist = again && c->build_every > before;
+    return NBX_OK;
 }
 
 static int grow_lists(nbx_ctx* c, mx_plan& p, double& grow) {
@@ -566,6 +589,7 @@ static int ensure_ready(nbx_ctx* c, mx_plan& p, bool run = false) {
             if ((rc = read_flags(c, h))) return rc;
         }
         std::memcpy(&c->speed2, h + NBX_FLAG_SPEED, sizeof(double));
+        c->speed_step = c->steps_taken;
         return NBX_OK;
     }
     std::string why;
@@ -715,7 +739,8 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
     mx_plan p;
     int rc;
     if ((rc = ensure_ready(c, p, true))) return rc;
-    choose_build_every(c, p, dt);
+    bool relist = false;
+    if ((rc = choose_build_every(c, p, dt, &relist))) return rc;
     // the run keeps the state in the sorted order and returns it in the user's order
     const bool sorting = allow_sort && sort_enabled(c, p);
     struct order_guard {
@@ -730,15 +755,18 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
         if (!c->perm_identity) {
             if ((rc = permute_state(c, c->d_perm))) return rc;
             og.c = c;
-            if (!c->list_sorted && (rc = rebuild_list(c, p))) return rc;
+            if ((!c->list_sorted || relist) && (rc = rebuild_list(c, p))) return rc;
         } else {
             og.c = c;
+            if (relist && (rc = rebuild_list(c, p))) return rc;
         }
     } else if (!c->perm_identity || c->list_sorted) {
         // not sorted from here on (an internal caller, or the plan no longer sorts): the
         // state is in the user's order, the list was made for the sorted one
         if ((rc = mx_reset_order(c))) return rc;
         if ((rc = rebuild_list(c, p))) return rc;
+    } else if (relist && (rc = rebuild_list(c, p))) {
+        return rc;
     }
     double grow = 1.0;
     hipStream_t s = c->stream;

@@ -108,3 +108,39 @@ def test_lanes_of_water(nbx):
         ctx = water_ctx(per_side)
         ctx.vv_run(0.0005, 1)
         assert ctx.stats()["lanes"] == lanes
+
+
+def test_another_time_step_chooses_again(nbx):
+    s = gen.lj_liquid(6, rho=0.8442, T=0.5, seed=3)
+    speed = float(np.sqrt((s.v ** 2).sum(1)).max())
+    small, large = 1e-4, 0.03 / speed   # M = 5; past M = 2
+    assert expected_every(0.8 * speed, large, 0.3) == 1 and expected_every(2 * speed, small, 0.3) == 5
+    print("[case] small step, then a large one", flush=True)
+    ctx = lj_ctx(s.u, s.v, s.L)
+    ctx.vv_run(small, 8)
+    assert ctx.stats()["build_every"] == 5
+    ctx.vv_run(large, 3)
+    st = ctx.stats()
+    assert st["build_every"] == 1 and st["stale_replays"] == 0
+    print("[case] and back", flush=True)
+    ctx.vv_run(small, 20)
+    st = ctx.stats()
+    assert st["build_every"] == 5 and st["stale_replays"] == 0
+
+
+def test_another_time_step_looks_at_the_speeds_again(nbx):
+    s = gen.lj_liquid(6, rho=0.8442, T=0.1, seed=3)
+    ctx = lj_ctx(s.u, s.v, s.L)
+    d = s.u - s.u[0]
+    d -= s.L * np.rint(d / s.L)
+    r = np.sqrt((d ** 2).sum(1))
+    r[0] = np.inf
+    s.u[r.argmin()] = s.u[0] + 0.75 * d[r.argmin()] / r.min()   # two atoms thrown apart
+    ctx.set_state(s.u, 0 * s.v)
+    print("[case] at rest, then moving", flush=True)
+    ctx.vv_run(1e-4, 100)
+    assert ctx.stats()["build_every"] == 5
+    speed = float(np.sqrt((ctx.get_state()[1] ** 2).sum(1)).max())
+    assert speed > 4.0
+    ctx.vv_run(2e-3, 1)
+    assert ctx.stats()["build_every"] == expected_every(speed, 2e-3, 0.3) < 5
