@@ -311,9 +311,9 @@ bool folds_temperature(const nbx_ctx* c, const mx_plan& p) {
 }
 
 // buffers of a launch that reads x in X[par] and (when drifting) writes X[par ^ 1];
-// next_opp: the next step has a build opportunity
-mx_io make_io(nbx_ctx* c, const mx_plan& p, int par, int do_drift, double dt = 0.0,
-              int next_opp = 1) {
+// next_opp: the next step has a build opportunity, M: steps between two of them
+mx_io make_io(nbx_ctx* c, const mx_plan& p, int par, int do_drift, double dt, int next_opp,
+              int M) {
     mx_io io{};
     io.x_in = xbuf(c, par);
     io.x_out = xbuf(c, par ^ 1);
@@ -332,7 +332,6 @@ mx_io make_io(nbx_ctx* c, const mx_plan& p, int par, int do_drift, double dt = 0
         // with a build opportunity every M steps a rebuild is requested at
         // (skin/2)(1 - (M-1)/(2M)), so that the M-1 steps to the next opportunity rarely take
         // an atom past skin/2; one that does marks the chunk stale (replayed with M = 1)
-        const int M = build_every(c);
         const double trig = 0.5 * c->nl.skin * (1.0 - (double)(M - 1) / (2.0 * M));
         io.xref = c->nl.d_xref;
         io.half_skin2 = trig * trig;
@@ -383,7 +382,7 @@ void timing_events(nbx_ctx* c, hipEvent_t* e0, hipEvent_t* e1) {
 void launch_step(nbx_ctx* c, const mx_plan& p, const mx_kick_params& kp, int par, int do_drift,
                  bool timed = false, int next_opp = 1) {
     hipStream_t s = c->stream;
-    const mx_io io = make_io(c, p, par, do_drift, kp.dt, next_opp);
+    const mx_io io = make_io(c, p, par, do_drift, kp.dt, next_opp, build_every(c));
     // the step's kick takes the temperature of the drift before it from its partials
     const bool fold = kp.do_kick && folds_temperature(c, p);
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -920,7 +919,7 @@ static int mx_vv_run(nbx_ctx* c, double dt, int64_t nsteps, uint64_t seed, int64
                 kp.step_off = 0;
                 kp.ids = sorting ? c->d_perm : nullptr;
                 const int first_opp = (step0 % build_every(c)) == 0 ? 1 : 0;
-                mx_io io0 = make_io(c, p, 0, 1, dt, first_opp);
+                mx_io io0 = make_io(c, p, 0, 1, dt, first_opp, build_every(c));
                 // a redone drift recomputes xi but leaves zeta as its first pass left it
                 if (c->nh_advanced) io0.nh.advance = 0;
                 mx_launch_drift(s, c, kp, io0);
@@ -1042,7 +1041,7 @@ int mx_time_force(nbx_ctx* c, int iters, double* avg_ms, const char** name) {
     hipStream_t s = c->stream;
     refresh_positions(c, p, false);  // P[0] <- X[0] (the list stays valid for it)
     const mx_kick_params kp = kick_params(c, 0, 0.0, 0);
-    const mx_io io = make_io(c, p, 0, 0);
+    const mx_io io = make_io(c, p, 0, 0, 0.0, 1, build_every(c));
     mx_nb_launch nb = p.nb;
     nb.lanes = c->nl.lanes;
     auto launch = [&]() {
@@ -1353,6 +1352,9 @@ int mx_learned_run(nbx_ctx* c, const nbx_model* m, double dt, int stride, int64_
     const int builds0 = hflags[2];
     const double D = dt * stride;
     const int nblk = lr_infer_blocks(n);
+    // every strided step has a build opportunity: a rebuild is requested at skin/2, whatever
+    // interval a plain run chose (an interval that was set keeps its earlier request)
+    const int M = c->every_auto ? 1 : build_every(c);
 
     // the corrected start of a strided step from the state in X[par] / P[par]
     auto start_step = [&](int par) {
@@ -1371,7 +1373,8 @@ int mx_learned_run(nbx_ctx* c, const nbx_model* m, double dt, int stride, int64_
         ip.dlab = dlab.as<float>();
         ip.part = mpart.as<double>();
         lr_launch_mlp_infer(s, ip);
-        lr_launch_drift(s, mpart.as<double>(), nblk, dlab.as<float>(), D, make_io(c, p, par, 1, D), n);
+        lr_launch_drift(s, mpart.as<double>(), nblk, dlab.as<float>(), D,
+                        make_io(c, p, par, 1, D, 1, M), n);
         after_drift(c, p, par ^ 1, true);
     };
     auto run_chunk = [&](int64_t msteps) -> int {

@@ -9,6 +9,7 @@ import pytest
 
 from nbodysimulator import _lib
 from nbodysimulator import generators as gen
+from oracle import mlp_oracle as M
 
 pytestmark = pytest.mark.gpu
 
@@ -144,3 +145,23 @@ def test_another_time_step_looks_at_the_speeds_again(nbx):
     assert speed > 4.0
     ctx.vv_run(2e-3, 1)
     assert ctx.stats()["build_every"] == expected_every(speed, 2e-3, 0.3) < 5
+
+
+def test_learned_run_keeps_its_own_request(nbx):
+    """A learned run has a build opportunity at every step: the interval that a plain run
+    before it chose changes neither its lists nor its steps."""
+    got = []
+    for plain in (False, True):
+        print(f"[case] learned run, after a plain one: {plain}", flush=True)
+        s = gen.lj_liquid(5, rho=0.8442, T=0.9, seed=6)
+        ctx = lj_ctx(s.u, s.v, s.L)
+        if plain:
+            ctx.vv_run(1e-4, 0)
+            assert ctx.stats()["build_every"] == 5
+        m = _lib.Model(0)
+        m.set(np.zeros(M.NPARAM), np.concatenate([np.zeros(35), np.ones(35), np.ones(6)]))
+        rep = ctx.learned_run(m, 0.005, 4, 80, drift_tol=1.0, check_every=40)
+        assert rep["strided_steps"] == 80
+        got.append((rep["list_builds"], *ctx.get_state()))
+    assert got[0][0] == got[1][0]
+    assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2])
