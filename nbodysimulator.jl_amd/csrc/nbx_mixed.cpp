@@ -544,8 +544,10 @@ static int choose_build_every(nbx_ctx* c, const mx_plan& p, double dt, bool* rel
     if (c->therm != NBX_THERM_NONE && c->n > 0)
         v2 = std::max(v2, 25.0 * c->kb * c->therm_T * c->mass_wmin);
     const double reach = 1.25 * std::sqrt(v2) * dt;
+    const int gs = c->graph_steps;
     for (int M : {5, 2})
-        if (reach * M <= 0.5 * c->nl.skin * (double)(M - 1) / (2.0 * M)) {
+        if ((gs <= 0 || gs % 2 != 0 || gs % M == 0) &&   // blocks that are replayed hold whole intervals
+            reach * M <= 0.5 * c->nl.skin * (double)(M - 1) / (2.0 * M)) {
             c->build_every = M;
             break;
         }

@@ -165,3 +165,14 @@ def test_learned_run_keeps_its_own_request(nbx):
         got.append((rep["list_builds"], *ctx.get_state()))
     assert got[0][0] == got[1][0]
     assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2])
+
+
+def test_replayed_blocks_hold_whole_intervals(nbx, monkeypatch):
+    # blocks of 4 or 8 steps can be captured with M = 1 or 2, not with 5
+    s = gen.lj_liquid(6, rho=0.8442, T=0.1, seed=1)
+    for steps, every in ((4, 2), (8, 2), (50, 5), (0, 5)):
+        print(f"[case] blocks of {steps} steps", flush=True)
+        monkeypatch.setenv("NBX_GRAPH_STEPS", str(steps))
+        ctx = lj_ctx(s.u, s.v, s.L)
+        ctx.vv_run(0.002, 10)
+        assert ctx.stats()["build_every"] == every
