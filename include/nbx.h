@@ -228,9 +228,9 @@ int nbx_valu_probe(nbx_ctx* ctx, int32_t kind, int32_t reps, double* rate);
  * [2] best ms per step, [3] ms per step of the configuration on entry, [4] candidates
  * timed, [5] steps between list-build opportunities (1 for gravity).
  * Results are kept per (list | gravity plan, n, box side, cutoff, dt, trial_steps, system
- * kind, thermostat, device architecture) in the process and, when the environment variable
- * NBX_TUNE_CACHE names a file, in that file (tab-separated lines, appended); a kept result
- * is applied without trials and reports out[4] = 0. */
+ * kind, thermostat, device architecture, kernel revision) in the process and, when the
+ * environment variable NBX_TUNE_CACHE names a file, in that file (tab-separated lines,
+ * appended); a kept result is applied without trials and reports out[4] = 0. */
 int nbx_autotune(nbx_ctx* ctx, double dt, int32_t trial_steps, double* out, int32_t nout);
 /* Diagnostics of the mixed path (no reference counterpart): out[0] Verlet-list builds
  * so far, [1] list slots per atom, [2] cells per box side (0: all-pairs search),

@@ -1479,9 +1479,9 @@ int mx_learned_run(nbx_ctx* c, const nbx_model* m, double dt, int stride, int64_
 // out: [0] lanes | targets per thread, [1] skin | chunks, [2] best ms per step,
 //      [3] ms per step of the configuration found on entry, [4] candidates timed.
 // Results are kept per (plan kind, n, box side, cutoff, dt, trial steps, system kind,
-// thermostat, device architecture): in the process, and in the tab-separated file named by
-// NBX_TUNE_CACHE when that is set (one line per result, later lines win).  A result found
-// there is applied without trials (out[4] = 0).
+// thermostat, device architecture, kernel revision): in the process, and in the tab-separated
+// file named by NBX_TUNE_CACHE when that is set (one line per result, later lines win).  A
+// result found there is applied without trials (out[4] = 0).
 // =================================================================================
 #include <chrono>
 #include <cstdio>
@@ -1491,6 +1491,12 @@ int mx_learned_run(nbx_ctx* c, const nbx_model* m, double dt, int stride, int64_
 #include <sstream>
 
 namespace {
+
+// Revision of the tuned kernels, part of a result's key: raised when a change to them moves
+// their best shapes or the meaning of a shape's numbers, so that results timed on other kernels
+// are not applied.  2: gravity's chunks share a tile's half ring (they were slices of all
+// sources, and 1 x 64 a good shape), the list force kernel ends its steps by component.
+constexpr int TUNE_KERNELS = 2;
 
 struct tune_result {
     double shape0, shape1, best_ms, base_ms, every;
@@ -1512,10 +1518,10 @@ std::string tune_key(nbx_ctx* c, const mx_plan& p, bool grav, double dt, int tri
     arch = arch.substr(0, arch.find(':'));
     char buf[512];
     std::snprintf(buf, sizeof(buf),
-                  "%s n=%lld L=%.17g rc=%.17g dt=%.17g trial=%d sys=%d therm=%d lj=%d el=%d arch=%s",
+                  "%s n=%lld L=%.17g rc=%.17g dt=%.17g trial=%d sys=%d therm=%d lj=%d el=%d arch=%s kernels=%d",
                   grav ? "gravity" : "list", (long long)c->n, grav ? 0.0 : c->bc.b[0],
                   grav ? 0.0 : p.cutoff, dt, trial, c->sys, c->therm, grav ? 0 : p.nb.has_lj,
-                  grav ? 0 : p.nb.el_kind, arch.c_str());
+                  grav ? 0 : p.nb.el_kind, arch.c_str(), TUNE_KERNELS);
     return buf;
 }
 
