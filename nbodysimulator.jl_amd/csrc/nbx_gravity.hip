@@ -151,6 +151,7 @@ k_grav_tiled(const float4* __restrict__ pos, int n, int tiles, int o0, int o1,
     };
     if (item < b1 && loads) stage(WIDE ? 0 : wave, grav_body(pos, jlane(item), n));
     if (WIDE) __syncthreads();
+    else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // other lanes read the tile
     int par = 0;
     for (; item < b1; item += STEP) {
         float4 nxt = make_float4(0.f, 0.f, 0.f, 0.f);
