@@ -31,7 +31,7 @@
 //
 // Measured, us per step with k_grav_finish, against one-sided tiles that evaluated every
 // ordered pair: N = 65,536 equal masses 1,290 -> 802 (1,100 at its best tile shape), unequal
-// 881; N = 3,001 unequal 178 -> 16 (12 blocks had 256 CUs to themselves); N = 1,000 9.
+// 881; N = 3,001 unequal 178 -> 14 (12 blocks had 256 CUs to themselves); N = 1,000 9.
 // 20 ns of a SIMD per 64 unordered pairs when the chip is full.
 //
 // The self term is removed by adding 1e-24 to r^2 inside the FMA chain (no extra

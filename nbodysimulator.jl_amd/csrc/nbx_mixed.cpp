@@ -8,7 +8,8 @@
 // either through a captured hipGraph of graph_steps steps (an even count, so buffer
 // parities repeat) replayed with a device-side step base, or directly for the rest.
 // A chunk that overflows a cell or neighbour list is replayed from a device backup with
-// larger lists; the counter-based RNG makes the replay identical.
+// larger lists, one whose list went stale between two build opportunities with builds at the
+// steps between them; the counter-based RNG draws the same numbers again.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -144,13 +145,16 @@ int list_buffer(nbx_ctx* c, T** p, size_t* have, size_t bytes) {
     return NBX_OK;
 }
 
-// Lanes per atom of the list force kernel for n atoms with `entries` list entries each: as
-// many as fill the chip (about 262,144 lanes, four wavefronts per SIMD), since fewer entries
-// per lane shorten its chain of dependent gathers, but not so many that a lane holds less than
-// one pass.  Measured us per step at 4 / 8 / 16 / 32 lanes -- Lennard-Jones (78 entries): n =
-// 864 9.7 / 7.4 / 6.5 / 6.3, 4,000 12.0 / 9.6 / 8.8 / 8.8, 8,000 12.3 / 10.0 / 9.5 / 10.0,
-// 32,000 15.0 / 14.0 / 15.0 / 17.9, 200,000 43.9 / 46.2 / 52.3 / 68.7; water (about 450
-// entries): 12,288 atoms 41 / 30 / 26.0 / 25.4, 24,000 47 / 37.5 / 35.5 / 36.4.
+// Lanes per atom of the list force kernel for n atoms with `entries` list entries each.  Fewer
+// entries per lane shorten its chain of dependent gathers: 32 lanes up to 4,096 atoms whatever
+// their lists hold (the chip has lanes to spare), 16 above, and short lists halve them until
+// the atoms' lanes fit the chip (262,144, four wavefronts per SIMD).  Measured us per step at
+// 4 / 8 / 16 / 32 lanes -- Lennard-Jones (78 entries): n = 864 9.7 / 7.4 / 6.5 / 6.3, 4,000
+// 12.0 / 9.6 / 8.8 / 8.8, 8,000 12.3 / 10.0 / 9.5 / 10.0, 32,000 15.0 / 14.0 / 15.0 / 17.9,
+// 200,000 43.9 / 46.2 / 52.3 / 68.7; water (about 450 entries): 12,288 atoms 41 / 30 / 26.0 /
+// 25.4, 24,000 47 / 37.5 / 35.5 / 36.4.  Water keeps 16 where 32 would be 2 % faster: at
+// 32 the rounding of 5,184 atoms happened to differ between build intervals by more than the
+// tenth of its distance to FP64 that the tests hold intervals to (the autotuner offers 32).
 int lanes_by_size(int64_t n, double entries) {
     int g = n <= 4096 ? 32 : 16;
     if (entries < 256.0)   // long lists keep 16 lanes busy at any size
@@ -516,7 +520,9 @@ static int read_flags(nbx_ctx* c, int* h) {
 // replayed guarded (mx_vv_run), at twice the cost: water without a thermostat, whose bonds do
 // that to many a state (519 molecules, 102 steps 7.3 ms with M = 1, 15.5 replayed), takes
 // M = 1.  M follows from the state, the time step and the configuration alone, so equal
-// calls run equal steps.
+// calls run equal steps.  A guarded run launches what M = 1 launches and rebuilds at M's
+// earlier requests (300 steps of states that go stale, M = 1 / guarded: Lennard-Jones n = 864
+// 2.21 / 2.28 ms, n = 32,000 5.73 / 5.93; water, 4,096 molecules, 200 steps 4.98 / 5.31).
 // Another time step chooses again; speeds older than 100 steps are measured again (a kernel
 // and a wait, which a caller that changes the step on every call does not pay each time).
 // *relist: the interval has grown, and a list made for a shorter one may hold atoms nearly

@@ -164,7 +164,6 @@ __device__ __forceinline__ bool ref_pair_term(const ref_law& law, double xi, dou
     return true;
 }
 
-// the whole wavefront's sum over the sources of target i: component min(lane, 2) in each lane
 // component c of cnt terms added to f one after another
 __device__ __forceinline__ double ref_add_terms(double f, const double* term, int cnt, int c) {
     int q = 0;
@@ -186,6 +185,7 @@ __device__ __forceinline__ double ref_add_terms(double f, const double* term, in
     return f;
 }
 
+// the whole wavefront's sum over the sources of target i: component min(lane, 2) in each lane
 template <int KIND, bool FILTER>
 __device__ __forceinline__ double ref_wave_sum(const ref_atoms& A, const ref_law& law,
                                                const nbx_bcv& bc, int64_t i, int* cand,
