@@ -125,3 +125,29 @@ def test_stale_lists_of_water_with_a_thermostat(nbx):
     ua, va = after([150])
     ub, vb = after([3, 50, 97])
     assert np.array_equal(ua, ub) and np.array_equal(va, vb)
+
+
+@pytest.mark.parametrize("kind", ["langevin", "andersen", "nosehoover", "euler-maruyama"])
+def test_stale_lists_with_thermostats(nbx, kind):
+    """The replay draws the same numbers and takes the thermostat's state back."""
+    print(f"[case] stale lists, {kind}", flush=True)
+    s = colliding(6, 0.7)
+    therm = {"langevin": (_lib.THERM_LANGEVIN, 0.2, 1.0), "andersen": (_lib.THERM_ANDERSEN, 0.2, 5.0),
+             "nosehoover": (_lib.THERM_NOSEHOOVER, 0.2, 0.5),
+             "euler-maruyama": (_lib.THERM_LANGEVIN, 0.2, 1.0)}[kind]
+
+    def after(parts):
+        c = lj_ctx(s.u, s.v, s.L, skin=0.2, thermostat=therm)
+        for k in parts:
+            (c.em_run if kind == "euler-maruyama" else c.vv_run)(0.002, k, seed=9)
+        assert c.stats()["stale_replays"] == 1
+        return (*c.get_state(), c.thermostat_state())
+
+    (ua, va, ta), (ub, vb, tb) = after([80]), after([4, 76])
+    if kind == "nosehoover":
+        # the drift redone at a run's start adds the temperature of the atoms in another order:
+        # sqrt(3 n) roundings of 2^-53 in T, in a rate of T / tau^2 over 76 steps
+        assert np.abs(ua - ub).max() < 1e-12 and np.abs(va - vb).max() < 1e-11
+        assert np.allclose(ta, tb, rtol=1e-11, atol=1e-12)
+    else:
+        assert np.array_equal(ua, ub) and np.array_equal(va, vb)
