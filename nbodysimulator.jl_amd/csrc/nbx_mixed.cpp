@@ -335,7 +335,7 @@ mx_io make_io(nbx_ctx* c, const mx_plan& p, int par, int do_drift, double dt, in
     if (list) {
         // with a build opportunity every M steps a rebuild is requested at
         // (skin/2)(1 - (M-1)/(2M)), so that the M-1 steps to the next opportunity rarely take
-        // an atom past skin/2; one that does marks the chunk stale (replayed with M = 1)
+        // an atom past skin/2; one that does marks the chunk stale (replayed: mx_vv_run)
         const double trig = 0.5 * c->nl.skin * (1.0 - (double)(M - 1) / (2.0 * M));
         io.xref = c->nl.d_xref;
         io.half_skin2 = trig * trig;

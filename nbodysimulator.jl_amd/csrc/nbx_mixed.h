@@ -3,8 +3,9 @@
 // nbx_mixed.cpp.
 //
 // Step k of a run, with x_k in buffer X[k & 1] and its wrapped copy in P[k & 1]:
-//   build(k)  : on build-opportunity steps, if req: Verlet list from the bins B; the last
-//               block to finish clears req (and, with per-step bins, the bins)
+//   build(k)  : on build-opportunity steps, if req (guarded runs: on the others, if the stale
+//               flag): Verlet list from the bins B; the last block to finish clears req and the
+//               flag it served (and, with per-step bins, the bins)
 //   step(k)   : a_k = f(x_k, vh_k); v_k = vh_k + dt a_k / 2 (+ Langevin B half step,
 //               Andersen collisions); then the start of step k+1: Langevin A half step
 //               (registers only), x_{k+1} = x_k + dt v + dt^2 a_k / 2 into X[(k+1) & 1],
